@@ -263,9 +263,9 @@ int mbk_grow_tree(mbk_context *ctx, const mbk_tree_shape *shape, const mbk_split
  * (feature-major [cols][rows]) under a forest given as host arrays of
  * num_trees*nodes_per_tree heap slots (mask: 8 words per node, NULL without
  * categorical splits); out (device) receives [rows][cols + 1] f32, the bias
- * base_score + the trees' cover-weighted leaf means in the last column.  Path
- * tables and, for more than 4,096 columns, the fp64 accumulators are context
- * scratch. */
+ * base_score + the trees' cover-weighted leaf means in the last column.  The
+ * contribution tables (up to 1 GB, usually under 256 MB), split outcomes and fp64
+ * sums are context scratch. */
 int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshold,
                  const uint8_t *flags, const float *leaf, const float *cover,
                  const uint32_t *mask, int32_t num_trees, int32_t nodes_per_tree,

@@ -321,15 +321,25 @@ void Booster::predict_contrib(const float *x, int64_t rows, int64_t cols, float 
 // child is the left one), and repeated features on a path share one unique
 // slot whose zero fraction is the product of theirs.  A tree whose root is a
 // leaf contributes only to the bias.
-ShapTables shap_tables(const std::vector<Tree> &trees, size_t first, size_t step,
+std::vector<TreeView> tree_views(const std::vector<Tree> &trees) {
+    std::vector<TreeView> v;
+    v.reserve(trees.size());
+    for (const Tree &t : trees)
+        v.push_back({(int)t.feature.size(), t.feature.data(), t.threshold.data(), t.leaf.data(),
+                     t.cover.size() == t.feature.size() ? t.cover.data() : nullptr,
+                     t.flags.data()});
+    return v;
+}
+
+ShapTables shap_tables(const std::vector<TreeView> &trees, size_t first, size_t step,
                        int nodes_per_tree) {
     ShapTables st;
     std::vector<uint8_t> reach;
     std::vector<int> up;
     for (size_t t = first; t < trees.size(); t += step) {
-        const Tree &tr = trees[t];
-        const int nn = (int)tr.feature.size();
-        if (tr.cover.size() != tr.feature.size() || !(tr.cover[0] > 0)) continue;
+        const TreeView &tr = trees[t];
+        const int nn = tr.nodes;
+        if (!(tr.cover && tr.cover[0] > 0)) continue;
         reach.assign((size_t)nn, 0);
         reach[0] = 1;
         for (int n = 0; 2 * n + 2 < nn; ++n)
@@ -378,34 +388,24 @@ void Booster::contrib_class(const float *x, int64_t rows, int64_t cols, int k, f
     const float bias = (float)shap_bias(k);
     if (rows <= 0) return;
     build_forest();
-    const ShapTables st = shap_tables(trees, (size_t)k, (size_t)K, forest.nodes_per_tree);
-    const std::vector<mbk::ShapPath> &paths = st.paths;
-    const std::vector<mbk::ShapElem> &elems = st.elems;
-    const std::vector<mbk::ShapUniq> &uniq = st.uniq;
-    if (paths.empty()) {
-        for (int64_t i = 0; i < rows; ++i) {
-            std::fill(out + (size_t)(i * width), out + (size_t)(i * width + cols), 0.0f);
-            out[(size_t)(i * width + cols)] = bias;
-        }
-        return;
-    }
     Device &d = device();
     DevBuf<float> xd((size_t)rows * (size_t)cols), od((size_t)rows * (size_t)width);
-    DevBuf<mbk::ShapPath> pd(paths.size());
-    DevBuf<mbk::ShapElem> ed(elems.size());
-    DevBuf<mbk::ShapUniq> ud(uniq.size());
     upload(xd.ptr, x, xd.bytes(), d.stream);
-    MB_HIP(hipMemcpyAsync(pd.ptr, paths.data(), pd.bytes(), hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(ed.ptr, elems.data(), ed.bytes(), hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(ud.ptr, uniq.data(), ud.bytes(), hipMemcpyHostToDevice, d.stream));
-    DevBuf<double> phi;
-    if (mbk::treeshap_needs_scratch((int)cols))
-        phi.alloc((size_t)((rows + 63) / 64) * 64 * (size_t)cols);
-    MB_HIP(mbk::launch_treeshap(d.stream, xd.ptr, rows, (int)cols, trained_num_bins - 1,
-                                forest.has_mask ? forest.mask.ptr : nullptr, pd.ptr,
-                                (int)paths.size(), st.max_elems, ed.ptr, ud.ptr, bias, od.ptr,
-                                phi.ptr));
-    download(out, od.ptr, od.bytes(), d.stream);
+    if (shap_plans.empty()) shap_plans.resize((size_t)K);
+    ShapScratch scratch;
+    scratch.pool();
+    const StreamIdle idle{d.stream};                   // before the scratch goes back
+    const ShapCall call{xd.ptr, rows, (int32_t)cols, trained_num_bins - 1,
+                        forest.has_mask ? forest.mask.ptr : nullptr, bias, od.ptr};
+    if (treeshap(d.stream, tree_views(trees), (size_t)k, (size_t)K, forest.nodes_per_tree, call,
+                 shap_plans[(size_t)k], scratch)) {
+        download(out, od.ptr, od.bytes(), d.stream);
+        return;
+    }
+    for (int64_t i = 0; i < rows; ++i) {               // no split anywhere
+        std::fill(out + (size_t)(i * width), out + (size_t)(i * width + cols), 0.0f);
+        out[(size_t)(i * width + cols)] = bias;
+    }
 }
 
 std::vector<float> Booster::feature_importance(int type) const {   // Booster.swift:1926-1940

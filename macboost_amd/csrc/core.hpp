@@ -187,6 +187,13 @@ struct DevBuf {
     size_t bytes() const { return n * sizeof(T); }
 };
 
+// Waits for a stream when it goes out of scope: declared after pooled buffers
+// that the stream's work uses, it also covers an exception on the way.
+struct StreamIdle {
+    hipStream_t s;
+    ~StreamIdle() { (void)hipStreamSynchronize(s); }
+};
+
 // Flattened forest resident on the device (forestBuffers, Booster.swift:1944-1985).
 struct ForestCache {
     bool valid = false;
@@ -198,6 +205,45 @@ struct ForestCache {
     DevBuf<uint8_t> flags;
     DevBuf<float> leaf;
     DevBuf<uint32_t> mask;
+};
+
+// A tree's arrays where they are (a Tree's, or a caller's flat forest).
+struct TreeView {
+    int nodes = 0;
+    const int32_t *feature = nullptr;
+    const float *threshold = nullptr, *leaf = nullptr;
+    const float *cover = nullptr;    // NULL: none recorded
+    const uint8_t *flags = nullptr;
+};
+std::vector<TreeView> tree_views(const std::vector<Tree> &trees);
+
+// The contribution-table plan of some trees (shap.cpp); its vectors keep their
+// memory when it is made again.
+struct ShapSetPlan {
+    mbk::ShapSet set;
+    std::vector<mbk::ShapTest> tests;
+    std::vector<mbk::ShapGroup> groups;
+    std::vector<double> vals;
+    std::vector<int32_t> col_feature;        // per column: its feature
+    std::vector<uint32_t> col_off, run_first, at, order;
+    std::vector<mbk::ShapItem> items;
+    std::vector<mbk::ShapBatch> batches;
+    void clear() {
+        set = mbk::ShapSet{};
+        tests.clear();
+        groups.clear();
+        vals.clear();
+        col_feature.clear();
+    }
+};
+struct ShapPlan {
+    bool made = false;
+    std::vector<ShapSetPlan> sets;
+    size_t num_sets = 0;
+    double evals = 0;          // path evaluations of the tables
+    double paths = 0;
+    bool fits = true;          // every group within SHAP_MAX_BITS
+    std::vector<uint8_t> height;
 };
 
 struct Booster {
@@ -217,6 +263,7 @@ struct Booster {
 
     std::unique_ptr<Device> dev;
     ForestCache forest;
+    std::vector<ShapPlan> shap_plans;    // per class, made by its first predict_contrib
 
     Booster() = default;
     Booster(const Booster &) = delete;
@@ -256,15 +303,41 @@ BinnedDataset *dataset_load(const std::string &path);
 Booster *load_model_file(const std::string &path);
 
 // Root-to-leaf path tables of trees first, first + step, ... for the TreeSHAP
-// kernels; max_elems is the longest path's split count.
+// path kernels; max_elems is the longest path's split count.
 struct ShapTables {
     std::vector<mbk::ShapPath> paths;
     std::vector<mbk::ShapElem> elems;
     std::vector<mbk::ShapUniq> uniq;
     int32_t max_elems = 1;
 };
-ShapTables shap_tables(const std::vector<Tree> &trees, size_t first, size_t step,
+ShapTables shap_tables(const std::vector<TreeView> &trees, size_t first, size_t step,
                        int nodes_per_tree);
+
+// Scratch of TreeSHAP calls; buffers grow when a call needs more.
+struct ShapScratch {
+    std::vector<char> blob;          // host image of `arrays`
+    DevBuf<char> arrays;             // the plan's or the path tables' arrays
+    DevBuf<double> table, runs;      // contribution tables and their sums
+    DevBuf<char> patterns;
+    DevBuf<double> sums;             // several table sets, or wide data by path
+    // Allocate through the device memory cache.
+    void pool() {
+        arrays.pooled = table.pooled = runs.pooled = patterns.pooled = sums.pooled = true;
+    }
+};
+struct ShapCall {
+    const float *x;                  // device, feature-major [cols][rows]
+    int64_t rows;
+    int32_t cols, data_bins;
+    const uint32_t *masks;           // device, 8 words per node, or NULL
+    float bias;
+    float *out;                      // device, [rows][cols + 1]
+};
+// TreeSHAP contributions of trees first, first + step, ... on stream s; waits
+// for them.  Makes the plan unless it is made.  False when no tree has a split
+// (nothing is written then).
+bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, size_t step,
+              int nodes_per_tree, const ShapCall &call, ShapPlan &plan, ShapScratch &scratch);
 
 // Incremental trainer (fitImpl, Booster.swift:445-1701).
 struct Trainer;

@@ -3,10 +3,11 @@
 // walk used for per-iteration validation (predict_tree_binned, :1763-1781) and
 // exact TreeSHAP (gpu_treeshap, :1656-1734).
 //
-// TreeSHAP here gives each row a wavefront and each root-to-leaf path a lane,
-// extending/unwinding in double precision and accumulating the row's phi in
-// LDS (the wavefront owns it, so the summation order is fixed), with a single
-// rounding to f32 at the end.
+// TreeSHAP here computes path contributions once per split outcome into tables
+// and looks every row's up, all in double precision with a fixed summation order
+// and a single rounding to f32 at the end.  Trees too deep for tables (more
+// outcomes than rows) give each row a wavefront and each root-to-leaf path a
+// lane, with the row's phi in LDS.
 #include <algorithm>
 
 #include "grad.h"
@@ -339,6 +340,72 @@ __global__ __launch_bounds__(64) void k_treeshap(const float *__restrict__ x, in
     orow[cols] = bias;
 }
 
+// The contributions of one root-to-leaf path with U unique features: zero[u] is
+// feature u's unfollowed share (1 for u >= U), bit u of ones says that the row
+// follows every split of feature u on the path.  emit(u, contribution), u = 0 ..
+// U - 1.
+template <int MAXU, typename Emit>
+__device__ __forceinline__ void path_contributions(int U, const double (&zero)[MAXU],
+                                                   uint32_t ones, double leaf, Emit emit) {
+    double one[MAXU];
+#pragma unroll
+    for (int u = 0; u < MAXU; ++u) one[u] = ((ones >> u) & 1u) ? 1.0 : 0.0;
+    // EXTEND with the dummy element at index 0 (SHAP.swift:266-279).  The
+    // weights (q+1)/(j+1) and (j-q)/(j+1) are compile-time constants here,
+    // one multiply each instead of a multiply and a divide (a rounding
+    // apart from the divided form).
+    double pw[MAXU + 1];
+    pw[0] = 1.0;
+#pragma unroll
+    for (int j = 1; j <= MAXU; ++j) {
+        pw[j] = 0.0;
+        if (j <= U) {
+            const double o = one[j - 1], z = zero[j - 1];
+#pragma unroll
+            for (int q = j - 1; q >= 0; --q) {
+                const double up = (double)(q + 1) / (double)(j + 1);
+                const double down = (double)(j - q) / (double)(j + 1);
+                pw[q + 1] += o * pw[q] * up;
+                pw[q] = z * pw[q] * down;
+            }
+        }
+    }
+    // 1 / (U - q) for q < U: U divisions per path, shared by every
+    // unique feature's unwinding
+    double inv_uq[MAXU];
+#pragma unroll
+    for (int q = 0; q < MAXU; ++q) inv_uq[q] = q < U ? 1.0 / (double)(U - q) : 0.0;
+    // unwound sums per unique feature (SHAP.swift:307-325).  one[u] is 0
+    // or 1, so the o != 0 form divides by the constant q + 1 (a multiply
+    // by its reciprocal here) and the o == 0 form by z (U - q) (one 1/z
+    // per feature).  Both forms share one loop: a wavefront's lanes take
+    // both.
+#pragma unroll
+    for (int u = 0; u < MAXU; ++u) {
+        if (u < U) {
+            const double o = one[u], z = zero[u];
+            const bool on = o != 0.0, live = on || z != 0.0;
+            const double inv_z = (!on && z != 0.0) ? 1.0 / z : 0.0;
+            double total = 0.0;
+            double next = 0.0;
+#pragma unroll
+            for (int q = MAXU; q >= 0; --q)
+                if (q == U) next = pw[q];
+#pragma unroll
+            for (int q = MAXU - 1; q >= 0; --q) {
+                if (q < U) {
+                    const double rq = 1.0 / (double)(q + 1);
+                    const double tmp = on ? next * rq
+                                          : (live ? pw[q] * inv_z * inv_uq[q] : 0.0);
+                    total += tmp;
+                    if (on) next = pw[q] - tmp * z * (double)(U - q);
+                }
+            }
+            emit(u, total * (double)(U + 1) * (o - z) * leaf);
+        }
+    }
+}
+
 // Path-parallel TreeSHAP: one wavefront per row (grid-stride), one lane per
 // root-to-leaf path, 64 paths per pass.  The row's feature values and its phi
 // sit in LDS; each lane runs the same fp64 EXTEND/UNWIND as k_treeshap for its
@@ -392,63 +459,9 @@ __global__ __launch_bounds__(64) void k_treeshap_rows(const float *__restrict__ 
                                                 data_bins);
                 if (left != ((el.flags & 0x100u) != 0)) ones &= ~(1u << el.uniq);
             }
-            double one[MAXU];
-#pragma unroll
-            for (int u = 0; u < MAXU; ++u) one[u] = ((ones >> u) & 1u) ? 1.0 : 0.0;
-            // EXTEND with the dummy element at index 0 (SHAP.swift:266-279).  The
-            // weights (q+1)/(j+1) and (j-q)/(j+1) are compile-time constants here,
-            // one multiply each instead of a multiply and a divide (a rounding
-            // apart from the divided form).
-            double pw[MAXU + 1];
-            pw[0] = 1.0;
-#pragma unroll
-            for (int j = 1; j <= MAXU; ++j) {
-                pw[j] = 0.0;
-                if (j <= U) {
-                    const double o = one[j - 1], z = zero[j - 1];
-#pragma unroll
-                    for (int q = j - 1; q >= 0; --q) {
-                        const double up = (double)(q + 1) / (double)(j + 1);
-                        const double down = (double)(j - q) / (double)(j + 1);
-                        pw[q + 1] += o * pw[q] * up;
-                        pw[q] = z * pw[q] * down;
-                    }
-                }
-            }
-            // 1 / (U - q) for q < U: U divisions per path, shared by every
-            // unique feature's unwinding
-            double inv_uq[MAXU];
-#pragma unroll
-            for (int q = 0; q < MAXU; ++q) inv_uq[q] = q < U ? 1.0 / (double)(U - q) : 0.0;
-            // unwound sums per unique feature (SHAP.swift:307-325).  one[u] is 0
-            // or 1, so the o != 0 form divides by the constant q + 1 (a multiply
-            // by its reciprocal here) and the o == 0 form by z (U - q) (one 1/z
-            // per feature).  Both forms share one loop: a wavefront's lanes take
-            // both.
-#pragma unroll
-            for (int u = 0; u < MAXU; ++u) {
-                if (u < U) {
-                    const double o = one[u], z = zero[u];
-                    const bool on = o != 0.0, live = on || z != 0.0;
-                    const double inv_z = (!on && z != 0.0) ? 1.0 / z : 0.0;
-                    double total = 0.0;
-                    double next = 0.0;
-#pragma unroll
-                    for (int q = MAXU; q >= 0; --q)
-                        if (q == U) next = pw[q];
-#pragma unroll
-                    for (int q = MAXU - 1; q >= 0; --q) {
-                        if (q < U) {
-                            const double rq = 1.0 / (double)(q + 1);
-                            const double tmp = on ? next * rq
-                                                  : (live ? pw[q] * inv_z * inv_uq[q] : 0.0);
-                            total += tmp;
-                            if (on) next = pw[q] - tmp * z * (double)(U - q);
-                        }
-                    }
-                    atomicAdd(&phi[feat[u]], total * (double)(U + 1) * (o - z) * P.leaf);
-                }
-            }
+            path_contributions<MAXU>(U, zero, ones, P.leaf, [&](int u, double v) {
+                atomicAdd(&phi[feat[u]], v);
+            });
         }
         __syncthreads();
         float *orow = out + i * (int64_t)(cols + 1);
@@ -456,6 +469,327 @@ __global__ __launch_bounds__(64) void k_treeshap_rows(const float *__restrict__ 
         if (lane == 0) orow[cols] = bias;
         __syncthreads();                               // before the next row reuses the LDS
     }
+}
+
+// ---- TreeSHAP from contribution tables -------------------------------------
+//
+// A path's contributions depend on the row only through which of its splits the
+// row follows, so they are computed once per outcome instead of once per row.
+// Paths are grouped by the lowest ancestors whose subtree holds at most two
+// levels of splits (four leaves): a group's outcome is one bit per feature
+// among its root's ancestors and one per split inside (7 bits at depth 6), and
+// its leaves' contributions to a feature are summed into one column of 2^bits
+// doubles.  Four launches:
+//   k_shap_tables    the columns (EXTEND/UNWIND once per group and outcome)
+//   k_shap_patterns  every row's outcome per group
+//   k_shap_sum       per row and feature the sum of its columns' entries
+//   k_shap_finish    the runs of k_shap_sum added up, in f32, row-major
+// Two levels per group: one level (leaf pairs) needs 192 lookups per row and
+// depth-6 tree, two 112, three 80 out of tables 6 times the size that no longer
+// stream through LDS.  200k rows x 100 trees of depth 6: 36.4 ms with a path
+// evaluation per row, now 1.2 ms (outcomes 0.62, sums 0.46, tables 0.03).
+
+constexpr int SHAP_LDS_DOUBLES = 4096;                 // one batch of columns
+constexpr int SHAP_THREADS = SHAP_BLOCK_ROWS / 4;      // four rows per thread
+
+// One workgroup of one wavefront per (group, 64 outcomes): a lane per outcome
+// walks the group's leaves; sums per column in LDS (a lane's own slots), then
+// stored coalesced.  Bound by fp64 arithmetic, but 128 outcomes per group
+// stand for any number of rows (100 trees of depth 6: 0.8M path evaluations
+// against 1280M for 200k rows).
+template <int MAXU>
+__global__ __launch_bounds__(64) void k_shap_tables(const ShapGroup *__restrict__ groups,
+                                                    const double *__restrict__ vals,
+                                                    const uint32_t *__restrict__ col_off,
+                                                    double *__restrict__ table) {
+    __shared__ double acc[SHAP_MAX_COLS][64];
+    const ShapGroup g = groups[blockIdx.x];
+    const uint32_t first = blockIdx.y * 64u;
+    if (first >= (1u << g.bits)) return;
+    const int lane = threadIdx.x;
+    const uint32_t pattern = first + (uint32_t)lane;
+    for (int c = 0; c < g.num_cols; ++c) acc[c][lane] = 0.0;
+    const double *anc = vals + g.val_start, *share = anc + g.anc;
+    for (int q = 0; q < 4; ++q) {
+        if (!((g.leaves >> q) & 1u)) continue;
+        double zero[MAXU];
+        int col[MAXU];
+        uint32_t ones = pattern & ((1u << g.anc) - 1u);
+#pragma unroll
+        for (int u = 0; u < MAXU; ++u) {
+            zero[u] = u < g.anc ? anc[u] : 1.0;
+            col[u] = u;
+        }
+        int slots = g.anc;
+        // the splits inside on this leaf's path: the root, then a child
+        const double *sh = share;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t in = g.inside[k];
+            if (in == 0) continue;
+            const double left = sh[0], right = sh[1];
+            sh += 2;
+            if (k > 0 && (q >> 1) != k - 1) continue;
+            const bool go_left = k == 0 ? q < 2 : (q & 1) == 0;
+            const bool follows = (((pattern >> ((in >> 8) & 0xFFu)) & 1u) != 0) == go_left;
+            const int c = (int)(in & 0xFFu);
+            int at = slots;
+#pragma unroll
+            for (int u = 0; u < MAXU; ++u)
+                if (u < slots && col[u] == c) at = u;
+#pragma unroll
+            for (int u = 0; u < MAXU; ++u) {
+                if (u == at) {
+                    zero[u] *= go_left ? left : right;
+                    col[u] = c;
+                }
+            }
+            if (at == slots) {
+                ones |= 1u << at;
+                ++slots;
+            }
+            if (!follows) ones &= ~(1u << at);
+        }
+        path_contributions<MAXU>(slots, zero, ones, vals[g.leaf_start + q], [&](int u, double v) {
+            acc[col[u]][lane] += v;
+        });
+    }
+    if (pattern < (1u << g.bits))
+        for (int c = 0; c < g.num_cols; ++c)
+            table[(size_t)col_off[g.col_start + c] + pattern] = acc[c][lane];
+}
+
+template <typename PT> struct ShapPack;                // four rows' outcomes
+template <> struct ShapPack<uint8_t> {
+    uint32_t w;
+    __device__ __forceinline__ void set(const uint32_t (&p)[4]) {
+        w = p[0] | (p[1] << 8) | (p[2] << 16) | (p[3] << 24);
+    }
+    __device__ __forceinline__ uint32_t get(int k) const { return (w >> (8 * k)) & 0xFFu; }
+};
+template <> struct ShapPack<uint16_t> {
+    uint32_t w[2];
+    __device__ __forceinline__ void set(const uint32_t (&p)[4]) {
+        w[0] = p[0] | (p[1] << 16);
+        w[1] = p[2] | (p[3] << 16);
+    }
+    __device__ __forceinline__ uint32_t get(int k) const {
+        return (w[k >> 1] >> (16 * (k & 1))) & 0xFFFFu;
+    }
+};
+
+// Outcomes of SHAP_BLOCK_ROWS rows x per_block groups per workgroup; a lane holds rows
+// lane, lane + 64, + 128, + 192 of its wavefront's 256, so the feature loads are
+// coalesced (the split is the same for every lane: its column is a scalar
+// address) and its four outcomes are one packed store.  Bound by the
+// instructions per row and split: with the split's flags scalar, a numeric one is
+// a single compare (v > thr where missing goes left, v <= thr where not; NaN
+// fails both) and the bit's conditional set (200k rows x 1,600 groups: 755 us,
+// 1,640 us with the general form for every split, 615 us once small launches
+// were spread over more workgroups).
+template <typename PT>
+__global__ __launch_bounds__(SHAP_THREADS) void k_shap_patterns(
+    const float *__restrict__ x, int64_t rows, int64_t row0, int32_t data_bins,
+    const uint32_t *__restrict__ masks, const ShapGroup *__restrict__ groups, int32_t num_groups,
+    const ShapTest *__restrict__ tests, int32_t per_block,
+    ShapPack<PT> *__restrict__ out, size_t pitch) {
+    const int64_t base = row0 + (int64_t)blockIdx.x * SHAP_BLOCK_ROWS;
+    const int64_t past = rows - 1 - base;              // rows past the end: the last row
+    uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t i = (threadIdx.x >> 6) * 256 + (threadIdx.x & 63) + 64 * k;
+        r[k] = (int64_t)i <= past ? i : (uint32_t)past;
+    }
+    const float *xb = x + base;
+    const int g0 = blockIdx.y * per_block, g1 = min(num_groups, g0 + per_block);
+    for (int gi = g0; gi < g1; ++gi) {
+        const ShapGroup g = groups[gi];
+        uint32_t fail[4] = {0, 0, 0, 0};
+        // four tests at a time: one 64-B scalar load, 16 feature loads in flight
+        for (int t = 0; t < g.num_tests; t += 4) {
+            ShapTest T[4];
+            float v[4][4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) T[j] = tests[g.test_start + t + j];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float *col = xb + (int64_t)T[j].feature * rows;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[j][k] = col[r[k]];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t flags = T[j].flags, bit = 1u << (flags >> 16);
+                const bool when_left = (flags & 0x100u) != 0;
+                if (flags & FLAG_CATEGORICAL) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const bool left = raw_goes_left(
+                            v[j][k], flags & 0xFFu, T[j].threshold,
+                            masks ? masks + (int64_t)T[j].node * 8 : nullptr, data_bins);
+                        if (left != when_left) fail[k] |= bit;
+                    }
+                } else if (flags & FLAG_DEFAULT_LEFT) {
+                    const uint32_t above = when_left ? bit : 0u, rest = bit ^ above;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) fail[k] |= v[j][k] > T[j].threshold ? above : rest;
+                } else {
+                    const uint32_t rest = when_left ? bit : 0u, within = bit ^ rest;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) fail[k] |= v[j][k] <= T[j].threshold ? within : rest;
+                }
+            }
+        }
+        uint32_t pat[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) pat[k] = ~fail[k] & ((1u << g.bits) - 1u);
+        ShapPack<PT> w;
+        w.set(pat);
+        out[(size_t)gi * pitch + (size_t)blockIdx.x * SHAP_THREADS + threadIdx.x] = w;
+    }
+}
+
+// One workgroup per (SHAP_BLOCK_ROWS rows, share of the batches).  Items (one column of
+// one group) are ordered by feature; a batch's columns are contiguous and go
+// through LDS, where 64 lanes look up their outcomes.  A lane's four rows sum in
+// registers until the feature ends or the share does (a run), then the run's
+// sums are stored: no atomics, so the order is fixed.  Bound by the random
+// 8-byte LDS reads (depth 6: 2.2G of them for 200k rows x 100 trees in 459 us)
+// and, for long columns, by their loads: 20k rows x 50 trees of depth 8 took 405
+// us with 1,024 rows per workgroup and 249 us with 2,048.
+template <typename PT>
+__global__ __launch_bounds__(SHAP_THREADS) void k_shap_sum(const ShapItem *__restrict__ items,
+                                                  const ShapBatch *__restrict__ batches,
+                                                  int32_t num_batches,
+                                                  const double *__restrict__ table,
+                                                  const ShapPack<PT> *__restrict__ patterns,
+                                                  size_t pitch, double *__restrict__ runs,
+                                                  size_t run_pitch) {
+    __shared__ double2 cols2[SHAP_LDS_DOUBLES / 2];
+    double *cols = reinterpret_cast<double *>(cols2);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int b0 = (int)((int64_t)num_batches * blockIdx.y / gridDim.y);
+    const int b1 = (int)((int64_t)num_batches * (blockIdx.y + 1) / gridDim.y);
+    const ShapPack<PT> *pat = patterns + (size_t)blockIdx.x * SHAP_THREADS + threadIdx.x;
+    double *dst = runs + (size_t)blockIdx.x * SHAP_BLOCK_ROWS + wave * 256 + lane;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = b0; b < b1; ++b) {
+        const ShapBatch B = batches[b];
+        __syncthreads();                               // the last batch's lookups are done
+        const double2 *src = reinterpret_cast<const double2 *>(table + B.table_off);
+        for (uint32_t k = threadIdx.x; k < B.table_len / 2; k += SHAP_THREADS) cols2[k] = src[k];
+        __syncthreads();
+        const ShapItem *it = items + B.item_start;
+        for (int i = 0; i < B.num_items; i += 4) {
+            ShapPack<PT> w[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (i + j < B.num_items) w[j] = pat[(size_t)it[i + j].group * pitch];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (i + j >= B.num_items) break;
+                const uint32_t off = it[i + j].offset_run & 0xFFFu, run = it[i + j].offset_run >> 12;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) acc[k] += cols[off + w[j].get(k)];
+                if (run != 0) {
+                    double *d = dst + (size_t)(run - 1) * run_pitch;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        d[64 * k] = acc[k];
+                        acc[k] = 0.0;
+                    }
+                }
+            }
+        }
+    }
+}
+
+// Adds up each feature's runs (and, with several table sets, the sums of the
+// earlier ones: total, [cols][rows] f64), 64 rows x 64 features per workgroup
+// through an LDS transpose; the last set writes f32 rows and the bias.
+__global__ __launch_bounds__(256) void k_shap_finish(const double *__restrict__ runs,
+                                                     size_t run_pitch,
+                                                     const uint32_t *__restrict__ run_first,
+                                                     int64_t row0, int64_t rows, int32_t cols,
+                                                     double *__restrict__ total, int first,
+                                                     int last, float bias,
+                                                     float *__restrict__ out) {
+    __shared__ float tile[64][65];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r0 = row0 + (int64_t)blockIdx.x * 64;
+    const int f0 = blockIdx.y * 64;
+    const int nf = min(64, cols - f0);
+    const int64_t row = r0 + lane;
+    for (int f = wave; f < nf; f += 4) {
+        double v = 0.0;
+        if (!first && row < rows) v = total[(size_t)(f0 + f) * (size_t)rows + (size_t)row];
+        for (uint32_t k = run_first[f0 + f]; k < run_first[f0 + f + 1]; ++k)
+            v += runs[(size_t)k * run_pitch + (size_t)(row - row0)];
+        if (!last) {
+            if (row < rows) total[(size_t)(f0 + f) * (size_t)rows + (size_t)row] = v;
+        } else {
+            tile[lane][f] = (float)v;
+        }
+    }
+    if (!last) return;
+    __syncthreads();
+    const int64_t nr = rows - r0 < 64 ? rows - r0 : 64;
+    for (int q = wave; q < nr; q += 4) {
+        float *o = out + (r0 + q) * (int64_t)(cols + 1);
+        if (lane < nf) o[f0 + lane] = tile[q][lane];
+        if (lane == 0 && f0 + 64 >= cols) o[cols] = bias;
+    }
+}
+
+hipError_t launch_shap_tables(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                              double *table) {
+    if (set.num_groups == 0) return hipSuccess;
+    const dim3 grid((unsigned)set.num_groups, (unsigned)((((size_t)1 << set.max_bits) + 63) / 64));
+#define MBK_SHAP_TABLES(U)                                                                      \
+    hipLaunchKernelGGL(k_shap_tables<U>, grid, dim3(64), 0, s, d.groups, d.vals, d.col_off, table)
+    if (set.max_slots <= 4) MBK_SHAP_TABLES(4);
+    else if (set.max_slots <= 6) MBK_SHAP_TABLES(6);
+    else if (set.max_slots <= 8) MBK_SHAP_TABLES(8);
+    else MBK_SHAP_TABLES(SHAP_MAX_U);
+#undef MBK_SHAP_TABLES
+    return hipGetLastError();
+}
+
+template <typename PT>
+static hipError_t shap_slab(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                            const ShapSlab &w) {
+    const unsigned blocks = (unsigned)(w.slab_rows / SHAP_BLOCK_ROWS);
+    const size_t pitch = (size_t)w.slab_rows / 4;
+    ShapPack<PT> *pat = reinterpret_cast<ShapPack<PT> *>(w.patterns);
+    if (set.num_groups > 0) {
+        // a group is a chain of scalar and feature loads: at least 2,048
+        // workgroups (eight per CU) hide it, at most 64 groups each
+        const int64_t per = std::max<int64_t>(1, (int64_t)set.num_groups * blocks / 2048);
+        const int32_t per_block = (int32_t)std::min<int64_t>(per, 64);
+        hipLaunchKernelGGL(k_shap_patterns<PT>,
+                           dim3(blocks, (unsigned)((set.num_groups + per_block - 1) / per_block)),
+                           dim3(SHAP_THREADS), 0, s, w.x, w.rows, w.row0, w.data_bins, w.masks, d.groups,
+                           set.num_groups, d.tests, per_block, pat, pitch);
+        hipLaunchKernelGGL(k_shap_sum<PT>, dim3(blocks, (unsigned)set.shares),
+                           dim3(SHAP_THREADS), 0, s,
+                           d.items, d.batches, set.num_batches, w.table, pat, pitch, w.runs,
+                           (size_t)w.slab_rows);
+    }
+    const int64_t live = std::min<int64_t>(w.slab_rows, w.rows - w.row0);
+    hipLaunchKernelGGL(k_shap_finish, dim3((unsigned)((live + 63) / 64), (unsigned)((w.cols + 63) / 64)),
+                       dim3(256), 0, s, w.runs, (size_t)w.slab_rows, d.run_first, w.row0, w.rows,
+                       w.cols, w.total, w.first, w.last, w.bias, w.out);
+    return hipGetLastError();
+}
+
+hipError_t launch_shap_slab(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                            const ShapSlab &w) {
+    if (w.rows <= 0 || w.slab_rows <= 0 || w.slab_rows % SHAP_BLOCK_ROWS != 0 ||
+        set.max_bits > SHAP_MAX_BITS || set.shares < 1 || set.shares > 65535 ||
+        (!(w.first && w.last) && !w.total))
+        return hipErrorInvalidValue;
+    return set.max_bits > 8 ? shap_slab<uint16_t>(s, set, d, w) : shap_slab<uint8_t>(s, set, d, w);
 }
 
 // Columns up to which k_treeshap_rows runs (12 B of LDS per column).

@@ -682,4 +682,79 @@ hipError_t launch_treeshap(hipStream_t s, const float *x, int64_t rows, int32_t 
                            const ShapUniq *uniq, float bias, float *out, double *phi_global);
 bool treeshap_needs_scratch(int cols);
 
+
+// ---- TreeSHAP from contribution tables (kernels_infer.hip) ----
+constexpr int SHAP_MAX_COLS = 16;     // features of a group: 10 ancestors + 3 splits at depth 12
+constexpr int SHAP_BLOCK_ROWS = 2048; // rows of a workgroup: a column's LDS load serves them all
+constexpr int SHAP_MAX_BITS = 12;     // a column of 2^12 doubles is one LDS batch
+
+// One split whose outcome enters a group's bit (flags >> 16): the bit stays set
+// while the row goes left (0x100 in flags) or right (not); low flags as a split's.
+struct ShapTest {
+    int32_t feature;
+    float threshold;
+    uint32_t flags;
+    int32_t node;         // global node index (tree * nodes_per_tree + node)
+};
+// A group: bits 0 .. anc - 1 are its ancestors' features (column b belongs to
+// bit b), one more per split inside (root, left child, right child).  vals holds
+// the ancestors' unfollowed shares, then (left, right) shares per split inside.
+struct ShapGroup {
+    int32_t test_start, num_tests;   // padded to a multiple of 4 by repeats
+    int32_t val_start, leaf_start;   // in vals; the four leaf positions' values
+    int32_t col_start, num_cols;
+    int32_t anc, bits;
+    uint32_t inside[3];              // column | bit << 8 | 0x10000, or 0: no split
+    uint32_t leaves;                 // which leaf positions are leaves
+};
+// Items in feature order: one column of one group.  offset_run: the column's
+// first double within its batch | (run + 1) << 12 when its feature's sums go to
+// that run after this item (0: they continue).
+struct ShapItem {
+    uint32_t group, offset_run;
+};
+struct ShapBatch {
+    uint32_t item_start;
+    int32_t num_items;
+    uint32_t table_off, table_len;   // doubles, both even
+};
+// One set of trees whose tables are in memory together: its sizes, and its
+// arrays on the device.
+struct ShapSet {
+    int32_t num_groups = 0, num_batches = 0;
+    int32_t max_bits = 1, max_slots = 1;
+    int32_t shares = 1;              // workgroups per SHAP_BLOCK_ROWS rows
+    int32_t num_runs = 0;
+    size_t table_len = 0;            // doubles
+};
+struct ShapSetDev {
+    const ShapTest *tests;
+    const ShapGroup *groups;
+    const double *vals;
+    const uint32_t *col_off;
+    const ShapItem *items;
+    const ShapBatch *batches;
+    const uint32_t *run_first;       // [cols + 1]
+};
+// Rows [row0, row0 + slab_rows) of x (slab_rows a multiple of SHAP_BLOCK_ROWS; rows past
+// the end are not written).  total: [cols][rows] f64, needed when there are
+// several sets; first / last: of the sets.
+struct ShapSlab {
+    const float *x;
+    int64_t rows, row0, slab_rows;
+    int32_t cols, data_bins;
+    const uint32_t *masks;
+    const double *table;
+    void *patterns;                  // num_groups * slab_rows bytes, 2 per row past 8 bits
+    double *runs;                    // num_runs * slab_rows
+    double *total;
+    int first, last;
+    float bias;
+    float *out;
+};
+hipError_t launch_shap_tables(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                              double *table);
+hipError_t launch_shap_slab(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                            const ShapSlab &w);
+
 }  // namespace mbk

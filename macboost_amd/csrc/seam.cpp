@@ -60,11 +60,9 @@ struct Scratch {
     DevBuf<mbk::TreeCtl> qctl;                       // mbk_quantize
     DevBuf<uint32_t> gmax_part;
     DevBuf<uint32_t> keys_a, keys_b, key_counts;     // mbk_quantile_edges
-    DevBuf<mbk::ShapPath> paths;                     // mbk_treeshap
-    DevBuf<mbk::ShapElem> elems;
-    DevBuf<mbk::ShapUniq> uniq;
+    mb::ShapPlan shap_plan;                          // mbk_treeshap
+    mb::ShapScratch shap;
     DevBuf<uint32_t> shap_mask;
-    DevBuf<double> phi;
 };
 
 }  // namespace
@@ -526,20 +524,15 @@ int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshol
         need(ctx != nullptr, "null kernel-seam context");
         need(num_trees >= 0 && nodes_per_tree >= 1, "empty forest shape");
         need(rows >= 0 && cols >= 1, "rows and cols must be positive");
-        std::vector<mb::Tree> trees((size_t)num_trees);
+        std::vector<mb::TreeView> trees((size_t)num_trees);
         const size_t npt = (size_t)nodes_per_tree;
-        for (size_t t = 0; t < trees.size(); ++t) {
-            mb::Tree &tr = trees[t];
-            tr.feature.assign(feature + t * npt, feature + (t + 1) * npt);
-            tr.threshold.assign(threshold + t * npt, threshold + (t + 1) * npt);
-            tr.flags.assign(flags + t * npt, flags + (t + 1) * npt);
-            tr.leaf.assign(leaf + t * npt, leaf + (t + 1) * npt);
-            tr.cover.assign(cover + t * npt, cover + (t + 1) * npt);
-        }
+        for (size_t t = 0; t < trees.size(); ++t)
+            trees[t] = {nodes_per_tree, feature + t * npt, threshold + t * npt, leaf + t * npt,
+                        cover + t * npt, flags + t * npt};
         // expected raw score: base + each tree's cover-weighted leaf mean
         // (SHAP.swift:56-72)
         double bias = (double)base_score;
-        for (const mb::Tree &tr : trees) {
+        for (const mb::TreeView &tr : trees) {
             const double total = (double)tr.cover[0];
             if (!(total > 0)) continue;
             double mean = 0;
@@ -547,38 +540,19 @@ int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshol
             while (!stack.empty()) {
                 const int n = stack.back();
                 stack.pop_back();
-                if (tr.feature[(size_t)n] >= 0 && 2 * n + 2 < nodes_per_tree) {
+                if (tr.feature[n] >= 0 && 2 * n + 2 < nodes_per_tree) {
                     stack.push_back(2 * n + 1);
                     stack.push_back(2 * n + 2);
                 } else {
-                    mean += (double)tr.leaf[(size_t)n] * (double)tr.cover[(size_t)n] / total;
+                    mean += (double)tr.leaf[n] * (double)tr.cover[n] / total;
                 }
             }
             bias += mean;
         }
-        const mb::ShapTables st = mb::shap_tables(trees, 0, 1, nodes_per_tree);
         hipStream_t s = ctx->dev->stream;
         const int64_t width = (int64_t)cols + 1;
         if (rows == 0) return 0;
         Scratch &sc = ctx->scratch;
-        if (st.paths.empty()) {
-            std::vector<float> row((size_t)width, 0.0f);
-            row[(size_t)cols] = (float)bias;
-            for (int64_t i = 0; i < rows; ++i)
-                MB_HIP(hipMemcpyAsync(out + i * width, row.data(), (size_t)width * 4,
-                                      hipMemcpyHostToDevice, s));
-            MB_HIP(hipStreamSynchronize(s));
-            return 0;
-        }
-        reserve(sc.paths, st.paths.size());
-        reserve(sc.elems, st.elems.size());
-        reserve(sc.uniq, st.uniq.size());
-        MB_HIP(hipMemcpyAsync(sc.paths.ptr, st.paths.data(), st.paths.size() * sizeof(mbk::ShapPath),
-                              hipMemcpyHostToDevice, s));
-        MB_HIP(hipMemcpyAsync(sc.elems.ptr, st.elems.data(), st.elems.size() * sizeof(mbk::ShapElem),
-                              hipMemcpyHostToDevice, s));
-        MB_HIP(hipMemcpyAsync(sc.uniq.ptr, st.uniq.data(), st.uniq.size() * sizeof(mbk::ShapUniq),
-                              hipMemcpyHostToDevice, s));
         const uint32_t *mask_dev = nullptr;
         if (mask) {
             const size_t words = (size_t)num_trees * npt * 8;
@@ -586,13 +560,16 @@ int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshol
             MB_HIP(hipMemcpyAsync(sc.shap_mask.ptr, mask, words * 4, hipMemcpyHostToDevice, s));
             mask_dev = sc.shap_mask.ptr;
         }
-        double *phi = nullptr;
-        if (mbk::treeshap_needs_scratch(cols))
-            phi = reserve(sc.phi, (size_t)((rows + 63) / 64) * 64 * (size_t)cols);
-        MB_HIP(mbk::launch_treeshap(s, x, rows, cols, data_bins, mask_dev, sc.paths.ptr,
-                                    (int)st.paths.size(), st.max_elems, sc.elems.ptr, sc.uniq.ptr,
-                                    (float)bias, out, phi));
-        MB_HIP(hipStreamSynchronize(s));
+        const mb::ShapCall call{x, rows, cols, data_bins, mask_dev, (float)bias, out};
+        sc.shap_plan.made = false;                     // this call's forest
+        if (!mb::treeshap(s, trees, 0, 1, nodes_per_tree, call, sc.shap_plan, sc.shap)) {
+            std::vector<float> row((size_t)width, 0.0f);
+            row[(size_t)cols] = (float)bias;
+            for (int64_t i = 0; i < rows; ++i)
+                MB_HIP(hipMemcpyAsync(out + i * width, row.data(), (size_t)width * 4,
+                                      hipMemcpyHostToDevice, s));
+            MB_HIP(hipStreamSynchronize(s));
+        }
         return 0;
     }, -1);
 }

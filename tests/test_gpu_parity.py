@@ -1155,6 +1155,24 @@ def test_treeshap_wide_data_matches_oracle():
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("rows,cols,trees,depth", [
+    (1, 8, 40, 6),            # one row: every share of the columns its own workgroup
+    (2049, 9, 5, 1),          # one-split groups, a row past a row block
+    (2047, 70, 30, 9),        # outcomes of more than 8 bits, features past one finish tile
+    (2000, 8, 60, 9),         # several table sets
+    (70, 4100, 3, 12),        # wide and too deep for tables: the lane-per-row kernel
+])
+def test_treeshap_tables_edges(rows, cols, trees, depth):
+    x, y = O.friedman(30000, cols, 91)
+    x[1, ::7] = np.nan
+    h, obj = gpu_fit(x, y, {"num_trees": trees, "max_depth": depth, "min_child_weight": 0.0,
+                            "lambda": 0.0})
+    xs = np.ascontiguousarray(x[:, :rows])
+    c = mb.predict_contrib(h, xs, feature_major=True)
+    want = O.treeshap(model_io.forest_from_json(obj), obj["baseScore"], obj["numBins"], xs)
+    assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
+
+
 # --------------------------------------------------------------------------
 # Row checks and the base score's sums on the device (k_label_stats)
 # --------------------------------------------------------------------------
