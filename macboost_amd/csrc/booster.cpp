@@ -197,36 +197,56 @@ void Booster::build_forest() {                    // forestBuffers, Booster.swif
         has_cats = has_cats || !t.cat_mask.empty();
     }
     const size_t nt = trees.size(), total = nt * (size_t)nodes;
-    std::vector<int32_t> feat(total, -1);
-    std::vector<float> thr(total, 0.0f), leaf(total, 0.0f);
-    std::vector<uint8_t> flags(total, 0);
-    std::vector<uint32_t> mask(has_cats ? total * 8 : 8, 0u);
+    const size_t mask_at = total * sizeof(mbk::PredNode);
+    const size_t info_at = mask_at + (has_cats ? total * 32 : 0);
+    std::vector<char> image(info_at + mbk::PRED_INFO_WORDS * 4, 0);
+    mbk::PredNode *node = reinterpret_cast<mbk::PredNode *>(image.data());
+    uint32_t *mask = reinterpret_cast<uint32_t *>(image.data() + mask_at);
+    uint32_t *info = reinterpret_cast<uint32_t *>(image.data() + info_at);
+    // the slots of the features the trees split on
+    uint32_t *slot = info + 1 + mbk::PRED_SLOTS, used = 0;
+    bool past = false;
+    for (const Tree &tr : trees)
+        for (int32_t f : tr.feature) {
+            if (f >= mbk::PRED_MAP) past = true;
+            else if (f >= 0) slot[f] = 1;
+        }
+    for (uint32_t f = 0; f < (uint32_t)mbk::PRED_MAP; ++f) {
+        const bool in = slot[f] != 0;
+        slot[f] = used;
+        if (in && used < (uint32_t)mbk::PRED_SLOTS) info[1 + used] = f;
+        used += in;
+    }
+    const bool slots = !past && used <= (uint32_t)mbk::PRED_SLOTS;
+    info[0] = slots ? used : 0xFFFFFFFFu;
     for (size_t t = 0; t < nt; ++t) {
         const Tree &tr = trees[t];
-        for (size_t n = 0; n < tr.feature.size(); ++n) {
-            const size_t k = t * nodes + n;
-            feat[k] = tr.feature[n];
-            thr[k] = n < tr.threshold.size() ? tr.threshold[n] : 0.0f;
-            leaf[k] = n < tr.leaf.size() ? tr.leaf[n] : 0.0f;
-            flags[k] = n < tr.flags.size() ? tr.flags[n] : 0;
-            if (has_cats && tr.cat_mask.size() >= (n + 1) * 8)
-                for (int w = 0; w < 8; ++w) mask[k * 8 + w] = tr.cat_mask[n * 8 + w];
+        const size_t size = tr.feature.size();
+        for (size_t n = 0; n < (size_t)nodes; ++n) {
+            mbk::PredNode &nd = node[t * nodes + n];
+            const int32_t f = n < size ? tr.feature[n] : -1;
+            if (f < 0) {
+                nd = {n < tr.leaf.size() ? tr.leaf[n] : 0.0f, -1};
+                continue;
+            }
+            const int32_t flags = n < tr.flags.size() ? tr.flags[n] & 3 : 0;
+            nd = {n < tr.threshold.size() ? tr.threshold[n] : 0.0f,
+                  (slots ? (int32_t)slot[f] : f) << 2 | flags};
+            if (!has_cats && (flags & mbk::FLAG_CATEGORICAL)) nd = {NAN, nd.meta & ~3};
         }
+        if (has_cats && tr.cat_mask.size() >= size * 8)
+            std::memcpy(mask + t * nodes * 8, tr.cat_mask.data(), size * 32);
     }
-    forest.feature.alloc(total);
-    forest.threshold.alloc(total);
-    forest.flags.alloc(total);
-    forest.leaf.alloc(total);
-    forest.mask.alloc(mask.size());
-    MB_HIP(hipMemcpyAsync(forest.feature.ptr, feat.data(), total * 4, hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(forest.threshold.ptr, thr.data(), total * 4, hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(forest.flags.ptr, flags.data(), total, hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(forest.leaf.ptr, leaf.data(), total * 4, hipMemcpyHostToDevice, d.stream));
-    MB_HIP(hipMemcpyAsync(forest.mask.ptr, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, d.stream));
+    forest.memory.pooled = true;
+    forest.memory.alloc(image.size());
+    MB_HIP(hipMemcpyAsync(forest.memory.ptr, image.data(), image.size(), hipMemcpyHostToDevice,
+                          d.stream));
     MB_HIP(hipStreamSynchronize(d.stream));
+    forest.packed = reinterpret_cast<mbk::PredNode *>(forest.memory.ptr);
+    forest.mask = has_cats ? reinterpret_cast<uint32_t *>(forest.memory.ptr + mask_at) : nullptr;
+    forest.features = reinterpret_cast<uint32_t *>(forest.memory.ptr + info_at);
     forest.nodes_per_tree = nodes;
     forest.num_trees = (int)nt;
-    forest.has_mask = has_cats;
     forest.valid = true;
 }
 
@@ -251,12 +271,12 @@ std::vector<float> Booster::predict_raw(const float *x, int64_t rows, int64_t co
         DevBuf<float> xd((size_t)rows * (size_t)cols), od((size_t)rows * (size_t)K);
         upload(xd.ptr, x, xd.bytes(), d.stream);
         for (int k = 0; k < K; ++k) {
-            mbk::ForestDev f{forest.feature.ptr, forest.threshold.ptr, forest.flags.ptr,
-                             forest.leaf.ptr, forest.has_mask ? forest.mask.ptr : nullptr,
-                             forest.num_trees, forest.nodes_per_tree, k, K, K};
+            const mbk::ForestDev f{nullptr, nullptr, nullptr, nullptr, forest.mask,
+                                   forest.num_trees, forest.nodes_per_tree, k, K, K};
             MB_HIP(mbk::launch_predict_forest(d.stream, f, xd.ptr, rows, trained_num_bins - 1,
                                               K > 1 ? base_scores[(size_t)k] : base_score,
-                                              od.ptr + k));
+                                              od.ptr + k, forest.features, forest.packed,
+                                              num_features));
         }
         MB_HIP(hipMemcpyAsync(out.data(), od.ptr, od.bytes(), hipMemcpyDeviceToHost, d.stream));
         MB_HIP(hipStreamSynchronize(d.stream));
@@ -396,7 +416,7 @@ void Booster::contrib_class(const float *x, int64_t rows, int64_t cols, int k, f
     scratch.pool();
     const StreamIdle idle{d.stream};                   // before the scratch goes back
     const ShapCall call{xd.ptr, rows, (int32_t)cols, trained_num_bins - 1,
-                        forest.has_mask ? forest.mask.ptr : nullptr, bias, od.ptr};
+                        forest.mask, bias, od.ptr};
     if (treeshap(d.stream, tree_views(trees), (size_t)k, (size_t)K, forest.nodes_per_tree, call,
                  shap_plans[(size_t)k], scratch)) {
         download(out, od.ptr, od.bytes(), d.stream);

@@ -194,17 +194,16 @@ struct StreamIdle {
     ~StreamIdle() { (void)hipStreamSynchronize(s); }
 };
 
-// Flattened forest resident on the device (forestBuffers, Booster.swift:1944-1985).
+// The forest resident on the device (forestBuffers, Booster.swift:1944-1985), as
+// the batch walk reads it (launch_forest_pack's arrays, made on the host).
 struct ForestCache {
     bool valid = false;
     int nodes_per_tree = 0;
     int num_trees = 0;
-    bool has_mask = false;
-    DevBuf<int32_t> feature;
-    DevBuf<float> threshold;
-    DevBuf<uint8_t> flags;
-    DevBuf<float> leaf;
-    DevBuf<uint32_t> mask;
+    DevBuf<char> memory;
+    const mbk::PredNode *packed = nullptr;
+    const uint32_t *features = nullptr;
+    const uint32_t *mask = nullptr;      // NULL without categorical splits
 };
 
 // A tree's arrays where they are (a Tree's, or a caller's flat forest).

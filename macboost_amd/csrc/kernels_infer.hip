@@ -31,36 +31,6 @@ __device__ __forceinline__ bool raw_goes_left(float v, uint32_t flags, float thr
     return v <= thr;
 }
 
-__global__ __launch_bounds__(256) void k_predict_forest(ForestDev f, const float *__restrict__ x,
-                                                        int64_t rows, int32_t data_bins, float base,
-                                                        float *__restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows) return;
-    float acc = base;                                  // seeded with the base, trees in order
-    for (int32_t t = f.tree_first; t < f.num_trees; t += f.tree_step) {
-        const int64_t b = (int64_t)t * f.nodes_per_tree;
-        int32_t n = 0;
-        int32_t feat = f.feature[b];
-        while (feat >= 0) {
-            const float v = x[(int64_t)feat * rows + i];
-            const bool left = raw_goes_left(v, f.flags[b + n], f.threshold[b + n],
-                                            f.mask ? f.mask + (b + n) * 8 : nullptr, data_bins);
-            n = 2 * n + 1 + (left ? 0 : 1);
-            feat = f.feature[b + n];
-        }
-        acc += f.leaf[b + n];
-    }
-    out[i * f.out_stride] = acc;
-}
-
-hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x, int64_t rows,
-                                 int32_t data_bins, float base, float *out) {
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_predict_forest, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, f,
-                       x, rows, data_bins, base, out);
-    return hipGetLastError();
-}
-
 // Compute units of the current device (cached per device id).
 static int device_cus() {
     static int cache[64] = {};
@@ -74,6 +44,232 @@ static int device_cus() {
         cache[dev] = n;
     }
     return cache[dev];
+}
+
+// Batch prediction: a workgroup takes 64 rows, a row per lane.  Each of its 16
+// wavefronts walks them down every 16th tree of a chunk, two trees at a time, and
+// leaves their values in LDS, where the first wavefront adds them in tree order
+// (f32, as one thread walking them in turn would: bit for bit).  The first `stage`
+// heap slots of a chunk's trees are staged in LDS as one 8-byte word each
+// (threshold or leaf value; feature and flags, negative at a leaf), and so are the
+// rows' values of the features the forest uses ([slot][64]: lanes reading different
+// features of their own rows hit different banks), so a step of the walk is two LDS
+// reads.  One thread per row took a chain of three dependent global loads per step,
+// each lane's on a line of its own: 100 trees of depth 6 over 100 features took 208
+// us for 1 to 20k rows (15 and 39 us now) and 603 us for 500k (480 us).  Bound by the
+// instructions and LDS latency of a step.  A forest whose nodes fit next to a tile's
+// features (160 KB) is staged once per workgroup; else LDS is held to 80 KB where the
+// features allow it, for two workgroups (32 wavefronts) per CU.
+constexpr int PRED_THREADS = 1024;
+constexpr int PRED_WAVES = PRED_THREADS / 64;
+
+__global__ __launch_bounds__(1024) void k_forest_features(const int32_t *__restrict__ feature,
+                                                          int64_t nodes,
+                                                          uint32_t *__restrict__ info) {
+    __shared__ uint32_t used[PRED_MAP];
+    __shared__ uint32_t tot[16];
+    __shared__ uint32_t past;
+    if (threadIdx.x == 0) past = 0;
+    for (int k = threadIdx.x; k < PRED_MAP; k += 1024) used[k] = 0;
+    __syncthreads();
+    for (int64_t k = threadIdx.x; k < nodes; k += 1024) {
+        const int32_t f = feature[k];
+        if (f >= PRED_MAP) past = 1;
+        else if (f >= 0) used[f] = 1;
+    }
+    __syncthreads();
+    uint32_t u[4], mine = 0;                           // features 4 t .. 4 t + 3
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        u[q] = used[4 * threadIdx.x + q];
+        mine += u[q];
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t p = (uint32_t)__shfl_up((int)incl, o, 64);
+        if (lane >= o) incl += p;
+    }
+    if (lane == 63) tot[wave] = incl;
+    __syncthreads();
+    uint32_t slot = incl - mine, total = 0;
+    for (int w = 0; w < 16; ++w) {
+        if (w < wave) slot += tot[w];
+        total += tot[w];
+    }
+    if (threadIdx.x == 0) info[0] = past || total > (uint32_t)PRED_SLOTS ? 0xFFFFFFFFu : total;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        info[1 + PRED_SLOTS + 4 * threadIdx.x + q] = slot;
+        if (u[q]) {
+            if (slot < (uint32_t)PRED_SLOTS) info[1 + slot] = 4 * threadIdx.x + q;
+            ++slot;
+        }
+    }
+}
+
+// Heap slot g of the forest as a walk reads it, the feature given by its slot
+// when the rows' features are in LDS.
+__device__ __forceinline__ PredNode pred_node(const ForestDev &f, int64_t g, bool in_lds,
+                                              const uint32_t *info) {
+    const int32_t feat = f.feature[g];
+    if (feat < 0) return PredNode{f.leaf[g], -1};
+    const int32_t slot = in_lds ? (int32_t)info[1 + PRED_SLOTS + feat] : feat;
+    const int32_t flags = f.flags[g] & 3;
+    // a categorical split without masks sends every row right
+    if ((flags & FLAG_CATEGORICAL) && !f.mask) return PredNode{NAN, slot << 2};
+    return PredNode{f.threshold[g], slot << 2 | flags};
+}
+
+__global__ __launch_bounds__(256) void k_forest_pack(ForestDev f, int64_t nodes,
+                                                     const uint32_t *__restrict__ info,
+                                                     int32_t max_slots,
+                                                     PredNode *__restrict__ packed) {
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g < nodes) packed[g] = pred_node(f, g, info[0] <= (uint32_t)max_slots, info);
+}
+
+hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
+                              uint32_t *info, PredNode *packed) {
+    const int64_t nodes = (int64_t)f.num_trees * f.nodes_per_tree;
+    hipLaunchKernelGGL(k_forest_features, dim3(1), dim3(1024), 0, s, f.feature, nodes, info);
+    if (packed && nodes > 0)
+        hipLaunchKernelGGL(k_forest_pack, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, s, f,
+                           nodes, info, std::min(max_slots, PRED_SLOTS), packed);
+    return hipGetLastError();
+}
+
+// CAT: the forest has category masks; DEEP: heaps of more than `stage` slots;
+// X_LDS: the rows' features are in LDS.
+template <bool CAT, bool DEEP, bool X_LDS>
+__device__ __forceinline__ void predict_rows(PredNode *pred_lds, const ForestDev &f,
+                                             const float *__restrict__ x, int64_t rows,
+                                             int32_t data_bins, float base,
+                                             float *__restrict__ out,
+                                             const uint32_t *__restrict__ info,
+                                             const PredNode *__restrict__ packed, int32_t chunk,
+                                             int32_t stage, int32_t steps) {
+    const int32_t npt = f.nodes_per_tree;
+    PredNode *s_node = pred_lds;                                          // [chunk][stage]
+    float *s_leaf = reinterpret_cast<float *>(s_node + (size_t)chunk * stage);   // [chunk][64]
+    float *s_x = s_leaf + chunk * 64;                                     // [slots][64]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t mine = f.tree_first < f.num_trees
+                             ? (f.num_trees - f.tree_first + f.tree_step - 1) / f.tree_step : 0;
+    for (int64_t row0 = (int64_t)blockIdx.x * 64; row0 < rows; row0 += (int64_t)gridDim.x * 64) {
+        const int64_t past = rows - 1 - row0;              // rows past the end: the last row
+        const uint32_t r = (int64_t)lane <= past ? (uint32_t)lane : (uint32_t)past;
+        const float *xb = x + row0;
+        if (X_LDS)
+            for (uint32_t c = wave; c < info[0]; c += PRED_WAVES)
+                s_x[c * 64 + lane] = xb[(int64_t)info[1 + c] * rows + r];
+        float acc = base;                                  // seeded with the base, trees in order
+        for (int32_t t0 = 0; t0 < mine; t0 += chunk) {
+            const int32_t nt = min(chunk, mine - t0);
+            auto heap = [&](int32_t t) {                   // chunk tree t's first node
+                return (int64_t)(f.tree_first + (int64_t)(t0 + t) * f.tree_step) * npt;
+            };
+            auto load = [&](int64_t g) { return packed ? packed[g] : pred_node(f, g, X_LDS, info); };
+            // a forest of one chunk stays for every tile of rows
+            for (int32_t t = mine <= chunk && row0 >= (int64_t)gridDim.x * 64 ? nt : wave; t < nt;
+                 t += PRED_WAVES) {
+                const int64_t h = heap(t);
+                for (int32_t n = lane; n < stage; n += 64) s_node[t * stage + n] = load(h + n);
+            }
+            __syncthreads();
+            for (int32_t t = wave; t < nt; t += 2 * PRED_WAVES) {
+                const int32_t t2 = t + PRED_WAVES < nt ? t + PRED_WAVES : t;
+                const int32_t first[2] = {t * stage, t2 * stage};
+                const int64_t h[2] = {heap(t), heap(t2)};
+                int32_t n[2] = {0, 0};
+                PredNode nd[2] = {s_node[first[0]], s_node[first[1]]};
+                for (int32_t d = 0; d < steps; ++d) {
+                    if (__ballot((nd[0].meta & nd[1].meta) >= 0) == 0) break;   // leaves everywhere
+                    float v[2];
+    #pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const int32_t slot = max(nd[j].meta, 0) >> 2;
+                        v[j] = X_LDS ? s_x[slot * 64 + lane] : xb[(int64_t)slot * rows + r];
+                    }
+    #pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const uint32_t meta = (uint32_t)nd[j].meta;
+                        const bool split = nd[j].meta >= 0;
+                        bool left = (v[j] <= nd[j].value) | (isnan(v[j]) & ((meta & FLAG_DEFAULT_LEFT) != 0));
+                        if (CAT && split && (meta & FLAG_CATEGORICAL))
+                            left = raw_goes_left(v[j], FLAG_CATEGORICAL, 0.0f,
+                                                 f.mask + (h[j] + n[j]) * 8, data_bins);
+                        // a leaf stays where it is
+                        n[j] = split ? 2 * n[j] + 2 - (int32_t)left : n[j];
+                        if (!DEEP || n[j] < stage) nd[j] = s_node[first[j] + n[j]];
+                        else if (split) nd[j] = load(h[j] + n[j]);
+                    }
+                }
+                s_leaf[t * 64 + lane] = nd[0].value;
+                s_leaf[t2 * 64 + lane] = nd[1].value;
+            }
+            __syncthreads();
+            if (wave == 0) {
+                int32_t t = 0;
+                for (; t + 8 <= nt; t += 8) {
+                    float v[8];
+    #pragma unroll
+                    for (int j = 0; j < 8; ++j) v[j] = s_leaf[(t + j) * 64 + lane];
+    #pragma unroll
+                    for (int j = 0; j < 8; ++j) acc += v[j];
+                }
+                for (; t < nt; ++t) acc += s_leaf[t * 64 + lane];
+            }
+        }
+        if (wave == 0 && (int64_t)lane <= past) out[(row0 + lane) * f.out_stride] = acc;
+    }
+}
+
+template <bool CAT, bool DEEP>
+__global__ __launch_bounds__(PRED_THREADS) void k_predict_forest(
+    ForestDev f, const float *__restrict__ x, int64_t rows, int32_t data_bins, float base,
+    float *__restrict__ out, const uint32_t *__restrict__ info,
+    const PredNode *__restrict__ packed, int32_t max_slots, int32_t chunk, int32_t stage,
+    int32_t steps) {
+    extern __shared__ PredNode pred_lds[];
+    if (info && info[0] <= (uint32_t)max_slots)
+        predict_rows<CAT, DEEP, true>(pred_lds, f, x, rows, data_bins, base, out, info, packed,
+                                      chunk, stage, steps);
+    else
+        predict_rows<CAT, DEEP, false>(pred_lds, f, x, rows, data_bins, base, out, info, packed,
+                                       chunk, stage, steps);
+}
+
+hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x, int64_t rows,
+                                 int32_t data_bins, float base, float *out, const uint32_t *info,
+                                 const PredNode *packed, int32_t max_slots) {
+    if (rows <= 0) return hipSuccess;
+    const int32_t slots = info ? std::max(0, std::min(max_slots, PRED_SLOTS)) : 0;
+    const int32_t mine =
+        std::max(1, (f.num_trees - f.tree_first + f.tree_step - 1) / f.tree_step);
+    // whole trees up to depth 7, the first seven levels of deeper ones: a chunk
+    // has to hold a tree for every wavefront
+    const int32_t npt = std::max(1, f.nodes_per_tree), stage = npt <= 255 ? npt : 127;
+    const int32_t x_bytes = slots * 64 * 4, tree_bytes = stage * (int32_t)sizeof(PredNode) + 64 * 4;
+    const bool whole = x_bytes + (int64_t)mine * tree_bytes <= 160 << 10;
+    const int32_t budget = (x_bytes <= (40 << 10) ? 80 : 160) << 10;
+    int32_t chunk = (budget - x_bytes) / tree_bytes;
+    if (chunk > PRED_WAVES) chunk -= chunk % PRED_WAVES;   // whole rounds of the wavefronts
+    chunk = whole ? mine : std::max(1, std::min(chunk, mine));
+    const size_t lds = (size_t)chunk * tree_bytes + (size_t)x_bytes;
+    const int64_t tiles = (rows + 63) / 64, resident = lds <= (80 << 10) ? 2 : 1;
+    const int64_t grid = whole ? std::min(tiles, resident * device_cus()) : tiles;
+    int32_t steps = 0;                                 // splits on the longest path of the heap
+    while (steps < 30 && (2 << steps) <= npt) ++steps;
+    const bool deep = npt > stage;
+    auto *kern = f.mask ? (deep ? &k_predict_forest<true, true> : &k_predict_forest<true, false>)
+                        : (deep ? &k_predict_forest<false, true> : &k_predict_forest<false, false>);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(PRED_THREADS), lds, s, f, x,
+                       rows, data_bins, base, out, info, packed, slots, chunk, stage, steps);
+    return hipGetLastError();
 }
 
 // The same walk over the training rows, eight rows per thread walked level by

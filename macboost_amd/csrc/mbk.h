@@ -628,8 +628,29 @@ struct ForestDev {
     int32_t tree_step = 1;
     int32_t out_stride = 1;    // out[i * out_stride]
 };
+// Heap slot as the batch walk reads it.
+struct PredNode {
+    float value;          // threshold, or the leaf's value
+    int32_t meta;         // feature (or its slot) << 2 | flags, or -1
+};
+// A forest prepared for batch walks: the features it splits on in info, and in
+// packed its num_trees * nodes_per_tree heap slots, for walks with the same
+// max_slots.  info[0]: the number of features (0xFFFFFFFF: more than PRED_SLOTS, or
+// one past PRED_MAP), info[1 ..]: those features ascending, info[1 + PRED_SLOTS ..]:
+// the slot of every feature below PRED_MAP.  packed names features by slot when
+// info[0] <= max_slots; its threshold is NaN (every row goes right) at a
+// categorical split of a forest without masks.
+constexpr int PRED_SLOTS = 384;       // features in LDS, at most (96 KB of 64 rows)
+constexpr int PRED_MAP = 4096;        // features the slot map covers
+constexpr size_t PRED_INFO_WORDS = 1 + PRED_SLOTS + PRED_MAP;
+hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
+                              uint32_t *info, PredNode *packed);
+// info and packed as launch_forest_pack made them; either may be NULL.  The rows'
+// features go through LDS when the forest uses at most max_slots.
 hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x,
-                                 int64_t rows, int32_t data_bins, float base, float *out);
+                                 int64_t rows, int32_t data_bins, float base, float *out,
+                                 const uint32_t *info, const PredNode *packed,
+                                 int32_t max_slots);
 hipError_t launch_predict_binned(hipStream_t s, const uint8_t *bins_fm, int64_t rows,
                                  int32_t num_bins, int32_t max_depth, const TreeOut tree,
                                  float *preds);

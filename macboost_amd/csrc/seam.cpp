@@ -63,6 +63,9 @@ struct Scratch {
     mb::ShapPlan shap_plan;                          // mbk_treeshap
     mb::ShapScratch shap;
     DevBuf<uint32_t> shap_mask;
+    // mbk_predict_forest, allocated with the context (its calls allocate nothing)
+    DevBuf<uint32_t> forest_features;
+    DevBuf<mbk::PredNode> nodes;
 };
 
 }  // namespace
@@ -80,6 +83,8 @@ struct mbk_context {
 };
 
 namespace {
+
+constexpr int32_t PREDICT_SLOTS = 160;
 
 void need(bool ok, const char *what) {
     if (!ok) mb::invalid(what);
@@ -215,6 +220,8 @@ int mbk_context_create(int32_t device, mbk_context **out, char **err) {
     return guarded(err, [&]() -> int {
         auto c = std::make_unique<mbk_context>();
         c->dev = std::make_unique<mb::Device>(device);
+        c->scratch.forest_features.alloc(mbk::PRED_INFO_WORDS);
+        c->scratch.nodes.alloc((size_t)1 << 18);
         *out = c.release();
         return 0;
     }, -1);
@@ -510,7 +517,20 @@ int mbk_predict_forest(mbk_context *ctx, const int32_t *feature, const float *th
                        int32_t data_bins, float base_score, float *out, char **err) {
     return guarded(err, [&]() -> int {
         mbk::ForestDev f{feature, threshold, flags, leaf, mask, num_trees, nodes_per_tree, 0, 1, 1};
-        MB_HIP(mbk::launch_predict_forest(ctx->dev->stream, f, x, rows, data_bins, base_score, out));
+        need(ctx != nullptr, "null kernel-seam context");
+        // listing the features and packing the nodes pay for their launches
+        // from some thousand rows on; 160 features in LDS leave room for two
+        // workgroups per CU
+        hipStream_t s = ctx->dev->stream;
+        const Scratch &sc = ctx->scratch;
+        const bool prepared = rows >= 4096;
+        const bool pack = prepared && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
+        if (prepared)
+            MB_HIP(mbk::launch_forest_pack(s, f, PREDICT_SLOTS, sc.forest_features.ptr,
+                                           pack ? sc.nodes.ptr : nullptr));
+        MB_HIP(mbk::launch_predict_forest(s, f, x, rows, data_bins, base_score, out,
+                                          prepared ? sc.forest_features.ptr : nullptr,
+                                          pack ? sc.nodes.ptr : nullptr, PREDICT_SLOTS));
         return 0;
     }, -1);
 }

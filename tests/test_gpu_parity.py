@@ -1155,6 +1155,37 @@ def test_treeshap_wide_data_matches_oracle():
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("cols,trees,depth,leaves", [
+    (1, 1, 1, 0), (5, 3, 1, 0), (9, 33, 3, 0), (70, 65, 6, 0), (12, 40, 7, 0),
+    (9, 17, 8, 0), (9, 5, 12, 31), (500, 80, 6, 0), (4200, 20, 5, 0)])
+def test_predict_forest_edges(cols, trees, depth, leaves):
+    # chunk and wavefront remainders of trees, heaps past the staged levels,
+    # more features than LDS slots or than the slot map covers; host rows and
+    # the seam's (rows below and above its feature list), base and NaN rows
+    rng = np.random.default_rng(cols * 1000 + trees)
+    n = 6000
+    x = rng.random((cols, n), dtype=np.float32)
+    x[0, ::9] = np.nan
+    w = rng.standard_normal(cols).astype(np.float32)
+    y = (np.nan_to_num(x).T @ w + rng.standard_normal(n)).astype(np.float32)
+    params = {"num_trees": trees, "max_depth": depth, "min_child_weight": 0.0}
+    if leaves:
+        params["num_leaves"] = leaves
+    h, obj = gpu_fit(x, y, params)
+    f = model_io.forest_from_json(obj)
+    ctx = mb.Context(0)
+    dev = [ctx.upload(a) for a in (f.feature, f.threshold, f.flags, f.leaf)]
+    for rows in (1, 63, 65, 6000):
+        xs = np.ascontiguousarray(x[:, :rows])
+        want = O.predict(f, obj["baseScore"], obj["numBins"], xs)
+        assert np.array_equal(mb.predict(h, xs, feature_major=True), want)
+        out = ctx.alloc(rows * 4)
+        ctx.call("mbk_predict_forest", *dev, None, f.feature.shape[0], f.feature.shape[1],
+                 ctx.upload(xs), rows, obj["numBins"] - 1, obj["baseScore"], out)
+        ctx.sync()
+        assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
+
+
 @pytest.mark.parametrize("rows,cols,trees,depth", [
     (1, 8, 40, 6),            # one row: every share of the columns its own workgroup
     (2049, 9, 5, 1),          # one-split groups, a row past a row block
