@@ -2111,7 +2111,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 struct CatScratch {
-    float key[256];
+    __align__(16) float key[256];
     int64_t sg[256];
     int64_t sh[256];
     uint32_t mask[8];
@@ -2215,39 +2215,55 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
 
     // Categorical: non-empty bins (missing included) stably sorted by
     // g / (h + catSmooth) (cat_sort, Shaders.swift:339-359), prefixes scanned.
+    // The keys are compacted in bin order, so a lane ranks one non-empty bin
+    // (two to four past 64) against all of them, four keys per broadcast LDS
+    // read: m / 4 steps of one read and four compares.  Ranking each lane's own
+    // four bins against every bin one at a time, the search of a 256-bin level
+    // with a fifth of its columns categorical took 60 us (9 without any).
     bool ne[4];
+    float kb[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int b = b0 + j;
         const float hb = (float)hh[j] * h_inv;
         ne[j] = b < nb && hb > 0.0f;
-        cs->key[b] = ne[j] ? ((float)hg[j] * g_inv) / (hb + sp.cat_smooth) : 0.0f;
-        cs->sg[b] = 0; cs->sh[b] = 0;
+        kb[j] = ne[j] ? ((float)hg[j] * g_inv) / (hb + sp.cat_smooth) : 0.0f;
     }
     const uint64_t ne_bits0 = __ballot(ne[0]), ne_bits1 = __ballot(ne[1]);
     const uint64_t ne_bits2 = __ballot(ne[2]), ne_bits3 = __ballot(ne[3]);
+    const int m = __popcll(ne_bits0) + __popcll(ne_bits1) + __popcll(ne_bits2) + __popcll(ne_bits3);
+    int pos[4];
+    pos[0] = (int)(lanes_below(ne_bits0) + lanes_below(ne_bits1) + lanes_below(ne_bits2) +
+                   lanes_below(ne_bits3));
+#pragma unroll
+    for (int j = 1; j < 4; ++j) pos[j] = pos[j - 1] + (ne[j - 1] ? 1 : 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (ne[j]) cs->key[pos[j]] = kb[j];
+    if (lane < 3 && m + lane < 256) cs->key[m + lane] = NAN;   // the last read's tail ranks nobody
     if (lane < 8) cs->mask[lane] = 0;
     wave_lds_sync();
-    const int m = __popcll(ne_bits0) + __popcll(ne_bits1) + __popcll(ne_bits2) + __popcll(ne_bits3);
+    uint32_t *ranks = reinterpret_cast<uint32_t *>(cs->sg);    // by compact position, for now
+    for (int e0 = 0; e0 < m; e0 += 64) {             // uniform
+        const int e = e0 + lane;
+        const float ke = e < m ? cs->key[e] : 0.0f;
+        int r = 0;
+        for (int c = 0; c < m; c += 4) {
+            const float4 k4 = *reinterpret_cast<const float4 *>(&cs->key[c]);
+            r += (k4.x < ke || (k4.x == ke && c < e)) ? 1 : 0;
+            r += (k4.y < ke || (k4.y == ke && c + 1 < e)) ? 1 : 0;
+            r += (k4.z < ke || (k4.z == ke && c + 2 < e)) ? 1 : 0;
+            r += (k4.w < ke || (k4.w == ke && c + 3 < e)) ? 1 : 0;
+        }
+        if (e < m) ranks[e] = (uint32_t)r;
+    }
+    wave_lds_sync();
     int rank[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        rank[j] = -1;
-        if (ne[j]) {
-            const int b = b0 + j;
-            const float kb = cs->key[b];
-            int r = 0;
-            for (int c = 0; c < nb; ++c) {
-                const int cl = c >> 2, cj = c & 3;
-                const uint64_t bits = cj == 0 ? ne_bits0 : cj == 1 ? ne_bits1 : cj == 2 ? ne_bits2 : ne_bits3;
-                if ((bits >> cl) & 1ull) {
-                    const float kc = cs->key[c];
-                    r += (kc < kb || (kc == kb && c < b)) ? 1 : 0;
-                }
-            }
-            rank[j] = r;
-        }
-    }
+    for (int j = 0; j < 4; ++j) rank[j] = ne[j] ? (int)ranks[pos[j]] : -1;
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { cs->sg[b0 + j] = 0; cs->sh[b0 + j] = 0; }
     wave_lds_sync();
 #pragma unroll
     for (int j = 0; j < 4; ++j)

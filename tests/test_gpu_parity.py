@@ -1155,6 +1155,22 @@ def test_treeshap_wide_data_matches_oracle():
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
+def test_categorical_rank_sizes(card):
+    # the split search ranks a node's categories 64 at a time, four keys a read:
+    # counts at the edges of both, missing values, and labels of few distinct
+    # values so that many categories share a key
+    rng = np.random.default_rng(card)
+    n = 20000
+    x = np.stack([rng.integers(0, card, n), rng.integers(0, max(1, card // 2), n),
+                  rng.random(n)]).astype(np.float32)
+    x[0, rng.random(n) < 0.05] = np.nan
+    y = ((x[1] % 3 == 1) + (np.nan_to_num(x[0]) % 5 == 2)).astype(np.float32)
+    check_identical(np.ascontiguousarray(x), y,
+                    {"num_trees": 2, "max_depth": 4, "num_bins": 256,
+                     "categorical_features": [0, 1]}, is_cat=[1, 1, 0])
+
+
 @pytest.mark.parametrize("cols,trees,depth,leaves", [
     (1, 1, 1, 0), (5, 3, 1, 0), (9, 33, 3, 0), (70, 65, 6, 0), (12, 40, 7, 0),
     (9, 17, 8, 0), (9, 5, 12, 31), (500, 80, 6, 0), (4200, 20, 5, 0)])
