@@ -272,7 +272,7 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
     return hipGetLastError();
 }
 
-// The same walk over the training rows, eight rows per thread walked level by
+// The walk over the training rows, up to eight rows per thread walked level by
 // level together, that also counts the rows reaching each node of the deepest
 // level (counters in LDS, one global add per non-empty node per block).  The
 // split records (feature, bin | flags << 8) and leaf values are staged in LDS,
@@ -280,8 +280,13 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
 // With GRAD the walk also starts the next tree's gradient pass on the updated
 // predictions: per-block maxima of |g| and h into gpart (as k_grad_max's
 // partials) and, with g_out / h_out, every row's g and h.
-constexpr int WALK_THREADS = 1024;
-constexpr int WALK_ROWS = 8;
+// Rows per thread R and threads per block T go by the rows (walk_rows): R
+// independent rows hide the levels' gathers where there are rows enough to fill
+// the chip, but a few blocks of 8,192 rows each leave it idle (20k rows, depth 6:
+// three blocks, 24.3 us; 79 blocks of 256 single rows, 6.8 us; 1M rows 35.3 -> 22.0
+// us with 2 rows per thread, 2M 30.5 -> 26.4 with 4; 200k without gradients 27.9 ->
+// 6.8 with 1).
+constexpr int WALK_MAX_BLOCKS = 512;                   // two 1,024-thread blocks per CU
 
 struct WalkGrad {
     GradParams gp;
@@ -291,7 +296,7 @@ struct WalkGrad {
     float *g_out, *h_out;
 };
 
-template <bool GRAD>
+template <bool GRAD, int WALK_THREADS, int WALK_ROWS>
 __global__ __launch_bounds__(WALK_THREADS, 8) void k_walk_count(const uint8_t *__restrict__ bins_fm,
                                                              int64_t rows, int32_t nb,
                                                              int32_t max_depth, TreeOut tree,
@@ -330,6 +335,17 @@ __global__ __launch_bounds__(WALK_THREADS, 8) void k_walk_count(const uint8_t *_
                 if (i < rows && !kept[i]) counts &= ~(1u << k);
             }
         }
+        // few rows per thread: their predictions and labels load before the walk
+        constexpr bool EARLY = WALK_ROWS <= 2;
+        float early_p[WALK_ROWS], early_y[WALK_ROWS];
+        if (EARLY && preds) {
+#pragma unroll
+            for (int k = 0; k < WALK_ROWS; ++k) {
+                const int64_t i = base + (int64_t)k * WALK_THREADS;
+                early_p[k] = i < rows ? preds[i] : 0.0f;
+                early_y[k] = GRAD && i < rows ? wg.labels[i] : 0.0f;
+            }
+        }
         for (int32_t d = 0; d < max_depth; ++d) {
             uint32_t b[WALK_ROWS];
 #pragma unroll
@@ -355,12 +371,12 @@ __global__ __launch_bounds__(WALK_THREADS, 8) void k_walk_count(const uint8_t *_
             const int64_t i = base + (int64_t)k * WALK_THREADS;
             if (i >= rows) continue;
             if (preds) {                             // null: counts only
-                const float np = preds[i] + s_leaf[n[k]];
+                const float np = (EARLY ? early_p[k] : preds[i]) + s_leaf[n[k]];
                 preds[i] = np;
                 if (GRAD) {
                     float g, h;
                     const float w = wg.gp.has_weights ? wg.weights[i] : 1.0f;
-                    row_grad(wg.gp, np, wg.labels[i], w, g, h);
+                    row_grad(wg.gp, np, EARLY ? early_y[k] : wg.labels[i], w, g, h);
                     mg = max(mg, __float_as_uint(fabsf(g)));
                     mh = max(mh, __float_as_uint(h));
                     if (wg.g_out) { wg.g_out[i] = g; wg.h_out[i] = h; }
@@ -390,22 +406,39 @@ __global__ __launch_bounds__(WALK_THREADS, 8) void k_walk_count(const uint8_t *_
         if (s_cnt[k]) atomicAdd(&count[deep_start + k], s_cnt[k]);
 }
 
-static int64_t walk_grid(int64_t rows) {
-    const int64_t per = (int64_t)WALK_THREADS * WALK_ROWS;
-    // two 1024-thread blocks per CU, or one block per chunk when fewer
-    return std::max<int64_t>(1, std::min<int64_t>((rows + per - 1) / per, 2 * (int64_t)device_cus()));
+// Launches the walk with the rows per thread that fill 512 blocks (or, below
+// 131,072 rows, with single rows in 256-thread blocks); returns the grid.
+template <bool GRAD>
+static hipError_t walk_rows(hipStream_t s, const uint8_t *bins_fm, int64_t rows, int32_t num_bins,
+                            int32_t max_depth, const TreeOut &tree, float *preds, uint32_t *count,
+                            const uint8_t *kept, const WalkGrad &wg, int *blocks) {
+    const size_t deep = (size_t)1 << max_depth;
+    const size_t lds = (deep + 2 * (deep - 1) + (2 * deep - 1)) * sizeof(uint32_t);
+    int64_t grid = 0;
+#define MBK_WALK(T, R)                                                                           \
+    {                                                                                            \
+        grid = std::min<int64_t>((rows + (T) * (R) - 1) / ((T) * (R)), WALK_MAX_BLOCKS);         \
+        auto *kern = &k_walk_count<GRAD, T, R>;                                                  \
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(T), lds, s, bins_fm, rows, num_bins, \
+                           max_depth, tree, preds, count, kept, wg);                             \
+    }
+    if (rows <= 256 * WALK_MAX_BLOCKS) MBK_WALK(256, 1)
+    else if (rows <= 1024 * WALK_MAX_BLOCKS) MBK_WALK(1024, 1)
+    else if (rows <= 2048 * WALK_MAX_BLOCKS) MBK_WALK(1024, 2)
+    else if (rows <= 4096 * WALK_MAX_BLOCKS) MBK_WALK(1024, 4)
+    else MBK_WALK(1024, 8)
+#undef MBK_WALK
+    *blocks = (int)grid;
+    return hipGetLastError();
 }
 
 hipError_t launch_walk_count(hipStream_t s, const uint8_t *bins_fm, int64_t rows,
                              int32_t num_bins, int32_t max_depth, const TreeOut tree,
                              float *preds, uint32_t *count, const uint8_t *kept) {
     if (rows <= 0) return hipSuccess;
-    const size_t deep = (size_t)1 << max_depth;
-    const size_t lds = (deep + 2 * (deep - 1) + (2 * deep - 1)) * sizeof(uint32_t);
-    hipLaunchKernelGGL(k_walk_count<false>, dim3((unsigned)walk_grid(rows)), dim3(WALK_THREADS),
-                       lds, s, bins_fm, rows, num_bins, max_depth, tree, preds, count, kept,
-                       WalkGrad{});
-    return hipGetLastError();
+    int blocks = 0;
+    return walk_rows<false>(s, bins_fm, rows, num_bins, max_depth, tree, preds, count, kept,
+                            WalkGrad{}, &blocks);
 }
 
 hipError_t launch_walk_count_grad(hipStream_t s, const uint8_t *bins_fm, int64_t rows,
@@ -417,14 +450,8 @@ hipError_t launch_walk_count_grad(hipStream_t s, const uint8_t *bins_fm, int64_t
     *partials = 0;
     if (rows <= 0 || !preds) return hipErrorInvalidValue;
     if (gp.objective == 7) return hipErrorInvalidValue;   // one output per row only
-    const size_t deep = (size_t)1 << max_depth;
-    const size_t lds = (deep + 2 * (deep - 1) + (2 * deep - 1)) * sizeof(uint32_t);
-    const int64_t grid = walk_grid(rows);
-    hipLaunchKernelGGL(k_walk_count<true>, dim3((unsigned)grid), dim3(WALK_THREADS), lds, s,
-                       bins_fm, rows, num_bins, max_depth, tree, preds, count, kept,
-                       WalkGrad{gp, labels, weights, gpart, g_out, h_out});
-    *partials = (int)grid;
-    return hipGetLastError();
+    return walk_rows<true>(s, bins_fm, rows, num_bins, max_depth, tree, preds, count, kept,
+                           WalkGrad{gp, labels, weights, gpart, g_out, h_out}, partials);
 }
 
 // Binned single-tree prediction (predict_tree_binned, Shaders.swift:1763-1781):
