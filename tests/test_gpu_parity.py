@@ -1155,6 +1155,18 @@ def test_treeshap_wide_data_matches_oracle():
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("rows,depth,objective", [
+    (3, 2, "mae"), (8191, 1, "mae"), (8193, 1, "quantile"), (40000, 1, "mae"),
+    (300001, 2, "quantile")])
+def test_leaf_renewal_sizes(rows, depth, objective):
+    # leaves of fewer than four keys, around the keys a workgroup holds in
+    # registers and far past them; repeated residuals
+    x, y = O.friedman(rows, 6, 17)
+    y = np.round(y * 4) / 4
+    check_identical(x, y.astype(np.float32), {"num_trees": 2, "max_depth": depth,
+                                              "objective": objective, "alpha": 0.3})
+
+
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
 def test_categorical_rank_sizes(card):
     # the split search ranks a node's categories 64 at a time, four keys a read:
