@@ -866,9 +866,9 @@ static float base_score(const Params &p, const float *y, const float *w, int64_t
         const int64_t step = std::max<int64_t>(1, n / 200000);
         std::vector<float> s;
         for (int64_t i = 0; i < n; i += step) s.push_back(y[i]);
-        std::sort(s.begin(), s.end());
         const int64_t idx = std::min<int64_t>((int64_t)s.size() - 1,
                                               (int64_t)((float)s.size() * q));
+        std::nth_element(s.begin(), s.begin() + idx, s.end());
         return s[(size_t)idx];
     }
     const int64_t nblocks = (n + SUM_BLOCK - 1) / SUM_BLOCK;
@@ -1076,14 +1076,52 @@ static void setup_shape(Trainer &t, int64_t rows, int64_t cols) {
 }
 
 // Bins a raw feature-major validation set with the training edges (device).
-static void bin_valid(Trainer &t, const float *xv, int64_t vrows, const float *edges_dev) {
+// The categorical id rule on raw features in device memory (as
+// validate_categoricals on the host, which then words the error): first[j] is the
+// first offending row of the j-th categorical column, all ones if none.  Queued on
+// s; the results are there once s has drained.
+struct CategoricalCheck {
+    DevBuf<int32_t> cols;                            // pooled: s drains before they go
+    DevBuf<uint32_t> bad;
+    std::vector<int32_t> cols_h;
+    std::vector<uint32_t> first;
+    void queue(const Params &p, const float *x, int64_t rows, int64_t rs, int64_t cs,
+               hipStream_t s) {
+        cols_h.assign(p.categorical.begin(), p.categorical.end());
+        if (cols_h.empty()) return;
+        first.assign(cols_h.size(), mbk::NONE);
+        cols.pooled = bad.pooled = true;
+        cols.alloc(cols_h.size());
+        bad.alloc(cols_h.size());
+        MB_HIP(hipMemcpyAsync(cols.ptr, cols_h.data(), cols.bytes(), hipMemcpyHostToDevice, s));
+        MB_HIP(hipMemsetAsync(bad.ptr, 0xFF, bad.bytes(), s));
+        MB_HIP(mbk::launch_check_categorical(s, x, rows, rs, cs, cols.ptr, (int)cols_h.size(),
+                                             p.num_bins - 1, bad.ptr));
+        MB_HIP(hipMemcpyAsync(first.data(), bad.ptr, bad.bytes(), hipMemcpyDeviceToHost, s));
+    }
+    bool failed() const {
+        for (uint32_t r : first)
+            if (r != mbk::NONE) return true;
+        return false;
+    }
+};
+
+// Validation features to the device and into bins; check, when given, also
+// checks their categorical ids.  Waits for the stream.
+static void bin_valid(Trainer &t, const float *xv, int64_t vrows, const float *edges_dev,
+                      CategoricalCheck *check = nullptr) {
     hipStream_t s = t.dev->stream;
     t.has_valid = true;
     t.vrows = vrows;
-    DevBuf<float> xvd((size_t)vrows * (size_t)t.cols);
-    DevBuf<uint8_t> vt((size_t)t.sh.num_tiles * (size_t)vrows * (size_t)t.sh.tile_w);
+    DevBuf<float> xvd;
+    DevBuf<uint8_t> vt;
+    xvd.pooled = vt.pooled = true;
+    const StreamIdle idle{s};                        // before they go back to the cache
+    xvd.alloc((size_t)vrows * (size_t)t.cols);
+    vt.alloc((size_t)t.sh.num_tiles * (size_t)vrows * (size_t)t.sh.tile_w);
     t.vbins_fm.alloc((size_t)vrows * (size_t)t.cols);
-    MB_HIP(hipMemcpyAsync(xvd.ptr, xv, xvd.bytes(), hipMemcpyHostToDevice, s));
+    upload(xvd.ptr, xv, xvd.bytes(), s);
+    if (check) check->queue(t.p, xvd.ptr, vrows, 1, vrows, s);
     MB_HIP(mbk::launch_bin_data(s, xvd.ptr, vrows, t.cols, 1, vrows, edges_dev, t.is_cat.ptr,
                                 t.nb, t.sh.tile_w, t.sh.num_tiles, vt.ptr, t.vbins_fm.ptr));
     MB_HIP(hipStreamSynchronize(s));
@@ -1396,6 +1434,15 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
     // reference's order: a later check's error is reported only when the row
     // checks pass.
     const bool dev_rows = sums_base(pin);
+    // Categorical ids are checked on the device once the features are there; a
+    // failure, or any error from where the host check stood, words the host
+    // check's error (after the row checks').
+    bool cats_due = false;
+    auto check_categoricals = [&] {
+        if (!x_on_device)
+            validate_categoricals(pin, x, rows, cols, row_major ? cols : 1, row_major ? 1 : rows);
+        if (xv && yv && vrows > 0) validate_categoricals(pin, xv, vrows, cols, 1, vrows);
+    };
     struct HostPrep {
         std::thread th;
         std::exception_ptr err;
@@ -1453,9 +1500,10 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
                     leak_error = std::current_exception();
                 }
             });
-            validate_categoricals(p, x, rows, cols, rs, cs);
         }
-        if (xv && yv && vrows > 0) validate_categoricals(p, xv, vrows, cols, 1, vrows);
+        cats_due = true;
+        for (int f : p.categorical)
+            if (f < 0 || f >= cols) check_categoricals();
         setup_shape(t, rows, cols);
         hipStream_t s = t.dev->stream;
         const int tile_w = t.sh.tile_w;
@@ -1476,6 +1524,8 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
 
         // --- binning on the device: (upload,) quantile edges, bin_data --------
         std::vector<mbk::LabelStats> row_stats;       // the device row checks' blocks
+        CategoricalCheck cat_train, cat_valid;
+        const StreamIdle idle{s};                    // before the checks' buffers go back
         double t0 = now_s(), te = t0;
         struct Events {                              // destroyed after the streams drained
             std::vector<hipEvent_t> ev;
@@ -1544,6 +1594,7 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
                                             p.num_bins, tile_w, t.sh.num_tiles, t.bins_tiled.ptr,
                                             t.bins_fm.ptr));
             }
+            if (!x_on_device) cat_train.queue(p, xsrc, rows, rs, cs, s);
             // the root pass's planar copy follows the binning on the compute
             // stream, and the labels cross PCIe and are checked meanwhile; the
             // edges' copy to the host waits for both kernels
@@ -1575,7 +1626,7 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
             t.edges.resize((size_t)cols * ne);
             MB_HIP(hipMemcpyAsync(t.edges.data(), ed.ptr, t.edges.size() * 4, hipMemcpyDeviceToHost, s));
             MB_HIP(hipStreamSynchronize(cs2));
-            if (xv && yv && vrows > 0) bin_valid(t, xv, vrows, ed.ptr);
+            if (xv && yv && vrows > 0) bin_valid(t, xv, vrows, ed.ptr, &cat_valid);
             MB_HIP(hipStreamSynchronize(s));
             t.t_edges = now_s() - te;
         }
@@ -1598,6 +1649,10 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
                         "; weights must be finite and >= 0");
             if (xv && yv && vrows > 0) validate_labels(p, yv, vrows);
             prep.bases = {base_from_sums(p, s1, s2)};
+        }
+        if (cat_train.failed() || cat_valid.failed()) {
+            check_categoricals();
+            internal("categorical check failed");
         }
         Phase ph_rest("labels, buffers");
         if (leak.th.joinable()) leak.th.join();
@@ -1627,6 +1682,7 @@ static Trainer *create_raw(const Params &pin, const float *x, bool x_on_device, 
         prep.join();
         if (prep.err) std::rethrow_exception(prep.err);
         if (dev_rows) validate_rows(pin, rows, y, w, xv, vrows, yv);
+        if (cats_due) check_categoricals();
         throw;
     }
 }
