@@ -654,6 +654,16 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
 hipError_t launch_predict_binned(hipStream_t s, const uint8_t *bins_fm, int64_t rows,
                                  int32_t num_bins, int32_t max_depth, const TreeOut tree,
                                  float *preds);
+// Block sums of a metric's terms over the rows (metric_blocks(rows) doubles into
+// partial); param: the quantile's alpha or Tweedie's rho.
+enum Metric : int {
+    METRIC_RMSE, METRIC_MAE, METRIC_PINBALL, METRIC_LOGLOSS, METRIC_POISSON, METRIC_TWEEDIE,
+    METRIC_MULTI_LOGLOSS, METRIC_HOST,               // HOST: not a sum of terms (auc)
+};
+int metric_blocks(int64_t rows);
+hipError_t launch_metric(hipStream_t s, int metric, double param, int32_t num_classes,
+                         const float *preds, const float *labels, int64_t rows,
+                         double *partial);
 // Training-row walk of a finished tree: preds += leaf (unless preds is null),
 // and rows per node of the deepest level added to count[2^D - 1 ...] (unless
 // count is null; with kept non-null only rows with kept[i] != 0 count).

@@ -613,6 +613,12 @@ struct Trainer {
     int stale = 0;
     bool stopped = false;
     std::vector<float> eval_history;
+    // the metric's block sums of the rounds not read back yet (launch_metric)
+    static constexpr int METRIC_SLOTS = 256;
+    int metric = mbk::METRIC_HOST;
+    int metric_pending = 0;
+    DevBuf<float> vlabels;
+    DevBuf<double> metric_part;
     std::vector<std::string> warnings;
     double t_edges = 0.0, t_bin = 0.0;
 
@@ -623,7 +629,7 @@ struct Trainer {
         for (DevBuf<uint8_t> *b : {&bins_tiled, &bins_fm, &vbins_fm, &bins_root, &kept, &is_cat,
                                    &feat_mask})
             b->pooled = true;
-        for (DevBuf<float> *b : {&labels, &weights, &preds, &vpreds, &samp_g, &samp_h,
+        for (DevBuf<float> *b : {&labels, &weights, &preds, &vpreds, &vlabels, &samp_g, &samp_h,
                                  &samp_h_kept, &rn_delta, &spec_cover})
             b->pooled = true;
         for (DevBuf<uint32_t> *b : {&gmax_part, &goss_buckets, &count, &seg_a, &seg_b, &rn_leaf,
@@ -632,7 +638,7 @@ struct Trainer {
         for (DevBuf<int64_t> *b : {&hist_a, &hist_b, &node_g, &node_h}) b->pooled = true;
         order_a.pooled = order_b.pooled = partials.pooled = items.pooled = true;
         mono.pooled = route_cursor.pooled = pairs.pooled = results.pooled = true;
-        route_done.pooled = true;
+        route_done.pooled = metric_part.pooled = true;
         bounds.pooled = ctl.pooled = true;
         lw_state.pooled = lw_open.pooled = lwb_state.pooled = lwb_cand.pooled = true;
         spec_split.pooled = true;
@@ -902,6 +908,19 @@ static std::string effective_metric(const Params &p) {
     case OBJ_MULTICLASS: return "multi_logloss";
     default: return "rmse";
     }
+}
+
+// The metric as the device sums it (the others rank: on the host).
+static int device_metric(const Params &p, int K) {
+    if (K > 1) return mbk::METRIC_MULTI_LOGLOSS;
+    const std::string m = effective_metric(p);
+    if (m == "rmse") return mbk::METRIC_RMSE;
+    if (m == "mae") return mbk::METRIC_MAE;
+    if (m == "pinball") return mbk::METRIC_PINBALL;
+    if (m == "logloss") return mbk::METRIC_LOGLOSS;
+    if (m == "poisson") return mbk::METRIC_POISSON;
+    if (m == "tweedie") return mbk::METRIC_TWEEDIE;
+    return mbk::METRIC_HOST;
 }
 
 // evalMetricRaw (Booster.swift:1855-1918).
@@ -1213,6 +1232,13 @@ static void setup_buffers(Trainer &t, const float *y, const float *w, const floa
     t.base = K > 1 ? 0.0f : t.base_scores[0];
     if (t.has_valid) {
         t.vlabels_h.assign(yv, yv + vrows);
+        t.metric = device_metric(p, K);
+        if (t.metric != mbk::METRIC_HOST) {
+            t.vlabels.alloc((size_t)vrows);
+            upload(t.vlabels.ptr, t.vlabels_h.data(), (size_t)vrows * 4, s);
+            t.metric_part.alloc((size_t)Trainer::METRIC_SLOTS *
+                                (size_t)mbk::metric_blocks(vrows));
+        }
         t.vpreds.alloc((size_t)vrows * (size_t)K);
     }
     for (int k = 0; k < K; ++k) {
@@ -2240,6 +2266,37 @@ void trainer_grow(Trainer *tp, int num_trees) {
     auto metric = [&](const float *pred, const float *y, int64_t n) {
         return K > 1 ? multiclass_logloss(pred, y, n, K) : eval_metric(t.p, pred, y, n);
     };
+    // One round's validation metric into the history (Booster.swift:1665-1688).
+    auto record = [&](float vm, int round) {
+        t.eval_history.push_back(vm);
+        const bool higher = effective_metric(t.p) == "auc";
+        if (higher ? vm > t.best_metric : vm < t.best_metric) {
+            t.best_metric = vm;
+            t.best_iter = round;
+            t.stale = 0;
+        } else {
+            t.stale += 1;
+        }
+    };
+    // The rounds whose metric the device has summed: the block sums added in
+    // order, in double.
+    const bool dev_metric = t.has_valid && t.metric != mbk::METRIC_HOST;
+    const size_t mblocks = dev_metric ? (size_t)mbk::metric_blocks(t.vrows) : 0;
+    auto flush_metrics = [&] {
+        if (t.metric_pending == 0) return;
+        std::vector<double> part((size_t)t.metric_pending * mblocks);
+        MB_HIP(hipMemcpyAsync(part.data(), t.metric_part.ptr, part.size() * sizeof(double),
+                              hipMemcpyDeviceToHost, s));
+        MB_HIP(hipStreamSynchronize(s));
+        const int first = t.grown / K - t.metric_pending + 1;
+        for (int r = 0; r < t.metric_pending; ++r) {
+            double sum = 0;
+            for (size_t b = 0; b < mblocks; ++b) sum += part[(size_t)r * mblocks + b];
+            const double mean = sum / (double)t.vrows;
+            record((float)(t.metric == mbk::METRIC_RMSE ? std::sqrt(mean) : mean), first + r);
+        }
+        t.metric_pending = 0;
+    };
     for (int k = 0; k < num_trees && !t.stopped; ++k) {
         const int tree = t.grown;
         // tree t fits class t % K (Booster.swift:1315)
@@ -2257,6 +2314,15 @@ void trainer_grow(Trainer *tp, int num_trees) {
         const bool is_last = k + 1 == num_trees;
         const bool log_now = t.p.eval_every > 0 && (round % t.p.eval_every == 0 || is_last);
         if (!metric_each_tree && !log_now) continue;
+        if (dev_metric) {
+            const double param = t.metric == mbk::METRIC_TWEEDIE ? t.p.tweedie_power : t.p.alpha;
+            MB_HIP(mbk::launch_metric(s, t.metric, param, K, t.vpreds.ptr, t.vlabels.ptr, t.vrows,
+                                      t.metric_part.ptr + (size_t)t.metric_pending * mblocks));
+            // read back only when this round's value is needed now
+            if (++t.metric_pending < Trainer::METRIC_SLOTS && !log_now &&
+                t.p.early_stopping_rounds <= 0)
+                continue;
+        }
         MB_HIP(hipStreamSynchronize(s));
         std::string line;
         if (log_now) {
@@ -2274,18 +2340,14 @@ void trainer_grow(Trainer *tp, int num_trees) {
             line = buf;
         }
         if (t.has_valid) {
-            vp.resize((size_t)t.vrows * (size_t)K);
-            MB_HIP(hipMemcpy(vp.data(), t.vpreds.ptr, vp.size() * 4, hipMemcpyDeviceToHost));
-            const float vm = metric(vp.data(), t.vlabels_h.data(), t.vrows);
-            t.eval_history.push_back(vm);
-            const bool higher = effective_metric(t.p) == "auc";
-            if (higher ? vm > t.best_metric : vm < t.best_metric) {
-                t.best_metric = vm;
-                t.best_iter = round;
-                t.stale = 0;
+            if (dev_metric) {
+                flush_metrics();
             } else {
-                t.stale += 1;
+                vp.resize((size_t)t.vrows * (size_t)K);
+                MB_HIP(hipMemcpy(vp.data(), t.vpreds.ptr, vp.size() * 4, hipMemcpyDeviceToHost));
+                record(metric(vp.data(), t.vlabels_h.data(), t.vrows), round);
             }
+            const float vm = t.eval_history.back();
             if (log_now) {
                 char buf[96];
                 std::snprintf(buf, sizeof buf, "   valid-%s: %.5f", effective_metric(t.p).c_str(), vm);
@@ -2302,6 +2364,7 @@ void trainer_grow(Trainer *tp, int num_trees) {
         }
         if (t.p.verbose && !line.empty()) std::printf("%s\n", line.c_str());
     }
+    flush_metrics();
     if (t.fix_pending.active) {                      // the last tree's deepest covers
         const mbk::PendingFixup &f = t.fix_pending;
         MB_HIP(mbk::launch_final_fixup(s, f.la, f.count, t.tree_out(t.fix_tree),

@@ -1167,6 +1167,54 @@ def test_leaf_renewal_sizes(rows, depth, objective):
                                               "objective": objective, "alpha": 0.3})
 
 
+@pytest.mark.parametrize("objective,vrows", [
+    ("regression", 1), ("mae", 255), ("quantile", 257), ("binary", 70001), ("poisson", 5000),
+    ("tweedie", 66000), ("huber", 300), ("multiclass", 4099)])
+def test_validation_metric_on_device(objective, vrows):
+    # the device's block sums against a float64 restatement of the last round's
+    # metric (one f32 rounding apart at most), over several grow calls and more
+    # rounds than one readback holds
+    rng = np.random.default_rng(vrows)
+    x, y = O.friedman(2000 + vrows, 7, 5)
+    if objective == "binary":
+        y = (y > 14).astype(np.float32)
+    elif objective == "multiclass":
+        y = (y // 10).clip(0, 2).astype(np.float32)
+    elif objective in ("poisson", "tweedie"):
+        y = rng.poisson(np.exp(y / 20)).astype(np.float32)
+    xt, xv = np.ascontiguousarray(x[:, :2000]), np.ascontiguousarray(x[:, 2000:])
+    yt, yv = y[:2000], y[2000:]
+    params = {"num_trees": 1, "max_depth": 2, "objective": objective, "alpha": 0.7}
+    if objective == "huber":
+        params["alpha"] = 1.0
+    K = 3 if objective == "multiclass" else 1
+    if K > 1:
+        params["num_class"] = K
+    t = mb.Trainer(params, xt, yt, eval_set=(xv.T, yv), feature_major=True)
+    for n in (3, 260, 1):
+        t.grow(n * K)
+    h = t.booster()
+    hist = mb.eval_history(h)
+    assert hist.shape == (264,)
+    p, v = mb.predict(h, xv, feature_major=True).astype(np.float64), yv.astype(np.float64)
+    if objective in ("regression", "huber"):
+        want = np.sqrt(np.mean((p - v) ** 2))
+    elif objective == "mae":
+        want = np.mean(np.abs(p - v))
+    elif objective == "quantile":
+        want = np.mean(np.where(v >= p, 0.7 * (v - p), -0.3 * (v - p)))
+    elif objective == "binary":
+        q = 1 / (1 + np.exp(-p))
+        want = -np.mean(v * np.log(q) + (1 - v) * np.log(1 - q))
+    elif objective == "multiclass":
+        m = p.max(axis=1, keepdims=True)
+        logp = p - m - np.log(np.exp(p - m).sum(axis=1, keepdims=True))
+        want = -np.mean(logp[np.arange(vrows), yv.astype(int)])
+    else:
+        return                      # predictions are on the exp scale, rounded to f32
+    assert np.isclose(hist[-1], want, rtol=3e-7, atol=0)
+
+
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
 def test_categorical_rank_sizes(card):
     # the split search ranks a node's categories 64 at a time, four keys a read:
