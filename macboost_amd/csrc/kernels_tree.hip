@@ -1043,8 +1043,10 @@ static int grad_max_blocks(int64_t rows) {
 
 hipError_t launch_grad_max(hipStream_t s, const GradParams &gp, const float *preds,
                            const float *labels, const float *weights, int64_t rows,
-                           TreeCtl *ctl, uint32_t *partial, float *g_out, float *h_out) {
+                           TreeCtl *ctl, uint32_t *partial, float *g_out, float *h_out,
+                           int *partials) {
     const int blocks = grad_max_blocks(rows);
+    if (partials) *partials = blocks;
     const bool store = g_out != nullptr && h_out != nullptr;
     const bool vec = gp.objective != 7 &&
                      ((reinterpret_cast<uintptr_t>(preds) | reinterpret_cast<uintptr_t>(labels) |
@@ -1054,7 +1056,8 @@ hipError_t launch_grad_max(hipStream_t s, const GradParams &gp, const float *pre
                       : (store ? k_grad_max<false, true> : k_grad_max<false, false>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(GRAD_THREADS), 0, s, gp, preds, labels,
                        weights, rows, partial, g_out, h_out);
-    hipLaunchKernelGGL(k_grad_max_final, dim3(1), dim3(64), 0, s, partial, blocks, ctl);
+    if (!partials)
+        hipLaunchKernelGGL(k_grad_max_final, dim3(1), dim3(64), 0, s, partial, blocks, ctl);
     return hipGetLastError();
 }
 
@@ -2511,6 +2514,21 @@ __device__ void decide_node(const Shape &sh, const SplitParams &sp, const LevelA
                  node_g, node_h, bounds, monotone, out);
 }
 
+// Monotone bounds of a split's children from its node's (Shaders.swift:1424-1443).
+__device__ __forceinline__ void child_bounds(const SplitParams &sp, const SplitResult &r, int cst,
+                                             int64_t Gt, int64_t Ht, float g_inv, float h_inv,
+                                             float2 pb, float2 &lb, float2 &rb) {
+    lb = pb;
+    rb = pb;
+    if (cst == 0) return;
+    const float vl = -r.gl / (r.hl + sp.lambda);
+    const float gr = (float)(Gt - r.gl_int) * g_inv, hr = (float)(Ht - r.hl_int) * h_inv;
+    const float vr = -gr / (hr + sp.lambda);
+    const float mid = clampf(0.5f * (vl + vr), pb.x, pb.y);
+    if (cst > 0) { lb.y = fminf(lb.y, mid); rb.x = fmaxf(rb.x, mid); }
+    else { lb.x = fmaxf(lb.x, mid); rb.y = fminf(rb.y, mid); }
+}
+
 // decide_splits' outcome for node n (level-local `local`) once its best
 // feature bf (-1: none) and gain bg are known, by one lane: the node's split
 // or leaf, the children's sums and monotone bounds (Shaders.swift:1401-1451).
@@ -2532,17 +2550,8 @@ __device__ void decide_apply(const SplitParams &sp, int F, uint32_t n, uint32_t 
         const uint32_t lc = 2 * n + 1, rc = 2 * n + 2;
         node_g[lc] = r.gl_int; node_h[lc] = r.hl_int;
         node_g[rc] = Gt - r.gl_int; node_h[rc] = Ht - r.hl_int;
-        // monotone bounds (Shaders.swift:1424-1443)
-        float2 lb = pb, rb = pb;
-        const int cst = cat ? 0 : (int)monotone[bf];
-        if (cst != 0) {
-            const float vl = -r.gl / (r.hl + sp.lambda);
-            const float gr = (float)(Gt - r.gl_int) * g_inv, hr = (float)(Ht - r.hl_int) * h_inv;
-            const float vr = -gr / (hr + sp.lambda);
-            const float mid = clampf(0.5f * (vl + vr), pb.x, pb.y);
-            if (cst > 0) { lb.y = fminf(lb.y, mid); rb.x = fmaxf(rb.x, mid); }
-            else { lb.x = fmaxf(lb.x, mid); rb.y = fminf(rb.y, mid); }
-        }
+        float2 lb, rb;
+        child_bounds(sp, r, cat ? 0 : (int)monotone[bf], Gt, Ht, g_inv, h_inv, pb, lb, rb);
         bounds[lc] = lb;
         bounds[rc] = rb;
     } else {
@@ -4547,6 +4556,438 @@ hipError_t launch_lwb_select(hipStream_t s, const Shape &sh, const SplitParams &
     else if (words <= 4) MBK_LWB_SELECT(4);
     else MBK_LWB_SELECT(lwb_mask_words(LWB_MAX_DEPTH));
 #undef MBK_LWB_SELECT
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Level-wise trees of few rows.  The passes above are shaped for millions of
+// rows: at 20k rows each of their six launches per level is a latency chain of its
+// own (partition 12.6 us, histograms 9.2, reduction 4.1, split search 8.2), most of
+// it planning, segments and partials.  Here a row keeps its node's number instead
+// of being moved, and a level is two launches:
+//   k_small_level  one workgroup per feature: every row streamed (coalesced), the
+//                  built children's histograms of that feature in LDS, siblings by
+//                  subtraction, the split search of every node of the level
+//   k_small_route  decisions from the split keys, every row's node number moved
+//                  to the child; after the deepest split level also the leaf
+//                  values, predictions, the next tree's gradient maxima and the
+//                  rows per node
+// with k_small_start (maxima, quantisation, the finished tree's covers) before them.
+// Sums are exact integers and the search is node_split, so trees are the same.
+// 20k x 100, 100 trees of depth 6: 22.8 -> 12.3 ms of kernels (k_small_level 13.1 us,
+// k_small_route 4.2, k_small_start 7.0, the last route 6.4); 1,000 x 10, 20 trees of
+// depth 4: 2.52 -> 1.32 ms.  A workgroup streams some 6.5 rows per ns, so the form
+// pays up to 100k to 250k rows (small_trees in trainer.cpp).
+// Histograms are packed words (HIST_QH_BITS: rows below 2^20), [feature][node][bin],
+// which one workgroup writes and reads again at the next level.
+// ---------------------------------------------------------------------------
+
+constexpr int SMALL_THREADS = 1024;
+constexpr int SMALL_WAVES = SMALL_THREADS / 64;
+constexpr int SMALL_ROUTE_THREADS = 256;
+constexpr int SMALL_QUADS = 4;                         // row quads in flight per thread
+
+__device__ __forceinline__ uint32_t load_u8x4(const uint8_t *p) {   // any alignment
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+
+// copies: counters per histogram cell (by lane, so that lanes of one bin do not
+// serialise), at least 2: after the sums, copy 0 holds the built node's word and
+// copy 1 the derived one's.
+__global__ __launch_bounds__(SMALL_THREADS) void k_small_level(SmallArgs a, SplitParams sp,
+                                                               int32_t level, int32_t copies) {
+    extern __shared__ uint64_t small_lds[];
+    const int f = blockIdx.x, tid = threadIdx.x, lane = lane_id();
+    const bool allowed = a.feat_mask[f] != 0;
+    if (!allowed && f != 0) return;                    // feature 0 also leaves the node sums
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = a.num_bins;
+    const uint32_t num_level = 1u << level, level_start = num_level - 1u;
+    const uint32_t pairs = level == 0 ? 1u : num_level >> 1;
+    const uint32_t cells = pairs * (uint32_t)nb;
+    CatScratch *cs_all = reinterpret_cast<CatScratch *>(small_lds + (size_t)cells * copies);
+    // parents that split (bit p) and, of those, the ones whose right child is built
+    uint64_t split = 1, right = 0;
+    if (level > 0) {
+        const uint32_t side = (uint32_t)lane < pairs ? a.side[lane] : 2u;
+        right = __ballot(side == 1u);
+        split = __ballot(side < 2u);
+    }
+    for (uint32_t k = tid; k < cells * (uint32_t)copies; k += SMALL_THREADS) small_lds[k] = 0;
+    __syncthreads();
+    const uint8_t *bins = a.bins_fm + (size_t)f * (size_t)a.rows;
+    // A row's cell is (its pair, its bin): slot holds the pair of a row in a built
+    // child, 0xFF otherwise.  Four quads per thread in flight (two: +3% at 131k rows;
+    // loading the next four during the adds: nothing).
+    uint64_t *mine = small_lds + (lane & (copies - 1));
+    const uint32_t pair_cells = (uint32_t)(nb * copies);
+    auto add = [&](uint32_t p, uint32_t bin, uint32_t ghq) {
+        if (p == 0xFFu) return;
+        static_assert(HIST_QH_BITS == 27, "qg << 27 by halves");
+        const uint32_t lo = ((ghq << 11) & 0xF8000000u) | (ghq & 0xFFFFu);
+        const uint32_t hi = (uint32_t)((int32_t)ghq >> 21);
+        atomicAdd(reinterpret_cast<unsigned long long *>(
+                      &mine[__umul24(p, pair_cells) + bin * (uint32_t)copies]),
+                  (unsigned long long)lo | ((unsigned long long)hi << 32));
+    };
+    const uint32_t quads = a.rows >> 2;
+    for (uint32_t q0 = tid; q0 < quads; q0 += SMALL_QUADS * SMALL_THREADS) {
+        uint32_t sl[SMALL_QUADS], bn[SMALL_QUADS];
+        uint4 g[SMALL_QUADS];
+#pragma unroll
+        for (int u = 0; u < SMALL_QUADS; ++u) {
+            const uint32_t q = q0 + u * SMALL_THREADS;
+            sl[u] = 0xFFFFFFFFu;
+            if (q < quads) {
+                sl[u] = level == 0 ? 0u : reinterpret_cast<const uint32_t *>(a.slot)[q];
+                bn[u] = load_u8x4(bins + 4 * (size_t)q);
+                g[u] = reinterpret_cast<const uint4 *>(a.ghq)[q];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SMALL_QUADS; ++u) {
+            if (sl[u] == 0xFFFFFFFFu) continue;
+            add(sl[u] & 0xFFu, bn[u] & 0xFFu, g[u].x);
+            add((sl[u] >> 8) & 0xFFu, (bn[u] >> 8) & 0xFFu, g[u].y);
+            add((sl[u] >> 16) & 0xFFu, (bn[u] >> 16) & 0xFFu, g[u].z);
+            add(sl[u] >> 24, bn[u] >> 24, g[u].w);
+        }
+    }
+    const uint32_t tail = (quads << 2) + tid;
+    if (tail < a.rows) add(level == 0 ? 0u : a.slot[tail], bins[tail], a.ghq[tail]);
+    __syncthreads();
+    // copies summed; the sibling's words = the parent's - the built child's
+    const size_t fbase = (size_t)f * a.max_nodes * nb;
+    const uint64_t *prev = a.hist[(level & 1) ^ 1] + fbase;
+    uint64_t *cur = a.hist[level & 1] + fbase;
+    const bool keep = level + 1 < a.depth;             // a parent of the next level
+    for (uint32_t c = tid; c < cells; c += SMALL_THREADS) {
+        uint64_t sum = 0;
+        for (int k = 0; k < copies; ++k) sum += small_lds[(size_t)c * copies + k];
+        small_lds[(size_t)c * copies] = sum;
+        if (level == 0) {
+            if (keep) cur[c] = sum;
+            continue;
+        }
+        const uint32_t p = c / (uint32_t)nb, bin = c - p * nb;
+        if (!((split >> p) & 1u)) continue;
+        const uint64_t other = prev[c] - sum;          // prev is [parent][bin] too
+        small_lds[(size_t)c * copies + 1] = other;
+        if (keep) {
+            const uint32_t bl = 2 * p + (uint32_t)((right >> p) & 1u);
+            cur[bl * (uint32_t)nb + bin] = sum;
+            cur[(bl ^ 1u) * (uint32_t)nb + bin] = other;
+        }
+    }
+    __syncthreads();
+    const float g_inv = f32_from_bits(a.ctl->max_gh[0]) / 32767.0f;
+    const float h_inv = f32_from_bits(a.ctl->max_gh[1]) / 127.0f;
+    const bool cat = a.is_cat[f] != 0;
+    const int cst = cat ? 0 : (int)a.monotone[f];
+    constexpr uint64_t HMASK = (1ull << HIST_QH_BITS) - 1;
+    uint64_t *keys = a.keys[level & 1];
+    for (uint32_t l = (uint32_t)w; l < num_level; l += SMALL_WAVES) {   // uniform per wavefront
+        const uint32_t p = l >> 1;
+        if (!((split >> p) & 1u)) continue;
+        const uint32_t derived = (uint32_t)((right >> p) & 1u) ^ (l & 1u);
+        const uint64_t *src = small_lds + (size_t)p * nb * copies + derived;
+        int64_t hg[4], hh[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int b = 4 * lane + j;
+            const uint64_t word = b < nb ? src[(size_t)b * copies] : 0;
+            hg[j] = (int64_t)word >> HIST_QH_BITS;
+            hh[j] = (int64_t)(word & HMASK);
+        }
+        const uint32_t n = level_start + l;
+        if (f == 0) {
+            const int64_t G = wave_sum(hg[0] + hg[1] + hg[2] + hg[3]);
+            const int64_t H = wave_sum(hh[0] + hh[1] + hh[2] + hh[3]);
+            if (lane == 0) { a.node_g[n] = G; a.node_h[n] = H; }
+        }
+        if (!allowed) continue;
+        const float gain = node_split(hg, hh, nb, cat, cst, g_inv, h_inv, sp, &cs_all[w],
+                                      a.results + (size_t)l * a.cols + f);
+        const uint64_t key = split_key(gain, f);
+        if (lane == 0 && key)
+            atomicMax(reinterpret_cast<unsigned long long *>(&keys[(size_t)l * KEY_STRIDE]),
+                      (unsigned long long)key);
+    }
+}
+
+// The covers of a finished tree (t.cover[n] = the rows of n's subtree, from the
+// rows per final node), and the counters zeroed again.
+__device__ void small_covers(uint32_t *count, float *cover, int32_t depth) {
+    __shared__ uint32_t c[256];
+    const uint32_t total = (2u << depth) - 1u;
+    for (uint32_t n = threadIdx.x; n < total; n += blockDim.x) c[n] = count[n];
+    __syncthreads();
+    for (uint32_t n = threadIdx.x; n < total; n += blockDim.x) {
+        uint32_t sum = 0;
+        for (uint32_t first = n, wd = 1; first < total; first = 2 * first + 1, wd *= 2)
+            for (uint32_t j = 0; j < wd; ++j) sum += c[first + j];
+        cover[n] = (float)sum;
+        count[n] = 0;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_small_covers(uint32_t *count, float *cover,
+                                                      int32_t depth) {
+    small_covers(count, cover, depth);
+}
+
+// The tree's start: every workgroup reduces the gradient maxima's partials and
+// quantises its rows; the first also hands over the control block, writes the
+// finished tree's covers (prev_cover, or NULL) and opens the root's key and bounds.
+__global__ __launch_bounds__(SMALL_ROUTE_THREADS) void k_small_start(
+    SmallArgs a, GradParams gp, const float *__restrict__ preds,
+    const float *__restrict__ labels, const float *__restrict__ weights,
+    const uint32_t *__restrict__ partial, int nparts, TreeCtl *ctl_out, float *prev_cover) {
+    __shared__ uint2 bc;
+    const uint32_t i = blockIdx.x * SMALL_ROUTE_THREADS + threadIdx.x;
+    float g = 0.0f, h = 0.0f;
+    if (i < a.rows) row_grad_at(gp, preds, labels, weights, i, g, h);
+    const uint2 m = reduce_partial_max(partial, nparts, &bc);
+    const float mg = f32_from_bits(m.x), mh = f32_from_bits(m.y);
+    if (i < a.rows) {
+        const float gscale = mg > 0.0f ? 32767.0f / mg : 0.0f;
+        const float hscale = mh > 0.0f ? 127.0f / mh : 0.0f;
+        const int qg = (int)rintf(g * gscale);
+        const uint32_t qh = (uint32_t)rintf(h * hscale);
+        a.ghq[i] = ((uint32_t)(qg & 0xFFFF) << 16) | (qh & 0x7Fu);
+    }
+    if (blockIdx.x != 0) return;
+    constexpr uint32_t CW = sizeof(TreeCtl) / 4;
+    if (threadIdx.x < CW) {
+        uint32_t *wd = reinterpret_cast<uint32_t *>(a.ctl);
+        const uint32_t v = wd[threadIdx.x];
+        if (ctl_out) reinterpret_cast<uint32_t *>(ctl_out)[threadIdx.x] = v;
+        wd[threadIdx.x] = threadIdx.x == 0 ? m.x : threadIdx.x == 1 ? m.y : 0u;
+    }
+    if (threadIdx.x == 0) {
+        a.keys[0][0] = 0;
+        a.bounds[0] = make_float2(-INFINITY, INFINITY);
+    }
+    if (prev_cover) small_covers(a.count, prev_cover, a.depth);
+}
+
+// Decisions of level `level` from its keys, and every row to its child.  Every
+// workgroup takes the level's splits into LDS; the first writes the model arrays,
+// the children's sums and bounds, which child is built (the smaller hessian: any
+// choice gives the same sums) and clears the next level's keys.  FINAL (the deepest
+// split level): leaf values, predictions (preds non-null) and with GRAD the next
+// tree's gradient maxima, and the rows per node in count.
+template <bool FINAL, bool GRAD>
+__global__ __launch_bounds__(SMALL_ROUTE_THREADS) void k_small_route(
+    SmallArgs a, SplitParams sp, int32_t level, TreeOut out, float *__restrict__ preds,
+    GradParams gp, const float *__restrict__ labels, const float *__restrict__ weights,
+    uint32_t *__restrict__ gpart) {
+    __shared__ int32_t s_feat[64];
+    __shared__ uint32_t s_bf[64], s_mask[64][8];   // bf: bin | flags << 8 | right built << 16
+    __shared__ float s_leaf[FINAL ? 256 : 1];
+    __shared__ uint32_t s_cnt[FINAL ? 256 : 1];
+    const uint32_t num_level = 1u << level, level_start = num_level - 1u;
+    const uint32_t total = 4u * num_level - 1u;        // FINAL: every node of the tree
+    const uint32_t tid = threadIdx.x;
+    const uint64_t *keys = a.keys[level & 1];
+    // this thread's four rows load while the splits do
+    const uint32_t i0 = (blockIdx.x * SMALL_ROUTE_THREADS + tid) * 4u;
+    uint32_t nd = 0;
+    if (level > 0 && i0 < a.rows) {                    // node is padded to whole quads
+        nd = reinterpret_cast<const uint32_t *>(a.node)[i0 >> 2];
+    }
+    if (FINAL)
+        for (uint32_t n = tid; n < total; n += SMALL_ROUTE_THREADS) {
+            s_cnt[n] = 0;
+            if (n < level_start) s_leaf[n] = out.leaf[n];
+        }
+    if (tid < num_level) {
+        const uint32_t n = level_start + tid;
+        const uint64_t key = keys[(size_t)tid * KEY_STRIDE];
+        const bool split = key_splits(key, 1u, sp.min_split_gain);
+        const int bf = split ? key_feature(key) : -1;
+        s_feat[tid] = bf;
+        SplitResult r = {};
+        if (split) {
+            r = a.results[(size_t)tid * a.cols + bf];
+            // the child of the smaller hessian is built
+            const uint32_t right = 2 * r.hl_int <= a.node_h[n] ? 0u : 1u;
+            s_bf[tid] = (r.bin & 0xFFu) | ((r.flags & 0xFFu) << 8) | (right << 16);
+            for (int k = 0; k < 8; ++k) s_mask[tid][k] = r.mask[k];
+            if (!FINAL && blockIdx.x == 0) a.side[tid] = (uint8_t)right;
+        } else if (!FINAL && blockIdx.x == 0) {
+            a.side[tid] = 2;
+        }
+        if (FINAL || blockIdx.x == 0) {
+            const int64_t Gt = a.node_g[n], Ht = a.node_h[n];
+            const float2 pb = a.bounds[n];
+            const uint32_t mgb = a.ctl->max_gh[0], mhb = a.ctl->max_gh[1];
+            const float g_inv = f32_from_bits(mgb) / 32767.0f, h_inv = f32_from_bits(mhb) / 127.0f;
+            auto leaf_of = [&](int64_t g, int64_t h, float2 bb) {
+                const float G = (float)g * g_inv, H = (float)h * h_inv;
+                return sp.learning_rate * clampf(-G / (H + sp.lambda), bb.x, bb.y);
+            };
+            if (FINAL) {
+                float2 lb, rb;
+                float left = 0.0f, right = 0.0f;
+                if (split) {
+                    const bool cat = (r.flags & FLAG_CATEGORICAL) != 0;
+                    child_bounds(sp, r, cat ? 0 : (int)a.monotone[bf], Gt, Ht, g_inv, h_inv, pb, lb,
+                                 rb);
+                    left = leaf_of(r.gl_int, r.hl_int, lb);
+                    right = leaf_of(Gt - r.gl_int, Ht - r.hl_int, rb);
+                }
+                s_leaf[n] = split ? 0.0f : leaf_of(Gt, Ht, pb);
+                s_leaf[2 * n + 1] = left;
+                s_leaf[2 * n + 2] = right;
+                if (blockIdx.x == 0) {
+                    for (uint32_t c = 2 * n + 1; c <= 2 * n + 2; ++c) {
+                        out.split[c] = NodeSplit{-1, 0, 0};
+                        out.gain[c] = 0.0f;
+                        out.leaf[c] = c == 2 * n + 1 ? left : right;
+                    }
+                }
+            }
+            if (blockIdx.x == 0) {
+                const float bg = key ? key_float((uint32_t)(key >> 32)) : -INFINITY;
+                decide_apply(sp, a.cols, n, tid, bf, bg, a.results, Gt, Ht, pb, mgb, mhb, a.node_g,
+                             a.node_h, a.bounds, a.monotone, out);
+            }
+        }
+    }
+    if (!FINAL && blockIdx.x == 0)
+        for (uint32_t l = tid; l < 2 * num_level; l += SMALL_ROUTE_THREADS)
+            a.keys[(level & 1) ^ 1][(size_t)l * KEY_STRIDE] = 0;
+    __syncthreads();
+    uint32_t n[4], bin[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        n[k] = (nd >> (8 * k)) & 0xFFu;
+        const uint32_t l = n[k] - level_start;
+        const int32_t f = i0 + k < a.rows && l < num_level ? s_feat[l] : -1;
+        bin[k] = f >= 0 ? a.bins_fm[(size_t)f * a.rows + i0 + k] : 0xFFFFFFFFu;
+    }
+    float p[4] = {}, y[4] = {};
+    if (FINAL && preds) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i0 + k < a.rows) {
+                p[k] = preds[i0 + k];
+                if (GRAD) y[k] = labels[i0 + k];
+            }
+    }
+    uint32_t slot = 0xFFFFFFFFu;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (bin[k] == 0xFFFFFFFFu) continue;
+        const uint32_t l = n[k] - level_start, bf = s_bf[l];
+        const NodeSplit ns{s_feat[l], bf & 0xFFu, (bf >> 8) & 0xFFu};
+        const bool left = bin_goes_left(bin[k], ns, a.num_bins, s_mask[l]);
+        n[k] = 2 * n[k] + (left ? 1u : 2u);
+        if (left != ((bf >> 16) != 0)) slot ^= (l ^ 0xFFu) << (8 * k);   // in the built child
+    }
+    if (!FINAL) {
+        if (i0 < a.rows) {
+            reinterpret_cast<uint32_t *>(a.node)[i0 >> 2] =
+                n[0] | (n[1] << 8) | (n[2] << 16) | (n[3] << 24);
+            reinterpret_cast<uint32_t *>(a.slot)[i0 >> 2] = slot;
+        }
+        return;
+    }
+    uint32_t mg = 0, mh = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (i0 + k >= a.rows) continue;
+        atomicAdd(&s_cnt[n[k]], 1u);
+        if (!preds) continue;
+        const float np = p[k] + s_leaf[n[k]];
+        preds[i0 + k] = np;
+        if (GRAD) {
+            float g, h;
+            row_grad(gp, np, y[k], gp.has_weights ? weights[i0 + k] : 1.0f, g, h);
+            mg = max(mg, __float_as_uint(fabsf(g)));
+            mh = max(mh, __float_as_uint(h));
+        }
+    }
+    if (GRAD) {
+        __shared__ uint32_t red[2][SMALL_ROUTE_THREADS / 64];
+        mg = wave_max_u32(mg);
+        mh = wave_max_u32(mh);
+        if (lane_id() == 0) { red[0][tid >> 6] = mg; red[1][tid >> 6] = mh; }
+        __syncthreads();
+        if (tid == 0) {
+            for (int k = 1; k < SMALL_ROUTE_THREADS / 64; ++k) {
+                mg = max(mg, red[0][k]);
+                mh = max(mh, red[1][k]);
+            }
+            gpart[2 * blockIdx.x] = mg;
+            gpart[2 * blockIdx.x + 1] = mh;
+        }
+    }
+    __syncthreads();
+    for (uint32_t c = tid; c < total; c += SMALL_ROUTE_THREADS)
+        if (s_cnt[c]) atomicAdd(&a.count[c], s_cnt[c]);
+}
+
+static unsigned small_blocks(uint32_t rows) {
+    return (rows + 4 * SMALL_ROUTE_THREADS - 1) / (4 * SMALL_ROUTE_THREADS);
+}
+
+hipError_t launch_small_start(hipStream_t s, const SmallArgs &a, const GradParams &gp,
+                              const float *preds, const float *labels, const float *weights,
+                              const uint32_t *partial, int nparts, TreeCtl *ctl_out,
+                              float *prev_cover) {
+    hipLaunchKernelGGL(k_small_start, dim3((a.rows + SMALL_ROUTE_THREADS - 1) / SMALL_ROUTE_THREADS),
+                       dim3(SMALL_ROUTE_THREADS), 0, s, a, gp, preds, labels, weights, partial,
+                       nparts, ctl_out, prev_cover);
+    return hipGetLastError();
+}
+
+hipError_t launch_small_level(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                              int32_t level, bool has_cats) {
+    const size_t cells = ((size_t)1 << std::max(0, level - 1)) * (size_t)a.num_bins;
+    // four counters per cell at most (2, 4, 8 and 16 measured alike but for
+    // clearing and summing them: 16 costs 0.5 ms per 40 trees)
+    int32_t copies = 4;
+    while (copies > 2 && cells * (size_t)copies * 8 > (size_t)65536) copies /= 2;
+    const size_t lds = cells * (size_t)copies * 8 + (has_cats ? SMALL_WAVES * sizeof(CatScratch) : 0);
+    if (lds > (size_t)160 << 10) return hipErrorInvalidValue;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_level),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_small_level, dim3((unsigned)a.cols), dim3(SMALL_THREADS), lds, s, a, sp,
+                       level, copies);
+    return hipGetLastError();
+}
+
+hipError_t launch_small_route(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                              int32_t level, const TreeOut &out) {
+    hipLaunchKernelGGL((k_small_route<false, false>), dim3(small_blocks(a.rows)),
+                       dim3(SMALL_ROUTE_THREADS), 0, s, a, sp, level, out, nullptr, GradParams{},
+                       nullptr, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_small_finish(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                               const TreeOut &out, float *preds, const GradParams &gp,
+                               const float *labels, const float *weights, uint32_t *gpart,
+                               int *partials) {
+    const unsigned blocks = small_blocks(a.rows);
+    if (partials) {
+        hipLaunchKernelGGL((k_small_route<true, true>), dim3(blocks), dim3(SMALL_ROUTE_THREADS), 0, s,
+                           a, sp, a.depth - 1, out, preds, gp, labels, weights, gpart);
+        *partials = (int)blocks;
+    } else {
+        hipLaunchKernelGGL((k_small_route<true, false>), dim3(blocks), dim3(SMALL_ROUTE_THREADS), 0,
+                           s, a, sp, a.depth - 1, out, preds, gp, labels, weights, gpart);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_small_covers(hipStream_t s, uint32_t *count, float *cover, int32_t depth) {
+    hipLaunchKernelGGL(k_small_covers, dim3(1), dim3(256), 0, s, count, cover, depth);
     return hipGetLastError();
 }
 

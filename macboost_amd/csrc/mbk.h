@@ -256,11 +256,13 @@ struct GradParams {
 };
 // ctl->max_gh = (max |g|, max h); partial: grad_max_scratch_words() u32 of
 // device scratch.  With g_out and h_out (rows floats each, 16-B aligned)
-// every row's g and h are stored too.
+// every row's g and h are stored too.  With partials the maxima are left as that
+// many pairs in partial (ctl is not written).
 hipError_t launch_grad_max(hipStream_t s, const GradParams &gp, const float *preds,
                            const float *labels, const float *weights, int64_t rows,
                            TreeCtl *ctl, uint32_t *partial, float *g_out = nullptr,
-                           float *h_out = nullptr);
+                           float *h_out = nullptr,
+                           int *partials = nullptr);
 size_t grad_max_scratch_words();
 
 // Row sampling (GOSS / bagging) for one tree over the gradients g, h and
@@ -713,6 +715,46 @@ hipError_t launch_treeshap(hipStream_t s, const float *x, int64_t rows, int32_t 
                            const ShapUniq *uniq, float bias, float *out, double *phi_global);
 bool treeshap_needs_scratch(int cols);
 
+
+// ---- Level-wise trees of few rows (kernels_tree.hip): per tree
+// launch_small_start, then launch_small_level and launch_small_route for levels 0 ..
+// depth - 2, launch_small_level(depth - 1) and launch_small_finish.
+constexpr int SMALL_MAX_DEPTH = 7;    // node numbers fit a byte, a level's nodes a 64-bit mask
+struct SmallArgs {
+    uint32_t rows;                    // below 2^20
+    int32_t cols, num_bins, depth;
+    uint32_t max_nodes;               // 2^(depth - 1)
+    const uint8_t *bins_fm;           // [cols][rows]
+    uint8_t *node;                    // per row, padded to whole quads
+    uint8_t *slot;                    // likewise: the pair of a row in a built child, or 0xFF
+    uint32_t *ghq;                    // per row, 16-B aligned
+    uint64_t *hist[2];                // [cols][max_nodes][num_bins] packed words, by level parity
+    uint64_t *keys[2];                // [max_nodes] at SPLIT_KEY_STRIDE, by level parity
+    uint8_t *side;                    // [max_nodes] which child is built: 0 left, 1 right, 2 no split
+    SplitResult *results;             // [max_nodes][cols]
+    int64_t *node_g, *node_h;
+    float2 *bounds;
+    const uint8_t *is_cat, *feat_mask;
+    const int8_t *monotone;
+    TreeCtl *ctl;
+    uint32_t *count;                  // rows per final node, zero before a tree
+};
+// Quantises with the maxima of nparts pairs in partial; ctl_out receives the
+// previous tree's control block, prev_cover its covers from count (either NULL: not).
+hipError_t launch_small_start(hipStream_t s, const SmallArgs &a, const GradParams &gp,
+                              const float *preds, const float *labels, const float *weights,
+                              const uint32_t *partial, int nparts, TreeCtl *ctl_out,
+                              float *prev_cover);
+hipError_t launch_small_level(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                              int32_t level, bool has_cats);
+hipError_t launch_small_route(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                              int32_t level, const TreeOut &out);
+// preds NULL: rows per node only; partials NULL: no gradient maxima.
+hipError_t launch_small_finish(hipStream_t s, const SmallArgs &a, const SplitParams &sp,
+                               const TreeOut &out, float *preds, const GradParams &gp,
+                               const float *labels, const float *weights, uint32_t *gpart,
+                               int *partials);
+hipError_t launch_small_covers(hipStream_t s, uint32_t *count, float *cover, int32_t depth);
 
 // ---- TreeSHAP from contribution tables (kernels_infer.hip) ----
 constexpr int SHAP_MAX_COLS = 16;     // features of a group: 10 ancestors + 3 splits at depth 12

@@ -582,6 +582,12 @@ struct Trainer {
     DevBuf<mbk::NodeSplit> spec_split;
     DevBuf<float> spec_cover;
     DevBuf<uint32_t> spec_mask;
+    // level-wise trees of few rows (launch_small_*)
+    bool small = false;
+    DevBuf<uint8_t> small_node, small_slot, small_side;
+    DevBuf<uint64_t> small_hist[2], small_keys;
+    bool count_zero = false;        // t.count holds zeros (between small trees)
+    int small_cover_tree = -1;      // finished tree whose covers are still in t.count
     DevBuf<mbk::NodeSplit> m_split;
     DevBuf<float> m_leaf, m_gain, m_cover;
     DevBuf<uint32_t> m_mask;
@@ -638,6 +644,8 @@ struct Trainer {
         for (DevBuf<int64_t> *b : {&hist_a, &hist_b, &node_g, &node_h}) b->pooled = true;
         order_a.pooled = order_b.pooled = partials.pooled = items.pooled = true;
         mono.pooled = route_cursor.pooled = pairs.pooled = results.pooled = true;
+        small_node.pooled = small_slot.pooled = small_side.pooled = small_keys.pooled = true;
+        small_hist[0].pooled = small_hist[1].pooled = true;
         route_done.pooled = metric_part.pooled = true;
         bounds.pooled = ctl.pooled = true;
         lw_state.pooled = lw_open.pooled = lwb_state.pooled = lwb_cand.pooled = true;
@@ -1203,6 +1211,20 @@ static std::vector<float> base_scores_of(const Params &p, const float *y, const 
     return {base_score(p, y, w, rows)};
 }
 
+// Whether the fit's trees grow on the kernels for few rows.  One workgroup per
+// feature streams every row at every level there.  Every split child has to hold a
+// row, which min_child_hess > 0 guarantees (as for kept_walk).
+static bool small_trees(const Trainer &t) {
+    const Params &p = t.p;
+    if (t.leafwise || p.goss || p.subsample < 1.0f || !(p.min_child_hess > 0.0f)) return false;
+    if (t.D > mbk::SMALL_MAX_DEPTH || (t.D == mbk::SMALL_MAX_DEPTH && t.has_cats)) return false;
+    // Measured crossings with the partitioning path (40 trees of depth 6): 135k rows
+    // at 10 columns, 210k at 37, 240k at 100, 290k at 200, 120k at 300, where a
+    // second round of workgroups starts.
+    const int64_t rounds = (t.cols + t.dev->num_cus - 1) / t.dev->num_cus;
+    return t.rows <= (100000 + 1000 * (int64_t)std::min(t.cols, 150)) / rounds;
+}
+
 static void setup_buffers(Trainer &t, const float *y, const float *w, const float *yv,
                           const std::vector<float> *bases = nullptr) {
     const Params &p = t.p;
@@ -1388,6 +1410,15 @@ static void setup_buffers(Trainer &t, const float *y, const float *w, const floa
     t.seg_a.alloc((size_t)1 << t.D);
     t.seg_b.alloc((size_t)1 << t.D);
     t.ctl.alloc(1);
+    t.small = small_trees(t);
+    if (t.small) {
+        t.small_node.alloc(((size_t)rows + 3) / 4 * 4);
+        t.small_slot.alloc(((size_t)rows + 3) / 4 * 4);
+        t.small_side.alloc((size_t)t.max_level_nodes);
+        t.small_keys.alloc((size_t)t.max_level_nodes * mbk::SPLIT_KEY_STRIDE);
+        for (auto &h : t.small_hist)
+            h.alloc((size_t)cols * (size_t)t.max_level_nodes * (size_t)p.num_bins);
+    }
     t.ensure_capacity(std::max(1, p.num_trees));
     if (!t.has_root_copy) build_root_copy(t);   // (create_raw builds it after the binning)
     MB_HIP(hipStreamSynchronize(s));
@@ -1962,8 +1993,89 @@ static void training_walk(Trainer &t, int tree, const mbk::TreeOut &out, uint32_
     }
 }
 
+// The covers a small tree left in t.count, written now.
+static void flush_small_covers(Trainer &t) {
+    if (t.small_cover_tree < 0) return;
+    MB_HIP(mbk::launch_small_covers(t.dev->stream, t.count.ptr, t.tree_out(t.small_cover_tree).cover,
+                                    t.D));
+    t.small_cover_tree = -1;
+}
+
+// Level-wise growth of few rows: two launches per level (mbk.h, SmallArgs).
+static void grow_small(Trainer &t, int tree) {
+    hipStream_t s = t.dev->stream;
+    const mbk::TreeOut out = t.tree_out(tree);
+    if (const uint8_t *m = tree_feature_mask(t, tree))
+        MB_HIP(hipMemcpyAsync(t.feat_mask.ptr, m, (size_t)t.cols, hipMemcpyHostToDevice, s));
+    mbk::SmallArgs a{};
+    a.rows = (uint32_t)t.rows;
+    a.cols = t.cols;
+    a.num_bins = t.nb;
+    a.depth = t.D;
+    a.max_nodes = (uint32_t)t.max_level_nodes;
+    a.bins_fm = t.bins_fm.ptr;
+    a.node = t.small_node.ptr;
+    a.slot = t.small_slot.ptr;
+    a.ghq = reinterpret_cast<uint32_t *>(t.order_a.ptr);
+    a.hist[0] = t.small_hist[0].ptr;
+    a.hist[1] = t.small_hist[1].ptr;
+    a.keys[0] = t.split_keys.ptr;
+    a.keys[1] = t.small_keys.ptr;
+    a.side = t.small_side.ptr;
+    a.results = t.results.ptr;
+    a.node_g = t.node_g.ptr;
+    a.node_h = t.node_h.ptr;
+    a.bounds = t.bounds.ptr;
+    a.is_cat = t.is_cat.ptr;
+    a.feat_mask = t.feat_mask.ptr;
+    a.monotone = t.mono.ptr;
+    a.ctl = t.ctl.ptr;
+    a.count = t.count.ptr;
+    // what earlier trees left: fixups of the other path, control block, covers
+    if (t.fix_pending.active) {
+        const mbk::PendingFixup &f = t.fix_pending;
+        MB_HIP(mbk::launch_final_fixup(s, f.la, f.count, t.tree_out(t.fix_tree),
+                                       f.zero_empty != 0));
+        t.fix_pending.active = 0;
+    }
+    mbk::TreeCtl *prev = t.ctl_pending >= 0 ? t.ctl_hist.ptr + t.ctl_pending : nullptr;
+    t.ctl_pending = -1;
+    float *prev_cover = t.small_cover_tree >= 0 ? t.tree_out(t.small_cover_tree).cover : nullptr;
+    t.small_cover_tree = -1;
+    if (!t.count_zero) {
+        MB_HIP(hipMemsetAsync(t.count.ptr, 0, t.count.bytes(), s));
+        t.count_zero = true;
+    }
+    int parts = t.walk_gparts;
+    t.walk_gparts = 0;
+    if (parts == 0)
+        MB_HIP(mbk::launch_grad_max(s, t.gp, t.preds.ptr, t.labels.ptr, t.weights.ptr, t.rows,
+                                    t.ctl.ptr, t.gmax_part.ptr, nullptr, nullptr, &parts));
+    MB_HIP(mbk::launch_small_start(s, a, t.gp, t.preds.ptr, t.labels.ptr, t.weights.ptr,
+                                   t.gmax_part.ptr, parts, prev, prev_cover));
+    for (int d = 0; d < t.D; ++d) {
+        MB_HIP(mbk::launch_small_level(s, a, t.sp, d, t.has_cats));
+        if (d + 1 < t.D) MB_HIP(mbk::launch_small_route(s, a, t.sp, d, out));
+    }
+    const bool grads = t.K == 1 && !t.renewal;
+    MB_HIP(mbk::launch_small_finish(s, a, t.sp, out, t.renewal ? nullptr : t.preds_cur, t.gp,
+                                    t.labels.ptr, t.weights.ptr, t.gmax_part.ptr,
+                                    grads ? &t.walk_gparts : nullptr));
+    if (t.renewal) {
+        renew_tree(t, out, nullptr);
+        MB_HIP(mbk::launch_predict_binned(s, t.bins_fm.ptr, t.rows, t.nb, t.D, out, t.preds_cur));
+    }
+    if (t.has_valid)
+        MB_HIP(mbk::launch_predict_binned(s, t.vbins_fm.ptr, t.vrows, t.nb, t.D, out,
+                                          t.vpreds_cur));
+    t.small_cover_tree = tree;
+    t.ctl_pending = tree;                            // copied by the next tree's start
+}
+
 static void grow_levelwise(Trainer &t, int tree) {
     hipStream_t s = t.dev->stream;
+    flush_small_covers(t);
+    t.count_zero = false;
     const mbk::Shape &sh = t.sh;
     mbk::TreeOut out = t.tree_out(tree);
     if (const uint8_t *m = tree_feature_mask(t, tree))
@@ -2306,6 +2418,8 @@ void trainer_grow(Trainer *tp, int num_trees) {
         t.vpreds_cur = t.has_valid ? t.vpreds.ptr + (size_t)cls * (size_t)t.vrows : nullptr;
         if (t.lw_rounds) grow_leafwise_rounds(t, tree);
         else if (t.leafwise) grow_leafwise(t, tree);
+        // (timed trees keep the kernels that the timing is of)
+        else if (t.small && !t.prof_tree(tree)) grow_small(t, tree);
         else grow_levelwise(t, tree);
         t.grown += 1;
         // metrics once per round of K trees (Booster.swift:1650-1688)
@@ -2365,6 +2479,7 @@ void trainer_grow(Trainer *tp, int num_trees) {
         if (t.p.verbose && !line.empty()) std::printf("%s\n", line.c_str());
     }
     flush_metrics();
+    flush_small_covers(t);
     if (t.fix_pending.active) {                      // the last tree's deepest covers
         const mbk::PendingFixup &f = t.fix_pending;
         MB_HIP(mbk::launch_final_fixup(s, f.la, f.count, t.tree_out(t.fix_tree),

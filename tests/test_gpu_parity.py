@@ -1155,6 +1155,41 @@ def test_treeshap_wide_data_matches_oracle():
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("rows,cols,params", [
+    (1, 1, {"max_depth": 1}), (2, 3, {"max_depth": 2}), (5, 2, {"max_depth": 7}),
+    (1027, 5, {"max_depth": 7, "num_bins": 17}), (4096, 260, {"max_depth": 3}),
+    (30001, 4, {"max_depth": 6, "min_child_weight": 40.0}),
+    (109999, 10, {"max_depth": 4}), (110001, 10, {"max_depth": 4}),
+    (3001, 6, {"max_depth": 5, "feature_fraction": 0.4}),
+    (3002, 6, {"max_depth": 5, "objective": "quantile", "alpha": 0.3}),
+    (3003, 6, {"max_depth": 6, "monotone_constraints": [1, -1, 0, 1, 0, 0]})])
+def test_few_rows_identical(rows, cols, params):
+    # the two-launch levels of small fits: row remainders, one row, both sides of
+    # the row limit, more features than compute units, and the options that enter
+    # a level's decisions
+    rng = np.random.default_rng(rows)
+    x = rng.random((cols, rows), dtype=np.float32)
+    if rows > 100:
+        x[0, rng.random(rows) < 0.1] = np.nan
+        x[cols - 1] = rng.random(rows) < 0.02          # two values, one of them rare
+    y = (np.nan_to_num(x[0]) * 3 + x[cols - 1] + rng.standard_normal(rows)).astype(np.float32)
+    check_identical(x, y, {"num_trees": 3, **params})
+
+
+def test_few_rows_timed_trees_alternate():
+    # timed trees take the large-fit kernels: covers, control blocks and gradients
+    # pass between both paths within one fit
+    x, y = O.friedman(5000, 8, 3)
+    params = {"num_trees": 9, "max_depth": 5}
+    t = mb.Trainer(params, x, y, feature_major=True)
+    for n, on in ((2, False), (2, True), (3, False), (1, True), (1, False)):
+        t.profile(on)
+        t.grow(n)
+    a, b = model_io.saved_model(t.booster()), model_io.saved_model(
+        mb.train(params, x, y, feature_major=True))
+    assert a["trees"] == b["trees"]
+
+
 @pytest.mark.parametrize("rows,depth,objective", [
     (3, 2, "mae"), (8191, 1, "mae"), (8193, 1, "quantile"), (40000, 1, "mae"),
     (300001, 2, "quantile")])
