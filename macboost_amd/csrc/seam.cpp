@@ -220,6 +220,7 @@ int mbk_context_create(int32_t device, mbk_context **out, char **err) {
     return guarded(err, [&]() -> int {
         auto c = std::make_unique<mbk_context>();
         c->dev = std::make_unique<mb::Device>(device);
+        c->scratch.forest_features.pooled = c->scratch.nodes.pooled = true;
         c->scratch.forest_features.alloc(mbk::PRED_INFO_WORDS);
         c->scratch.nodes.alloc((size_t)1 << 18);
         *out = c.release();
