@@ -63,8 +63,10 @@ static int device_cus() {
 constexpr int PRED_THREADS = 1024;
 constexpr int PRED_WAVES = PRED_THREADS / 64;
 
+// Features of the nodes a row can reach: heap slots under a leaf may hold anything,
+// and the walk reads every listed feature's column.
 __global__ __launch_bounds__(1024) void k_forest_features(const int32_t *__restrict__ feature,
-                                                          int64_t nodes,
+                                                          int64_t nodes, uint32_t nodes_per_tree,
                                                           uint32_t *__restrict__ info) {
     __shared__ uint32_t used[PRED_MAP];
     __shared__ uint32_t tot[16];
@@ -74,8 +76,17 @@ __global__ __launch_bounds__(1024) void k_forest_features(const int32_t *__restr
     __syncthreads();
     for (int64_t k = threadIdx.x; k < nodes; k += 1024) {
         const int32_t f = feature[k];
+        if (f < 0) continue;
+        const uint32_t n = (uint32_t)(k % nodes_per_tree);
+        const int32_t *heap = feature + (k - n);
+        int32_t above = 0;                             // negative: a leaf on the way
+        for (uint32_t a = n; a > 0;) {
+            a = (a - 1) >> 1;
+            above |= heap[a];
+        }
+        if (above < 0) continue;
         if (f >= PRED_MAP) past = 1;
-        else if (f >= 0) used[f] = 1;
+        else used[f] = 1;
     }
     __syncthreads();
     uint32_t u[4], mine = 0;                           // features 4 t .. 4 t + 3
@@ -114,7 +125,8 @@ __device__ __forceinline__ PredNode pred_node(const ForestDev &f, int64_t g, boo
                                               const uint32_t *info) {
     const int32_t feat = f.feature[g];
     if (feat < 0) return PredNode{f.leaf[g], -1};
-    const int32_t slot = in_lds ? (int32_t)info[1 + PRED_SLOTS + feat] : feat;
+    // (a slot under a leaf may hold a feature past the map)
+    const int32_t slot = in_lds ? (int32_t)info[1 + PRED_SLOTS + min(feat, PRED_MAP - 1)] : feat;
     const int32_t flags = f.flags[g] & 3;
     // a categorical split without masks sends every row right
     if ((flags & FLAG_CATEGORICAL) && !f.mask) return PredNode{NAN, slot << 2};
@@ -132,7 +144,8 @@ __global__ __launch_bounds__(256) void k_forest_pack(ForestDev f, int64_t nodes,
 hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
                               uint32_t *info, PredNode *packed) {
     const int64_t nodes = (int64_t)f.num_trees * f.nodes_per_tree;
-    hipLaunchKernelGGL(k_forest_features, dim3(1), dim3(1024), 0, s, f.feature, nodes, info);
+    hipLaunchKernelGGL(k_forest_features, dim3(1), dim3(1024), 0, s, f.feature, nodes,
+                       (uint32_t)f.nodes_per_tree, info);
     if (packed && nodes > 0)
         hipLaunchKernelGGL(k_forest_pack, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, s, f,
                            nodes, info, std::min(max_slots, PRED_SLOTS), packed);

@@ -1297,6 +1297,36 @@ def test_predict_forest_edges(cols, trees, depth, leaves):
         assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
 
 
+@pytest.mark.parametrize("rows", [100, 4096, 5001])
+def test_predict_forest_slots_under_leaves(rows):
+    # no walk reaches a heap slot under a leaf, so it may name any feature:
+    # below and above the rows from which the used features are listed
+    x, y = O.friedman(6000, 6, 23)
+    h, obj = gpu_fit(x, y, {"num_trees": 20, "max_depth": 5, "min_child_weight": 300.0})
+    f = model_io.forest_from_json(obj)
+    xs = np.ascontiguousarray(x[:, :rows])
+    want = O.predict(f, obj["baseScore"], obj["numBins"], xs)
+    feature = f.feature.copy()
+    nodes, under = feature.shape[1], 0
+    for t in range(feature.shape[0]):
+        for n in range(1, nodes):
+            up, leaf_above = n, False
+            while up:
+                up = (up - 1) // 2
+                leaf_above = leaf_above or f.feature[t, up] < 0
+            if leaf_above:
+                feature[t, n] = (7, 5000, 1 << 28, -1)[(t + n) % 4]
+                under += 1
+    assert under > 50
+    ctx = mb.Context(0)
+    dev = [ctx.upload(a) for a in (feature, f.threshold, f.flags, f.leaf)]
+    out = ctx.alloc(rows * 4)
+    ctx.call("mbk_predict_forest", *dev, None, *feature.shape, ctx.upload(xs), rows,
+             obj["numBins"] - 1, obj["baseScore"], out)
+    ctx.sync()
+    assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
+
+
 @pytest.mark.parametrize("rows,cols,trees,depth", [
     (1, 8, 40, 6),            # one row: every share of the columns its own workgroup
     (2049, 9, 5, 1),          # one-split groups, a row past a row block
