@@ -496,7 +496,8 @@ __device__ __forceinline__ double metric_term(int metric, double p, double y, do
     }
     case METRIC_LOGLOSS: {
         const double q = 1 / (1 + exp(-p));
-        return -(y * log(fmax(q, 1e-12)) + (1 - y) * log(fmax(1 - q, 1e-12)));
+        const double a = q < 1e-12 ? 1e-12 : q, b = 1 - q < 1e-12 ? 1e-12 : 1 - q;   // NaN stays
+        return -(y * log(a) + (1 - y) * log(b));
     }
     case METRIC_POISSON: {
         const double mu = exp(p);

@@ -1250,6 +1250,16 @@ def test_validation_metric_on_device(objective, vrows):
     assert np.isclose(hist[-1], want, rtol=3e-7, atol=0)
 
 
+def test_validation_metric_keeps_nan():
+    # predictions that overflow to inf - inf: the metric is NaN, as a sum on the host is
+    x = np.ones((1, 500), np.float32)
+    y = (np.arange(500) % 5 < 3).astype(np.float32)
+    h = mb.train({"num_trees": 4, "max_depth": 1, "objective": "binary", "learning_rate": 3e38},
+                 x, y, eval_set=(x.T, y), feature_major=True)
+    assert np.isnan(mb.predict(h, x, feature_major=True)).any()
+    assert np.isnan(mb.eval_history(h)[-1])
+
+
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
 def test_categorical_rank_sizes(card):
     # the split search ranks a node's categories 64 at a time, four keys a read:
