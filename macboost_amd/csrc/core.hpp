@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <set>
 #include <stdexcept>
 #include <string>
@@ -263,6 +264,7 @@ struct Booster {
     std::unique_ptr<Device> dev;
     ForestCache forest;
     std::vector<ShapPlan> shap_plans;    // per class, made by its first predict_contrib
+    std::mutex made_mu;                  // guards forest and shap_plans
 
     Booster() = default;
     Booster(const Booster &) = delete;

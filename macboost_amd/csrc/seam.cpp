@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "../../include/macboost.h"
@@ -66,6 +67,7 @@ struct Scratch {
     // mbk_predict_forest, allocated with the context (its calls allocate nothing)
     DevBuf<uint32_t> forest_features;
     DevBuf<mbk::PredNode> nodes;
+    std::mutex nodes_mu;             // listing, packing and walk queued together
 };
 
 }  // namespace
@@ -523,7 +525,8 @@ int mbk_predict_forest(mbk_context *ctx, const int32_t *feature, const float *th
         // from some thousand rows on; 160 features in LDS leave room for two
         // workgroups per CU
         hipStream_t s = ctx->dev->stream;
-        const Scratch &sc = ctx->scratch;
+        Scratch &sc = ctx->scratch;
+        std::lock_guard<std::mutex> lock(sc.nodes_mu);
         const bool prepared = rows >= 4096;
         const bool pack = prepared && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
         if (prepared)

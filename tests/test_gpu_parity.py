@@ -5,6 +5,7 @@ model are compared bit for bit; TreeSHAP within 1e-5 relative (+1e-6 abs)
 of the oracle's double-precision recursive TreeSHAP.
 """
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -1258,6 +1259,18 @@ def test_validation_metric_keeps_nan():
                  x, y, eval_set=(x.T, y), feature_major=True)
     assert np.isnan(mb.predict(h, x, feature_major=True)).any()
     assert np.isnan(mb.eval_history(h)[-1])
+
+
+def test_contributions_from_several_threads():
+    # calls on one model, each with its own number of rows
+    x, y = O.friedman(20000, 10, 77)
+    h, _ = gpu_fit(x, y, {"num_trees": 30, "max_depth": 6})
+    parts = [np.ascontiguousarray(x[:, :n]) for n in (300, 2500, 9000, 20000)]
+    want = [mb.predict_contrib(h, p, feature_major=True) for p in parts]
+    with ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(lambda p: mb.predict_contrib(h, p, feature_major=True), parts * 3))
+    for k, g in enumerate(got):
+        assert np.array_equal(g, want[k % 4])
 
 
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
