@@ -2120,41 +2120,55 @@ struct CatScratch {
     uint32_t mask[8];
 };
 
+// One lane's float in every lane.
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+    return f32_from_bits((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+
+// The lowest lane with the largest gain, -1 if none is above -inf (no lane may
+// hold NaN).
+__device__ __forceinline__ int wave_best_lane(float gain) {
+    const uint32_t key = gain_key(gain), top = wave_max_u32(key);
+    if (top == gain_key(-INFINITY)) return -1;
+    return __ffsll((unsigned long long)__ballot(key == top)) - 1;
+}
+
 // Best split of one node's feature histogram held as 4 consecutive bins per
 // lane (bins 4*lane .. 4*lane+3).  Mirrors find_splits (Shaders.swift:396-463)
-// with exact integer prefix sums.  Writes the result through dst (one lane)
+// with exact integer prefix sums in T.  Writes the result through dst (one lane)
 // and returns its gain in every lane (-inf: no valid split).
-__device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int32_t nb,
-                           bool is_cat, int cst, float g_inv, float h_inv, const SplitParams &sp,
-                           CatScratch *cs, SplitResult *dst) {
+template <typename T>
+__device__ __forceinline__ float node_split_sums(const T (&hg)[4], const T (&hh)[4], int32_t nb,
+                                                 bool is_cat, int cst, float g_inv, float h_inv,
+                                                 const SplitParams &sp, CatScratch *cs,
+                                                 SplitResult *dst) {
     const int lane = lane_id();
     const int b0 = 4 * lane;
     const int data_bins = nb - 1;
-    int64_t lg = 0, lh = 0;
+    T lg = 0, lh = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) { lg += hg[j]; lh += hh[j]; }
-    const int64_t G_tot = wave_sum(lg), H_tot = wave_sum(lh);
+    const T G_tot = wave_sum(lg), H_tot = wave_sum(lh);
     const float G = (float)G_tot * g_inv, H = (float)H_tot * h_inv;
     const float parent = (G * G) / (H + sp.lambda);
 
     float best_gain = -INFINITY;
-    int best_seq = 0x7FFFFFFF;
     uint32_t best_bin = 0, best_flags = 0;
     float best_gl = 0.0f, best_hl = 0.0f;
-    int64_t best_gli = 0, best_hli = 0;
+    T best_gli = 0, best_hli = 0;
 
     if (!is_cat) {
         // missing-bin totals live in the lane holding bin nb-1
         const int ml = data_bins >> 2, mj = data_bins & 3;
-        int64_t mg = 0, mh = 0;
+        T mg = 0, mh = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (j == mj) { mg = hg[j]; mh = hh[j]; }
-        const int64_t GM = __shfl(mg, ml, 64), HM = __shfl(mh, ml, 64);
+        const T GM = __shfl(mg, ml, 64), HM = __shfl(mh, ml, 64);
         const float Hm = (float)HM * h_inv;
-        const int64_t ex_g = wave_inclusive_scan(lg) - lg;
-        const int64_t ex_h = wave_inclusive_scan(lh) - lh;
-        int64_t GL = ex_g, HL = ex_h;
+        const T ex_g = wave_inclusive_scan(lg) - lg;
+        const T ex_h = wave_inclusive_scan(lh) - lh;
+        T GL = ex_g, HL = ex_h;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int b = b0 + j;
@@ -2172,13 +2186,13 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
                         }
                         const float gain = split_gain(gl, hl, gr, hr, sp.lambda, parent);
                         if (ok && gain > best_gain) {
-                            best_gain = gain; best_seq = 2 * b; best_bin = (uint32_t)b;
+                            best_gain = gain; best_bin = (uint32_t)b;
                             best_flags = 0; best_gl = gl; best_hl = hl; best_gli = GL; best_hli = HL;
                         }
                     }
                 }
                 if (Hm > 0.0f) {   // missing goes left
-                    const int64_t LG = GL + GM, LH = HL + HM;
+                    const T LG = GL + GM, LH = HL + HM;
                     const float lgf = (float)LG * g_inv, lhf = (float)LH * h_inv;
                     const float rg = (float)(G_tot - LG) * g_inv, rh = (float)(H_tot - LH) * h_inv;
                     if (lhf >= sp.min_child_hess && rh >= sp.min_child_hess) {
@@ -2189,7 +2203,7 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
                         }
                         const float gain = split_gain(lgf, lhf, rg, rh, sp.lambda, parent);
                         if (ok && gain > best_gain) {
-                            best_gain = gain; best_seq = 2 * b + 1; best_bin = (uint32_t)b;
+                            best_gain = gain; best_bin = (uint32_t)b;
                             best_flags = FLAG_DEFAULT_LEFT; best_gl = lgf; best_hl = lhf;
                             best_gli = LG; best_hli = LH;
                         }
@@ -2197,23 +2211,21 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
                 }
             }
         }
-        float wg = best_gain;
-        int ws = best_seq;
-        wave_argmax(wg, ws);
-        if (ws == 0x7FFFFFFF) {
+        const int winner = wave_best_lane(best_gain);  // the lowest bin of equal gains
+        if (winner < 0) {
             if (lane == 0) {
                 SplitResult r = {};
                 r.gain = -INFINITY;
                 *dst = r;
             }
             return -INFINITY;
-        } else if (ws == best_seq && best_gain == wg) {
+        } else if (lane == winner) {
             SplitResult r = {};
             r.gain = best_gain; r.bin = best_bin; r.gl = best_gl; r.hl = best_hl;
             r.flags = best_flags; r.gl_int = best_gli; r.hl_int = best_hli;
             *dst = r;
         }
-        return wg;
+        return lane_f32(best_gain, winner);
     }
 
     // Categorical: non-empty bins (missing included) stably sorted by
@@ -2272,11 +2284,11 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
     for (int j = 0; j < 4; ++j)
         if (ne[j]) { cs->sg[rank[j]] = hg[j]; cs->sh[rank[j]] = hh[j]; }
     wave_lds_sync();
-    int64_t pg[4], ph[4];
-    int64_t tg = 0, th = 0;
+    T pg[4], ph[4];
+    T tg = 0, th = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { pg[j] = cs->sg[b0 + j]; ph[j] = cs->sh[b0 + j]; tg += pg[j]; th += ph[j]; }
-    int64_t GL = wave_inclusive_scan(tg) - tg, HL = wave_inclusive_scan(th) - th;
+    for (int j = 0; j < 4; ++j) { pg[j] = (T)cs->sg[b0 + j]; ph[j] = (T)cs->sh[b0 + j]; tg += pg[j]; th += ph[j]; }
+    T GL = wave_inclusive_scan(tg) - tg, HL = wave_inclusive_scan(th) - th;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int i = b0 + j;                         // sorted position
@@ -2288,17 +2300,15 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
             if (!(hl < sp.min_child_hess || hr < sp.min_child_hess)) {
                 const float gain = split_gain(gl, hl, gr, hr, sp.lambda, parent);
                 if (gain > best_gain) {
-                    best_gain = gain; best_seq = i; best_bin = (uint32_t)(i + 1);
+                    best_gain = gain; best_bin = (uint32_t)(i + 1);
                     best_flags = FLAG_CATEGORICAL; best_gl = gl; best_hl = hl;
                     best_gli = GL; best_hli = HL;
                 }
             }
         }
     }
-    float wg = best_gain;
-    int ws = best_seq;
-    wave_argmax(wg, ws);
-    if (ws == 0x7FFFFFFF) {
+    const int winner = wave_best_lane(best_gain);
+    if (winner < 0) {
         if (lane == 0) {
             SplitResult r = {};
             r.gain = -INFINITY;
@@ -2306,12 +2316,12 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
         }
         return -INFINITY;
     }
-    const int k = ws + 1;                            // left subset size
+    const int k = __builtin_amdgcn_readlane((int)best_bin, winner);   // left subset size
 #pragma unroll
     for (int j = 0; j < 4; ++j)
         if (ne[j] && rank[j] < k) atomicOr(&cs->mask[(b0 + j) >> 5], 1u << ((b0 + j) & 31));
     wave_lds_sync();
-    if (ws == best_seq && best_gain == wg) {
+    if (lane == winner) {
         SplitResult r = {};
         r.gain = best_gain; r.bin = best_bin; r.gl = best_gl; r.hl = best_hl;
         r.flags = best_flags; r.gl_int = best_gli; r.hl_int = best_hli;
@@ -2319,24 +2329,58 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
         for (int w = 0; w < 8; ++w) r.mask[w] = cs->mask[w];
         *dst = r;
     }
-    return wg;
+    return lane_f32(best_gain, winner);
+}
+
+// A wavefront's 32-bit sums where every bin's are below 2^23 (256 of them stay
+// below 2^31), 64-bit sums otherwise: the same whole numbers and the same floats.
+// The search is bound by its instructions (two scans, and a conversion to float for
+// each of eight sums per bin: one instruction from 32 bits, a dozen from 64).  With
+// k_split's 16-byte cells at a padded LDS pitch and the winner by one DPP maximum:
+// k_split of 256 nodes x 53 features 38.2 -> 29.9 us, 32 x 100 15.6 -> 12.5 us, 2 x 53
+// 8.8 -> 7.7 us; a whole 20k x 100 fit 12.9 -> 11.7 ms.
+__device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int32_t nb,
+                            bool is_cat, int cst, float g_inv, float h_inv, const SplitParams &sp,
+                            CatScratch *cs, SplitResult *dst) {
+    bool small = true;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        small = small && (uint64_t)(hg[j] + (1 << 23) - 1) < (uint64_t)((1 << 24) - 1) &&
+                (uint64_t)hh[j] < (uint64_t)(1 << 23);
+    if (!__all(small))
+        return node_split_sums<int64_t>(hg, hh, nb, is_cat, cst, g_inv, h_inv, sp, cs, dst);
+    int32_t g[4], h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { g[j] = (int32_t)hg[j]; h[j] = (int32_t)hh[j]; }
+    return node_split_sums<int32_t>(g, h, nb, is_cat, cst, g_inv, h_inv, sp, cs, dst);
 }
 
 // One workgroup per (sibling pair, 4 features), one wavefront per (side,
 // feature): both sides' histogram rows [bin][f0 .. f0+3] (64 contiguous bytes
-// per bin) are staged through LDS together, eight independent loads per
+// per bin) are staged through LDS together, four independent loads per
 // thread, then wavefront (side, w) searches feature f0 + w of that side's node
 // (its 256 bins, 4 per lane).  The two sides' searches run at once.
 constexpr int SPLIT_FEATS = 4;
 constexpr int SPLIT_WAVES = 2 * SPLIT_FEATS;
 constexpr int SPLIT_THREADS = SPLIT_WAVES * 64;
-constexpr int SPLIT_ROW = 2 * SPLIT_FEATS;           // words per bin and side
-constexpr int SPLIT_STAGE_PER_THREAD = 2 * 256 * SPLIT_ROW / SPLIT_THREADS;
-constexpr size_t SPLIT_STAGE_BYTES = (size_t)2 * 256 * SPLIT_ROW * sizeof(int64_t);
+constexpr int SPLIT_CELLS_PER_THREAD = 2 * 256 * SPLIT_FEATS / SPLIT_THREADS;
+constexpr int SPLIT_SIDE_CELLS = 64 * (4 * SPLIT_FEATS + 1);
+constexpr size_t SPLIT_STAGE_BYTES = (size_t)2 * SPLIT_SIDE_CELLS * 16;
 constexpr size_t SPLIT_LDS_BYTES = SPLIT_STAGE_BYTES > SPLIT_WAVES * sizeof(CatScratch)
                                        ? SPLIT_STAGE_BYTES
                                        : SPLIT_WAVES * sizeof(CatScratch);
-static_assert(2 * 256 * SPLIT_ROW % SPLIT_THREADS == 0, "whole stage words per thread");
+static_assert(2 * 256 * SPLIT_FEATS % SPLIT_THREADS == 0, "whole cells per thread");
+
+// (g, h) of a histogram cell: one load from a caller's 8-byte aligned buffer, one
+// 16-byte LDS access.
+typedef int64_t StagedCell __attribute__((ext_vector_type(2)));
+typedef int64_t HistCell __attribute__((ext_vector_type(2), aligned(8)));
+
+// LDS cell of (side, bin, feature of the group): a pad every four bins, so that the
+// lanes of a search, four bins apart, read different banks.
+__device__ __forceinline__ int split_cell(int side, int bin, int q) {
+    return side * SPLIT_SIDE_CELLS + bin * SPLIT_FEATS + q + (bin >> 2);
+}
 
 __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams sp,
                                                          const Pair *__restrict__ pairs,
@@ -2350,7 +2394,7 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams s
                                                          SplitResult *__restrict__ results,
                                                          uint64_t *keys) {
     __shared__ __align__(16) unsigned char split_lds[SPLIT_LDS_BYTES];
-    int64_t *stage = reinterpret_cast<int64_t *>(split_lds);      // [side][bin][SPLIT_ROW]
+    StagedCell *stage = reinterpret_cast<StagedCell *>(split_lds);   // [split_cell]
     CatScratch *cs_all = reinterpret_cast<CatScratch *>(split_lds);
     const int F = sh.cols, nb = sh.num_bins;
     const uint32_t groups = (uint32_t)((F + SPLIT_FEATS - 1) / SPLIT_FEATS);
@@ -2367,36 +2411,30 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams s
     const bool active = fw < nf && local != NONE;
     __shared__ unsigned long long s_key[2];          // the workgroup's best key per side
     if (tid < 2) s_key[tid] = 0;
-    // stage both sides' rows (a side without a node stages zeros)
-    const int row = 2 * nf;
-    int64_t v[SPLIT_STAGE_PER_THREAD];
+    // stage both sides' cells, 16 bytes (g, h) at a time (a side without a node
+    // stages zeros)
+    HistCell v[SPLIT_CELLS_PER_THREAD];
 #pragma unroll
-    for (int k = 0; k < SPLIT_STAGE_PER_THREAD; ++k) {
-        const int idx = tid + k * SPLIT_THREADS;
-        const int sd = idx / (256 * SPLIT_ROW), rem = idx - sd * (256 * SPLIT_ROW);
-        const int b = rem / row, r = rem - b * row;
+    for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
+        const int c = tid + k * SPLIT_THREADS;
+        const int sd = c / (256 * SPLIT_FEATS), b = c / SPLIT_FEATS % 256, q = c % SPLIT_FEATS;
         const uint32_t node = sd == 0 ? pr.built : pr.derived;
-        v[k] = (b < nb && node != NONE)
-                   ? hist_cur[(((size_t)node * nb + b) * F + f0) * 2 + r]
-                   : 0;
+        v[k] = b < nb && q < nf && node != NONE
+                   ? reinterpret_cast<const HistCell *>(hist_cur)[((size_t)node * nb + b) * F + f0 + q]
+                   : HistCell{0, 0};
     }
 #pragma unroll
-    for (int k = 0; k < SPLIT_STAGE_PER_THREAD; ++k) {
-        const int idx = tid + k * SPLIT_THREADS;
-        const int sd = idx / (256 * SPLIT_ROW), rem = idx - sd * (256 * SPLIT_ROW);
-        const int b = rem / row, r = rem - b * row;
-        if (b < nb) stage[((size_t)sd * 256 + b) * SPLIT_ROW + r] = v[k];
+    for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
+        const int c = tid + k * SPLIT_THREADS;
+        stage[split_cell(c / (256 * SPLIT_FEATS), c / SPLIT_FEATS % 256, c % SPLIT_FEATS)] = v[k];
     }
     __syncthreads();
     int64_t hg[4], hh[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int b = 4 * lane + j;
-        hg[j] = 0; hh[j] = 0;
-        if (active && b < nb) {
-            hg[j] = stage[((size_t)side * 256 + b) * SPLIT_ROW + 2 * fw];
-            hh[j] = stage[((size_t)side * 256 + b) * SPLIT_ROW + 2 * fw + 1];
-        }
+        const StagedCell cell = stage[split_cell(side, 4 * lane + j, fw)];
+        hg[j] = cell.x;
+        hh[j] = cell.y;
     }
     __syncthreads();                                 // the stage becomes split scratch
     if (active) {                                    // uniform per wavefront

@@ -1191,6 +1191,19 @@ def test_few_rows_timed_trees_alternate():
     assert a["trees"] == b["trees"]
 
 
+@pytest.mark.parametrize("leaves", [0, 7])
+@pytest.mark.parametrize("rows", [512, 513, 514, 515, 140000])
+def test_split_sum_widths(rows, leaves):
+    # labels of +-1 quantise to +-32767, so a bin of 256 rows sums to just below
+    # 2^23, where the search leaves 32-bit sums, and one of 257 rows to just above
+    half = np.arange(rows) % 2
+    x = np.stack([half, np.arange(rows) // 4 % 7, np.arange(rows) % 251]).astype(np.float32)
+    x[1, ::11] = np.nan
+    for y in (2 * half - 1, np.where(np.arange(rows) % 3 == 0, 1, -1)):
+        check_identical(x, y.astype(np.float32), {"num_trees": 2, "max_depth": 3,
+                                                  "num_leaves": leaves})
+
+
 @pytest.mark.parametrize("rows,depth,objective", [
     (3, 2, "mae"), (8191, 1, "mae"), (8193, 1, "quantile"), (40000, 1, "mae"),
     (300001, 2, "quantile")])
