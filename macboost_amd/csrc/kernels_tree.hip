@@ -1983,7 +1983,7 @@ __global__ __launch_bounds__(256) void k_reduce(Shape sh, const Pair *__restrict
                                                 int64_t *__restrict__ hist_cur, const TreeCtl *ctl,
                                                 uint32_t blocks_per_tile, int derive,
                                                 uint64_t *keys, uint64_t *cursors,
-                                                uint32_t nzero) {
+                                                uint32_t nzero, uint64_t *keys_next) {
     constexpr int CELLS = 256 / S;
     __shared__ int64_t red[S > 1 ? S : 1][CELLS][2];
     if (blockIdx.x == 0) {
@@ -1993,6 +1993,9 @@ __global__ __launch_bounds__(256) void k_reduce(Shape sh, const Pair *__restrict
             if (keys) keys[(size_t)l * KEY_STRIDE] = 0;
             if (cursors) cursors[(size_t)l * CURSOR_STRIDE] = 0;
         }
+        if (keys_next)                               // the next level's search reduces itself
+            for (uint32_t l = threadIdx.x; l < 2 * nzero; l += blockDim.x)
+                keys_next[(size_t)l * KEY_STRIDE] = 0;
     }
     const int PW = sh.part_w, nb = sh.num_bins, F = sh.cols, T = sh.hist_tiles;
     const uint32_t bpt = blockIdx.x % blocks_per_tile;
@@ -2055,7 +2058,7 @@ __global__ __launch_bounds__(256) void k_reduce(Shape sh, const Pair *__restrict
 hipError_t launch_reduce(hipStream_t s, const Shape &sh, const Pair *pairs, uint32_t max_pairs,
                          const uint64_t *partials, const int64_t *hist_prev, int64_t *hist_cur,
                          const TreeCtl *ctl, bool derive, uint64_t *keys, uint64_t *cursors,
-                         uint32_t nzero) {
+                         uint32_t nzero, uint64_t *keys_next) {
     const uint32_t cells = (uint32_t)(sh.num_bins * sh.part_w);
     const int dv = derive ? 1 : 0;
     if (!keys && !cursors) nzero = 0;
@@ -2063,12 +2066,12 @@ hipError_t launch_reduce(hipStream_t s, const Shape &sh, const Pair *pairs, uint
         const uint32_t bpt = (cells + 255) / 256;
         hipLaunchKernelGGL(k_reduce<1>, dim3(max_pairs * (uint32_t)sh.hist_tiles * bpt), dim3(256),
                            0, s, sh, pairs, partials, hist_prev, hist_cur, ctl, bpt, dv, keys,
-                           cursors, nzero);
+                           cursors, nzero, keys_next);
     } else {
         const uint32_t bpt = (cells + 63) / 64;
         hipLaunchKernelGGL(k_reduce<4>, dim3(max_pairs * (uint32_t)sh.hist_tiles * bpt), dim3(256),
                            0, s, sh, pairs, partials, hist_prev, hist_cur, ctl, bpt, dv, keys,
-                           cursors, nzero);
+                           cursors, nzero, keys_next);
     }
     return hipGetLastError();
 }
@@ -2359,7 +2362,9 @@ __device__ float node_split(const int64_t (&hg)[4], const int64_t (&hh)[4], int3
 // feature): both sides' histogram rows [bin][f0 .. f0+3] (64 contiguous bytes
 // per bin) are staged through LDS together, four independent loads per
 // thread, then wavefront (side, w) searches feature f0 + w of that side's node
-// (its 256 bins, 4 per lane).  The two sides' searches run at once.
+// (its 256 bins, 4 per lane).  The two sides' searches run at once.  With REDUCE
+// the cells come from the built node's partials and the parent's histogram instead
+// (launch_split's rule).
 constexpr int SPLIT_FEATS = 4;
 constexpr int SPLIT_WAVES = 2 * SPLIT_FEATS;
 constexpr int SPLIT_THREADS = SPLIT_WAVES * 64;
@@ -2382,6 +2387,60 @@ __device__ __forceinline__ int split_cell(int side, int bin, int q) {
     return side * SPLIT_SIDE_CELLS + bin * SPLIT_FEATS + q + (bin >> 2);
 }
 
+// Pairs from which a level may reduce its partials in the search (launch_split).
+constexpr uint32_t SPLIT_REDUCE_PAIRS = 32;
+
+// What the search needs to reduce the partials itself.
+struct SplitReduce {
+    const uint64_t *partials;
+    const int64_t *hist_prev;
+    int64_t *store;                  // the level's histograms, or NULL: not read again
+    uint64_t *keys_next;             // zeroed for the next level's search (NULL: not)
+    uint64_t *cursors;               // zeroed for the level's partition (NULL: not)
+};
+
+// The built node's cells summed over the pair's chunks: this thread's are tid and
+// tid + SPLIT_THREADS of [bin][feature], four chunks' loads of both in flight.
+constexpr int SPLIT_CELLS = 256 * SPLIT_FEATS / SPLIT_THREADS;
+
+__device__ __forceinline__ void sum_partials(const Shape &sh, const Pair &pr, int f0, int nf,
+                                             const uint64_t *__restrict__ partials,
+                                             int64_t (&g)[SPLIT_CELLS], int64_t (&h)[SPLIT_CELLS]) {
+    const int nb = sh.num_bins, T = sh.hist_tiles;
+    const size_t stride = (size_t)(nb * sh.part_w), cstride = (size_t)T * stride;
+    const uint64_t *src[SPLIT_CELLS];
+    bool live[SPLIT_CELLS];
+#pragma unroll
+    for (int k = 0; k < SPLIT_CELLS; ++k) {
+        const int c = (int)threadIdx.x + k * SPLIT_THREADS, b = c / SPLIT_FEATS, q = c % SPLIT_FEATS;
+        int tile, col;
+        partial_column(sh, f0 + min(q, nf - 1), tile, col);
+        live[k] = b < nb && q < nf;
+        src[k] = partials + ((size_t)pr.item_first + (size_t)tile) * stride +
+                 (size_t)(min(b, nb - 1) * sh.part_w + col);
+        g[k] = 0;
+        h[k] = 0;
+    }
+    constexpr uint64_t HMASK = (1ull << HIST_QH_BITS) - 1;
+    for (uint32_t c = 0; c < pr.nchunks; c += 4) {     // the last chunk's loads repeat, unused
+        uint64_t w[4][SPLIT_CELLS];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int k = 0; k < SPLIT_CELLS; ++k)
+                w[j][k] = src[k][(size_t)min(c + j, pr.nchunks - 1) * cstride];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int k = 0; k < SPLIT_CELLS; ++k)
+                if (c + j < pr.nchunks && live[k]) {
+                    g[k] += (int64_t)w[j][k] >> HIST_QH_BITS;
+                    h[k] += (int64_t)(w[j][k] & HMASK);
+                }
+    }
+}
+
+template <bool REDUCE>
 __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams sp,
                                                          const Pair *__restrict__ pairs,
                                                          const int64_t *__restrict__ hist_cur,
@@ -2392,14 +2451,23 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams s
                                                          int64_t *node_g, int64_t *node_h,
                                                          uint32_t level_start,
                                                          SplitResult *__restrict__ results,
-                                                         uint64_t *keys) {
+                                                         uint64_t *keys, SplitReduce rd) {
     __shared__ __align__(16) unsigned char split_lds[SPLIT_LDS_BYTES];
     StagedCell *stage = reinterpret_cast<StagedCell *>(split_lds);   // [split_cell]
     CatScratch *cs_all = reinterpret_cast<CatScratch *>(split_lds);
     const int F = sh.cols, nb = sh.num_bins;
     const uint32_t groups = (uint32_t)((F + SPLIT_FEATS - 1) / SPLIT_FEATS);
-    const uint32_t pair_idx = blockIdx.x / groups;
-    const int f0 = (int)(blockIdx.x % groups) * SPLIT_FEATS;
+    // consecutive workgroups go to the eight XCDs in turn; four groups share the
+    // 128-B lines of the partials, so they get one XCD (whole runs of 32 only)
+    uint32_t blk = blockIdx.x;
+    if (REDUCE && blk == 0)
+        for (uint32_t l = threadIdx.x; l < 2 * (level_start + 1); l += SPLIT_THREADS) {
+            if (rd.keys_next) rd.keys_next[(size_t)l * KEY_STRIDE] = 0;
+            if (rd.cursors && l <= level_start) rd.cursors[(size_t)l * CURSOR_STRIDE] = 0;
+        }
+    if (REDUCE && (blk | 31u) < gridDim.x) blk = (blk & ~31u) | ((blk & 7u) << 2) | ((blk >> 3) & 3u);
+    const uint32_t pair_idx = blk / groups;
+    const int f0 = (int)(blk % groups) * SPLIT_FEATS;
     if (pair_idx >= ctl->num_pairs) return;          // uniform per block
     const int nf = min(SPLIT_FEATS, F - f0);
     const Pair pr = pairs[pair_idx];
@@ -2411,22 +2479,50 @@ __global__ __launch_bounds__(SPLIT_THREADS) void k_split(Shape sh, SplitParams s
     const bool active = fw < nf && local != NONE;
     __shared__ unsigned long long s_key[2];          // the workgroup's best key per side
     if (tid < 2) s_key[tid] = 0;
-    // stage both sides' cells, 16 bytes (g, h) at a time (a side without a node
-    // stages zeros)
-    HistCell v[SPLIT_CELLS_PER_THREAD];
+    if constexpr (REDUCE) {
+        // the parent's cells load with the partials; sibling = parent - built
+        HistCell parent[SPLIT_CELLS];
 #pragma unroll
-    for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
-        const int c = tid + k * SPLIT_THREADS;
-        const int sd = c / (256 * SPLIT_FEATS), b = c / SPLIT_FEATS % 256, q = c % SPLIT_FEATS;
-        const uint32_t node = sd == 0 ? pr.built : pr.derived;
-        v[k] = b < nb && q < nf && node != NONE
-                   ? reinterpret_cast<const HistCell *>(hist_cur)[((size_t)node * nb + b) * F + f0 + q]
-                   : HistCell{0, 0};
-    }
+        for (int k = 0; k < SPLIT_CELLS; ++k) {
+            const int c = tid + k * SPLIT_THREADS, b = c / SPLIT_FEATS, q = c % SPLIT_FEATS;
+            parent[k] = b < nb && q < nf && pr.derived != NONE
+                            ? reinterpret_cast<const HistCell *>(
+                                  rd.hist_prev)[((size_t)pr.parent * nb + b) * F + f0 + q]
+                            : HistCell{0, 0};
+        }
+        int64_t g[SPLIT_CELLS], h[SPLIT_CELLS];
+        sum_partials(sh, pr, f0, nf, rd.partials, g, h);
 #pragma unroll
-    for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
-        const int c = tid + k * SPLIT_THREADS;
-        stage[split_cell(c / (256 * SPLIT_FEATS), c / SPLIT_FEATS % 256, c % SPLIT_FEATS)] = v[k];
+        for (int k = 0; k < SPLIT_CELLS; ++k) {
+            const int c = tid + k * SPLIT_THREADS, b = c / SPLIT_FEATS, q = c % SPLIT_FEATS;
+            const HistCell built = {g[k], h[k]};
+            const HistCell other = pr.derived != NONE ? parent[k] - built : HistCell{0, 0};
+            stage[split_cell(0, b, q)] = built;
+            stage[split_cell(1, b, q)] = other;
+            if (rd.store && b < nb && q < nf) {
+                HistCell *out = reinterpret_cast<HistCell *>(rd.store);
+                out[((size_t)pr.built * nb + b) * F + f0 + q] = built;
+                if (pr.derived != NONE) out[((size_t)pr.derived * nb + b) * F + f0 + q] = other;
+            }
+        }
+    } else {
+        // stage both sides' cells, 16 bytes (g, h) at a time (a side without a node
+        // stages zeros)
+        HistCell v[SPLIT_CELLS_PER_THREAD];
+#pragma unroll
+        for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
+            const int c = tid + k * SPLIT_THREADS;
+            const int sd = c / (256 * SPLIT_FEATS), b = c / SPLIT_FEATS % 256, q = c % SPLIT_FEATS;
+            const uint32_t node = sd == 0 ? pr.built : pr.derived;
+            v[k] = b < nb && q < nf && node != NONE
+                       ? reinterpret_cast<const HistCell *>(hist_cur)[((size_t)node * nb + b) * F + f0 + q]
+                       : HistCell{0, 0};
+        }
+#pragma unroll
+        for (int k = 0; k < SPLIT_CELLS_PER_THREAD; ++k) {
+            const int c = tid + k * SPLIT_THREADS;
+            stage[split_cell(c / (256 * SPLIT_FEATS), c / SPLIT_FEATS % 256, c % SPLIT_FEATS)] = v[k];
+        }
     }
     __syncthreads();
     int64_t hg[4], hh[4];
@@ -2479,11 +2575,29 @@ hipError_t launch_split(hipStream_t s, const Shape &sh, const SplitParams &sp, c
                         int64_t *hist_cur, const uint8_t *is_cat, const int8_t *monotone,
                         const uint8_t *feat_mask, const TreeCtl *ctl, const uint32_t *count,
                         int64_t *node_g, int64_t *node_h, uint32_t level_start,
-                        SplitResult *results, uint64_t *keys, uint64_t *cursors) {
+                        SplitResult *results, uint64_t *keys, uint64_t *cursors,
+                        uint64_t *keys_next, bool last) {
     if (sh.num_bins > 256) return hipErrorInvalidValue;
+    // A level's partials are about one item per CU, whatever its pairs: with many pairs
+    // a pair has few chunks and the level workgroups enough to sum them in the search,
+    // which saves a launch and reading the histograms back, and on the last level
+    // writing them.  500,009 x 53, depth 9: 128 pairs (last) 48 -> 25 us, 64 pairs 31 ->
+    // 28, 32 pairs 20 -> 23 (when last, still faster: 1M x 100 depth 7 0.4%); from 16
+    // pairs on 1M x 100 depth 6 loses 2% (eight chunks a pair).  Whole fits: that one
+    // 32.5 -> 31.1 ms, 2M x 100 depth 8 15.9 -> 15.6, 1M x 130 63 leaves 33.5 -> 32.3.
+    if (max_pairs >= (last ? SPLIT_REDUCE_PAIRS : 2 * SPLIT_REDUCE_PAIRS)) {
+        const uint32_t groups = (uint32_t)((sh.cols + SPLIT_FEATS - 1) / SPLIT_FEATS);
+        hipLaunchKernelGGL(k_split<true>, dim3(max_pairs * groups), dim3(SPLIT_THREADS), 0, s, sh,
+                           sp, pairs, nullptr, is_cat, monotone, feat_mask, ctl, count, node_g,
+                           node_h, level_start, results, keys,
+                           SplitReduce{partials, hist_prev, last ? nullptr : hist_cur, keys_next,
+                                       cursors});
+        return hipGetLastError();
+    }
     // level_start = 2^d - 1: the level holds level_start + 1 nodes
     hipError_t e = launch_reduce(s, sh, pairs, max_pairs, partials, hist_prev, hist_cur, ctl, true,
-                                 keys, cursors, level_start + 1);
+                                 keys, cursors, level_start + 1,
+                                 2 * max_pairs >= SPLIT_REDUCE_PAIRS ? keys_next : nullptr);
     if (e != hipSuccess) return e;
     return launch_find_splits(s, sh, sp, pairs, max_pairs, hist_cur, is_cat, monotone, feat_mask,
                               ctl, count, node_g, node_h, level_start, results, keys);
@@ -2497,9 +2611,9 @@ hipError_t launch_find_splits(hipStream_t s, const Shape &sh, const SplitParams 
                               SplitResult *results, uint64_t *keys) {
     if (sh.num_bins > 256) return hipErrorInvalidValue;
     const uint32_t groups = (uint32_t)((sh.cols + SPLIT_FEATS - 1) / SPLIT_FEATS);
-    hipLaunchKernelGGL(k_split, dim3(max_pairs * groups), dim3(SPLIT_THREADS), 0, s, sh, sp, pairs,
-                       hist_cur, is_cat, monotone, feat_mask, ctl, count, node_g, node_h,
-                       level_start, results, keys);
+    hipLaunchKernelGGL(k_split<false>, dim3(max_pairs * groups), dim3(SPLIT_THREADS), 0, s, sh, sp,
+                       pairs, hist_cur, is_cat, monotone, feat_mask, ctl, count, node_g, node_h,
+                       level_start, results, keys, SplitReduce{});
     return hipGetLastError();
 }
 

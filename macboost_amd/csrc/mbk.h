@@ -142,6 +142,19 @@ __host__ __device__ inline int32_t partial_feature(const Shape &sh, int32_t t, i
     return e < tile_extra_count(sh, t)
         ? sh.hist_tiles * sh.tile_w + tile_extra_first(sh, t) + e : -1;
 }
+// The tile and column of feature f's partials (partial_feature's inverse).
+__host__ __device__ inline void partial_column(const Shape &sh, int32_t f, int32_t &tile,
+                                               int32_t &col) {
+    if (f < sh.hist_tiles * sh.tile_w) {
+        tile = f / sh.tile_w;
+        col = f - tile * sh.tile_w;
+        return;
+    }
+    const int32_t e = f - sh.hist_tiles * sh.tile_w;   // an extra of the folded last tile
+    const int32_t e2 = sh.extras > sh.hist_tiles ? sh.extras - sh.hist_tiles : 0;
+    tile = e < 2 * e2 ? e / 2 : e - e2;
+    col = sh.tile_w + (e < 2 * e2 ? e & 1 : 0);
+}
 inline void set_hist_tiling(Shape &sh, bool fold = true) {
     const int32_t last = sh.cols - (sh.num_tiles - 1) * sh.tile_w;   // features of the last tile
     if (fold && sh.tile_w == 32 && sh.num_tiles >= 2 && last <= 2 * (sh.num_tiles - 1)) {
@@ -393,14 +406,17 @@ hipError_t launch_planar_rows(hipStream_t s, const Shape &sh, const uint8_t *til
 // With keys (level-local, node l's at keys[l * SPLIT_KEY_STRIDE]) every node's
 // best (gain, feature) is also left there as a split_key maximum, for the next
 // partition to decide the level (launch_route with RouteDecide) in place of
-// launch_decide; cursors (non-null) are then zeroed for that partition.
+// launch_decide; cursors (non-null) are then zeroed for that partition, and
+// keys_next (the next level's keys, another buffer) for its search.  With last,
+// hist_cur is not read after the search and may stay unwritten.
 hipError_t launch_split(hipStream_t s, const Shape &sh, const SplitParams &sp,
                         const Pair *pairs, uint32_t max_pairs, const uint64_t *partials,
                         const int64_t *hist_prev, int64_t *hist_cur, const uint8_t *is_cat,
                         const int8_t *monotone, const uint8_t *feat_mask,
                         const TreeCtl *ctl, const uint32_t *count, int64_t *node_g,
                         int64_t *node_h, uint32_t level_start, SplitResult *results,
-                        uint64_t *keys = nullptr, uint64_t *cursors = nullptr);
+                        uint64_t *keys = nullptr, uint64_t *cursors = nullptr,
+                        uint64_t *keys_next = nullptr, bool last = false);
 
 // The two halves of launch_split, for the kernel seam: partials -> built
 // histograms (and, with derive, the derived siblings), and the split search
@@ -408,7 +424,8 @@ hipError_t launch_split(hipStream_t s, const Shape &sh, const SplitParams &sp,
 hipError_t launch_reduce(hipStream_t s, const Shape &sh, const Pair *pairs, uint32_t max_pairs,
                          const uint64_t *partials, const int64_t *hist_prev, int64_t *hist_cur,
                          const TreeCtl *ctl, bool derive, uint64_t *keys = nullptr,
-                         uint64_t *cursors = nullptr, uint32_t nzero = 0);
+                         uint64_t *cursors = nullptr, uint32_t nzero = 0,
+                         uint64_t *keys_next = nullptr);
 hipError_t launch_subtract(hipStream_t s, const Shape &sh, const Pair *pairs, uint32_t max_pairs,
                            const int64_t *hist_prev, int64_t *hist_cur, const TreeCtl *ctl);
 hipError_t launch_find_splits(hipStream_t s, const Shape &sh, const SplitParams &sp,

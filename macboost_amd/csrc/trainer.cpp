@@ -1323,7 +1323,7 @@ static void setup_buffers(Trainer &t, const float *y, const float *w, const floa
         2 * (int64_t)t.dev->num_cus,
         (rows + mbk::PART_ENTRIES - 1) / mbk::PART_ENTRIES + t.max_level_nodes);
     t.route_cursor.alloc((size_t)t.max_level_nodes * mbk::CURSOR_STRIDE);
-    t.split_keys.alloc((size_t)t.max_level_nodes * mbk::SPLIT_KEY_STRIDE);
+    t.split_keys.alloc(2 * (size_t)t.max_level_nodes * mbk::SPLIT_KEY_STRIDE);   // by level parity
     t.route_done.alloc(1);
     MB_HIP(hipMemsetAsync(t.route_done.ptr, 0, sizeof(uint32_t), t.dev->stream));
 
@@ -2111,16 +2111,19 @@ static void grow_levelwise(Trainer &t, int tree) {
     // partition (launch_route with RouteDecide) from the split search's keys:
     // one launch less per level.  The deepest split level keeps its decision
     // launch, which the final leaves and the walk read.
-    const mbk::RouteDecide rd{t.split_keys.ptr, t.results.ptr, t.sp,       t.cols,
-                              t.node_g.ptr,     t.node_h.ptr,  t.bounds.ptr, t.mono.ptr, ctl};
+    auto keys_of = [&](int level) {
+        return t.split_keys.ptr +
+               (size_t)(level & 1) * (size_t)t.max_level_nodes * mbk::SPLIT_KEY_STRIDE;
+    };
     auto split_level = [&](const mbk::Shape &shl, uint32_t pairs, const int64_t *hp, int64_t *hc,
                            const mbk::LevelArgs &la) {
         const bool fold = la.level + 1 < t.D;
         MB_HIP(mbk::launch_split(s, shl, t.sp, t.pairs.ptr, pairs, t.partials.ptr, hp, hc,
                                  t.is_cat.ptr, t.mono.ptr, t.feat_mask.ptr, ctl, t.count.ptr,
                                  t.node_g.ptr, t.node_h.ptr, la.level_start, t.results.ptr,
-                                 fold ? t.split_keys.ptr : nullptr,
-                                 fold ? t.route_cursor.ptr : nullptr));
+                                 fold ? keys_of(la.level) : nullptr,
+                                 fold ? t.route_cursor.ptr : nullptr,
+                                 la.level + 2 < t.D ? keys_of(la.level + 1) : nullptr, !fold));
         if (!fold)
             MB_HIP(mbk::launch_decide(s, sh, t.sp, la, t.results.ptr, t.count.ptr, t.node_g.ptr,
                                       t.node_h.ptr, t.bounds.ptr, t.mono.ptr, ctl,
@@ -2187,6 +2190,8 @@ static void grow_levelwise(Trainer &t, int tree) {
         // name them.
         const mbk::RoutePlan rp = t.route_plan(ln, seg_next);
         const bool built_only = d == t.D - 1 && !sampled && unit_hess;
+        const mbk::RouteDecide rd{keys_of(d - 1), t.results.ptr, t.sp,         t.cols,
+                                  t.node_g.ptr,   t.node_h.ptr,  t.bounds.ptr, t.mono.ptr, ctl};
         MB_HIP(mbk::launch_route(s, sh, lp, t.bins_fm.ptr, ord_cur, ord_next, seg_cur,
                                  t.count.ptr, out, t.route_cursor.ptr, t.route_grid, true, &rp,
                                  d == 1 && !sampled, &rd, built_only));
@@ -2360,7 +2365,8 @@ static void grow_leafwise_rounds(Trainer &t, int tree) {
         hist(ord_cur, r + 1);
         MB_HIP(mbk::launch_split(s, sh, t.sp, t.pairs.ptr, 1u << r, t.partials.ptr, h_prev, h_cur,
                                  t.is_cat.ptr, t.mono.ptr, t.feat_mask.ptr, ctl, t.count.ptr,
-                                 t.node_g.ptr, t.node_h.ptr, ln.level_start, t.results.ptr));
+                                 t.node_g.ptr, t.node_h.ptr, ln.level_start, t.results.ptr,
+                                 nullptr, nullptr, nullptr, r + 2 == t.D));
     }
     select(t.D);
     finish_leafwise(t, tree, out, la.deep_walk != 0);

@@ -1204,6 +1204,24 @@ def test_split_sum_widths(rows, leaves):
                                                   "num_leaves": leaves})
 
 
+@pytest.mark.parametrize("cols,depth,tile,params", [
+    (1, 8, "", {}), (5, 9, "", {"subsample": 0.7}), (33, 8, "32", {}), (34, 9, "32", {}),
+    (70, 8, "", {"num_bins": 37}), (30, 10, "", {"num_leaves": 63}),
+    (6, 12, "", {"min_child_weight": 0.0, "monotone_constraints": [1, -1, 0, 0, 0, 0]})])
+def test_deep_levels_reduce_in_search(cols, depth, tile, params, monkeypatch):
+    # levels of 32 pairs and more reduce their partials in the split search: feature
+    # groups cut short, folded tiles, the deepest level (nothing stored), empty
+    # pairs, and keys passed on from the levels before
+    if tile:
+        monkeypatch.setenv("MACBOOST_TILE_W", tile)
+    rng = np.random.default_rng(cols)
+    x = rng.random((cols, 60001), dtype=np.float32)
+    x[0, rng.random(60001) < 0.1] = np.nan
+    v = np.nan_to_num(x)
+    y = np.sin(9 * v[0]) + v[cols // 2] * 3 + rng.standard_normal(60001)
+    check_identical(x, y.astype(np.float32), {"num_trees": 3, "max_depth": depth, **params})
+
+
 @pytest.mark.parametrize("rows,depth,objective", [
     (3, 2, "mae"), (8191, 1, "mae"), (8193, 1, "quantile"), (40000, 1, "mae"),
     (300001, 2, "quantile")])
