@@ -4726,9 +4726,9 @@ hipError_t launch_lwb_select(hipStream_t s, const Shape &sh, const SplitParams &
 //                  rows per node
 // with k_small_start (maxima, quantisation, the finished tree's covers) before them.
 // Sums are exact integers and the search is node_split, so trees are the same.
-// 20k x 100, 100 trees of depth 6: 22.8 -> 12.3 ms of kernels (k_small_level 13.1 us,
-// k_small_route 4.2, k_small_start 7.0, the last route 6.4); 1,000 x 10, 20 trees of
-// depth 4: 2.52 -> 1.32 ms.  A workgroup streams some 6.5 rows per ns, so the form
+// 20k x 100, 100 trees of depth 6: 22.8 -> 12.3 ms of kernels, 10.6 since the search
+// is in 32 bits and covers are summed by level (k_small_level 10.9 us, k_small_route
+// 4.3, the last route 6.5); 1,000 x 10, 20 trees of depth 4: 2.52 -> 1.32 ms, then 1.24.  A workgroup streams some 6.5 rows per ns, so the form
 // pays up to 100k to 250k rows (small_trees in trainer.cpp).
 // Histograms are packed words (HIST_QH_BITS: rows below 2^20), [feature][node][bin],
 // which one workgroup writes and reads again at the next level.
@@ -4870,19 +4870,25 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small_level(SmallArgs a, Spli
 }
 
 // The covers of a finished tree (t.cover[n] = the rows of n's subtree, from the
-// rows per final node), and the counters zeroed again.
+// rows per final node), and the counters zeroed again.  A level at a time, parents
+// from their children: one thread adding up its node's whole subtree (127 nodes at
+// the root of depth 6) was the longest chain of k_small_start: a 20k x 100 fit of 100
+// trees took 11.73 ms, now 11.39.
 __device__ void small_covers(uint32_t *count, float *cover, int32_t depth) {
     __shared__ uint32_t c[256];
     const uint32_t total = (2u << depth) - 1u;
-    for (uint32_t n = threadIdx.x; n < total; n += blockDim.x) c[n] = count[n];
-    __syncthreads();
     for (uint32_t n = threadIdx.x; n < total; n += blockDim.x) {
-        uint32_t sum = 0;
-        for (uint32_t first = n, wd = 1; first < total; first = 2 * first + 1, wd *= 2)
-            for (uint32_t j = 0; j < wd; ++j) sum += c[first + j];
-        cover[n] = (float)sum;
+        c[n] = count[n];
         count[n] = 0;
     }
+    __syncthreads();
+    for (uint32_t first = total >> 1; first > 0;) {    // a level's first node, deepest split level up
+        first >>= 1;
+        for (uint32_t n = first + threadIdx.x; n <= 2 * first; n += blockDim.x)
+            c[n] += c[2 * n + 1] + c[2 * n + 2];
+        __syncthreads();
+    }
+    for (uint32_t n = threadIdx.x; n < total; n += blockDim.x) cover[n] = (float)c[n];
 }
 
 __global__ __launch_bounds__(256) void k_small_covers(uint32_t *count, float *cover,
