@@ -4726,9 +4726,10 @@ hipError_t launch_lwb_select(hipStream_t s, const Shape &sh, const SplitParams &
 //                  rows per node
 // with k_small_start (maxima, quantisation, the finished tree's covers) before them.
 // Sums are exact integers and the search is node_split, so trees are the same.
-// 20k x 100, 100 trees of depth 6: 22.8 -> 12.3 ms of kernels, 10.6 since the search
-// is in 32 bits and covers are summed by level (k_small_level 10.9 us, k_small_route
-// 4.3, the last route 6.5); 1,000 x 10, 20 trees of depth 4: 2.52 -> 1.32 ms, then 1.24.  A workgroup streams some 6.5 rows per ns, so the form
+// 20k x 100, 100 trees of depth 6: 22.8 -> 12.3 ms of kernels (k_small_level 13.1 us,
+// k_small_route 4.2, k_small_start 7.0, the last route 6.4: 11.3 ms; with the search in
+// 32 bits and covers by level 11.4, 4.0, 4.0 and 6.4 us: 9.9 ms); 1,000 x 10, 20 trees
+// of depth 4: 2.52 -> 1.32 ms.  A workgroup streams some 6.5 rows per ns, so the form
 // pays up to 100k to 250k rows (small_trees in trainer.cpp).
 // Histograms are packed words (HIST_QH_BITS: rows below 2^20), [feature][node][bin],
 // which one workgroup writes and reads again at the next level.
