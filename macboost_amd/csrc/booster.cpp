@@ -235,8 +235,9 @@ void Booster::build_forest() {                    // forestBuffers, Booster.swif
                   (slots ? (int32_t)slot[f] : f) << 2 | flags};
             if (!has_cats && (flags & mbk::FLAG_CATEGORICAL)) nd = {NAN, nd.meta & ~3};
         }
-        if (has_cats && tr.cat_mask.size() >= size * 8)
-            std::memcpy(mask + t * nodes * 8, tr.cat_mask.data(), size * 32);
+        // (a model file's masks may end at the tree's last categorical node)
+        std::copy_n(tr.cat_mask.begin(), std::min(tr.cat_mask.size(), size * 8),
+                    mask + t * nodes * 8);
     }
     forest.memory.pooled = true;
     forest.memory.alloc(image.size());

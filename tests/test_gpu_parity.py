@@ -5,6 +5,7 @@ model are compared bit for bit; TreeSHAP within 1e-5 relative (+1e-6 abs)
 of the oracle's double-precision recursive TreeSHAP.
 """
 import ctypes
+import json
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -1379,6 +1380,28 @@ def test_predict_forest_slots_under_leaves(rows):
              obj["numBins"] - 1, obj["baseScore"], out)
     ctx.sync()
     assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
+
+
+def test_model_masks_end_at_last_categorical_node(tmp_path):
+    # a model file may leave out a tree's mask words after its last categorical node
+    rng = np.random.default_rng(8)
+    n = 5000
+    x = np.stack([rng.integers(0, 40, n), rng.integers(0, 9, n), rng.random(n),
+                  rng.random(n)]).astype(np.float32)
+    x[0, ::17] = np.nan
+    y = (x[1] % 3 + (np.nan_to_num(x[0]) % 4 == 1) * 2 + x[2] * x[3]).astype(np.float32)
+    h, obj = gpu_fit(x, y, {"num_trees": 12, "max_depth": 5, "categorical_features": [0, 1]})
+    shorter = 0
+    for t in obj["trees"]:
+        last = max((k for k, f in enumerate(t["feature"]) if f >= 0 and t["flags"][k] & 2),
+                   default=-1)
+        shorter += 0 <= last < len(t["feature"]) - 1
+        t["catMask"] = t["catMask"][:8 * (last + 1)]
+    assert shorter > 6
+    (tmp_path / "m.json").write_text(json.dumps(obj))
+    cut = mb.load(tmp_path / "m.json")
+    for f in (mb.predict, mb.predict_contrib):
+        assert np.array_equal(f(cut, x, feature_major=True), f(h, x, feature_major=True))
 
 
 @pytest.mark.parametrize("rows,cols,trees,depth", [
