@@ -780,6 +780,9 @@ constexpr int SHAP_MAX_BITS = 12;     // a column of 2^12 doubles is one LDS bat
 
 // One split whose outcome enters a group's bit (flags >> 16): the bit stays set
 // while the row goes left (0x100 in flags) or right (not); low flags as a split's.
+// SHAP_GENERAL: a NaN threshold, whose missing values going left are no single
+// compare.
+constexpr uint32_t SHAP_GENERAL = 0x200;
 struct ShapTest {
     int32_t feature;
     float threshold;

@@ -49,7 +49,9 @@ private:
     mbk::ShapTest test(int n, bool left, int bit) const {
         if (tr_.feature[n] >= cols_) invalid("a tree splits on a feature past the data's columns");
         return {tr_.feature[n], tr_.threshold[n],
-                (uint32_t)tr_.flags[n] | (left ? 0x100u : 0u) | ((uint32_t)bit << 16),
+                (uint32_t)tr_.flags[n] | (left ? 0x100u : 0u) |
+                    (std::isnan(tr_.threshold[n]) ? mbk::SHAP_GENERAL : 0u) |
+                    ((uint32_t)bit << 16),
                 (int32_t)(node0_ + n)};
     }
 

@@ -1422,6 +1422,29 @@ def test_treeshap_tables_edges(rows, cols, trees, depth):
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+def test_treeshap_nan_thresholds(ctx):
+    # nothing is at or below a NaN threshold, whichever way missing values go, and
+    # an infinite one is a value like others
+    x, y = O.friedman(6000, 6, 29)
+    x[:, ::13] = np.nan
+    h, obj = gpu_fit(x, y, {"num_trees": 20, "max_depth": 5})
+    x[3, 5::17] = -np.inf
+    f = model_io.forest_from_json(obj)
+    split = np.argwhere(f.feature >= 0)
+    for k, (t, n) in enumerate(split):
+        f.flags[t, n] = k % 2
+        if k % 3 == 0:
+            f.threshold[t, n] = (np.nan, np.inf, -np.inf)[k // 3 % 3]
+    rows, cols = x.shape[1], x.shape[0]
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    out = ctx.alloc(rows * (cols + 1) * 4)
+    ctx.call("mbk_treeshap", P(f.feature), P(f.threshold), P(f.flags), P(f.leaf), P(f.cover), None,
+             *f.feature.shape, obj["baseScore"], obj["numBins"] - 1, ctx.upload(x), rows, cols, out)
+    got = ctx.download(out, (rows, cols + 1), np.float32)
+    want = O.treeshap(f, obj["baseScore"], obj["numBins"], x)
+    assert np.allclose(got, want, rtol=1e-5, atol=1e-6)
+
+
 # --------------------------------------------------------------------------
 # Row checks and the base score's sums on the device (k_label_stats)
 # --------------------------------------------------------------------------
