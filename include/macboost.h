@@ -6,8 +6,9 @@
  * widths, return codes and ownership.  Errors never cross the ABI as
  * exceptions: a failing call stores a malloc'd message in *err (free it with
  * macboost_free_string) and returns NULL / -1 (1 for macboost_select_features).
- * All arrays are borrowed for the duration of the call.  A handle is not safe
- * for concurrent use.
+ * All arrays are borrowed for the duration of the call.  Predictions and
+ * contributions of one booster may run from several threads at once; any other
+ * calls on one handle must not overlap.
  *
  * Part 2 is the kernel seam (MetalEngine.dispatch, MetalEngine.swift:87-118):
  * device-pointer entry points a host written in another language can drive.

@@ -268,8 +268,8 @@ std::vector<float> Booster::predict_raw(const float *x, int64_t rows, int64_t co
         for (int k = 0; k < K; ++k)
             out[(size_t)(i * K + k)] = K > 1 ? base_scores[(size_t)k] : base_score;
     if (rows > 0 && !trees.empty()) {
-        Device &d = device();
         build_forest();
+        Device &d = device();
         DevBuf<float> xd((size_t)rows * (size_t)cols), od((size_t)rows * (size_t)K);
         upload(xd.ptr, x, xd.bytes(), d.stream);
         for (int k = 0; k < K; ++k) {

@@ -264,13 +264,13 @@ struct Booster {
     std::unique_ptr<Device> dev;
     ForestCache forest;
     std::vector<ShapPlan> shap_plans;    // per class, made by its first predict_contrib
-    std::mutex made_mu;                  // guards forest and shap_plans
+    std::mutex made_mu;                  // guards dev's creation, forest and shap_plans
 
     Booster() = default;
     Booster(const Booster &) = delete;
     Booster &operator=(const Booster &) = delete;
     ~Booster();
-    Device &device();
+    Device &device();                    // made by the first build_forest: call that before
     void build_forest();
     std::vector<float> predict(const float *x_fm, int64_t rows, int64_t cols);
     std::vector<float> predict_raw(const float *x_fm, int64_t rows, int64_t cols);

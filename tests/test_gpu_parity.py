@@ -6,6 +6,7 @@ of the oracle's double-precision recursive TreeSHAP.
 """
 import ctypes
 import json
+import threading
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -1303,6 +1304,25 @@ def test_contributions_from_several_threads():
         got = list(pool.map(lambda p: mb.predict_contrib(h, p, feature_major=True), parts * 3))
     for k, g in enumerate(got):
         assert np.array_equal(g, want[k % 4])
+
+
+def test_first_calls_from_several_threads(tmp_path):
+    # a fresh model's device and its forest there are made once, whichever of its first
+    # predictions and contributions comes first
+    x, y = O.friedman(3000, 10, 78)
+    h, _ = gpu_fit(x, y, {"num_trees": 20, "max_depth": 5})
+    mb.save(h, tmp_path / "m.json")
+    want = [f(h, x, feature_major=True) for f in (mb.predict, mb.predict_contrib)]
+    for _ in range(4):
+        fresh, together = mb.load(tmp_path / "m.json"), threading.Barrier(8)
+
+        def first(k):
+            together.wait(60)
+            return (mb.predict, mb.predict_contrib)[k % 2](fresh, x, feature_major=True)
+
+        with ThreadPoolExecutor(8) as pool:
+            for k, got in enumerate(pool.map(first, range(8))):
+                assert np.array_equal(got, want[k % 2])
 
 
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
