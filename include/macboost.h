@@ -7,8 +7,9 @@
  * exceptions: a failing call stores a malloc'd message in *err (free it with
  * macboost_free_string) and returns NULL / -1 (1 for macboost_select_features).
  * All arrays are borrowed for the duration of the call.  Predictions and
- * contributions of one booster may run from several threads at once; any other
- * calls on one handle must not overlap.
+ * contributions of one booster may run from several threads at once, and so may
+ * mbk_predict_forest and mbk_treeshap on one context; any other calls on one handle
+ * must not overlap.
  *
  * Part 2 is the kernel seam (MetalEngine.dispatch, MetalEngine.swift:87-118):
  * device-pointer entry points a host written in another language can drive.

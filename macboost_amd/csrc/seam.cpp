@@ -64,6 +64,7 @@ struct Scratch {
     mb::ShapPlan shap_plan;                          // mbk_treeshap
     mb::ShapScratch shap;
     DevBuf<uint32_t> shap_mask;
+    std::mutex shap_mu;              // a call holds them until its work is done
     // mbk_predict_forest, allocated with the context (its calls allocate nothing)
     DevBuf<uint32_t> forest_features;
     DevBuf<mbk::PredNode> nodes;
@@ -577,6 +578,7 @@ int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshol
         const int64_t width = (int64_t)cols + 1;
         if (rows == 0) return 0;
         Scratch &sc = ctx->scratch;
+        std::lock_guard<std::mutex> lock(sc.shap_mu);
         const uint32_t *mask_dev = nullptr;
         if (mask) {
             const size_t words = (size_t)num_trees * npt * 8;

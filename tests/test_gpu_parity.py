@@ -1325,6 +1325,41 @@ def test_first_calls_from_several_threads(tmp_path):
                 assert np.array_equal(got, want[k % 2])
 
 
+def test_context_calls_from_several_threads(ctx):
+    # contributions and predictions of different forests on one context: the calls
+    # share its scratch and each gets its own forest's results
+    x, y = O.friedman(6000, 8, 79)
+    xd = ctx.upload(x)
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    work = []
+    for depth in (3, 5, 7, 9):
+        _, obj = gpu_fit(x, y, {"num_trees": 12, "max_depth": depth})
+        f = model_io.forest_from_json(obj)
+        dev = [ctx.upload(a) for a in (f.feature, f.threshold, f.flags, f.leaf)]
+        work.append((f, obj, dev, ctx.alloc(6000 * 9 * 4), ctx.alloc(6000 * 4)))
+
+    def call(w):
+        f, obj, dev, contrib, pred = w
+        for _ in range(5):
+            ctx.call("mbk_treeshap", P(f.feature), P(f.threshold), P(f.flags), P(f.leaf),
+                     P(f.cover), None, *f.feature.shape, obj["baseScore"], obj["numBins"] - 1, xd,
+                     6000, 8, contrib)
+            ctx.call("mbk_predict_forest", *dev, None, *f.feature.shape, xd, 6000,
+                     obj["numBins"] - 1, obj["baseScore"], pred)
+
+    def results():
+        ctx.sync()
+        return [ctx.download(w[k], (6000, n), np.float32) for w in work for k, n in ((3, 9), (4, 1))]
+
+    for w in work:
+        call(w)
+    want = results()
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(call, work))
+    for g, w in zip(results(), want):
+        assert np.array_equal(g, w)
+
+
 @pytest.mark.parametrize("card", [1, 2, 63, 64, 65, 128, 129, 254])
 def test_categorical_rank_sizes(card):
     # the split search ranks a node's categories 64 at a time, four keys a read:
