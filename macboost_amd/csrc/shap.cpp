@@ -31,7 +31,7 @@ public:
     size_t add() {
         std::vector<uint8_t> &h = plan_.height;
         h.assign((size_t)tr_.nodes, 0);
-        for (int n = (tr_.nodes - 3) / 2; n >= 0; --n)
+        for (int n = (tr_.nodes - 1) / 2 - 1; n >= 0; --n)    // slots with both children
             if (tr_.feature[n] >= 0)
                 h[(size_t)n] = (uint8_t)(1 + std::max(h[(size_t)(2 * n + 1)], h[(size_t)(2 * n + 2)]));
         if (h[0] > 0) walk(0);                         // a lone leaf: bias only

@@ -1477,6 +1477,27 @@ def test_treeshap_tables_edges(rows, cols, trees, depth):
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("nodes", [1, 2, 3, 4])
+def test_treeshap_smallest_heaps(ctx, nodes):
+    # a split without both its children in the heap is no split
+    feature = np.array([[1, -1, -1, -1], [0, 0, 0, -1]], np.int32)[:, :nodes].copy()
+    leaf = np.array([[1, 2, 4, 8], [16, 32, 64, 128]], np.float32)[:, :nodes].copy()
+    cover = np.array([[4, 1, 3, 0], [2, 1, 1, 0]], np.float32)[:, :nodes].copy()
+    threshold, flags = np.full(leaf.shape, 0.5, np.float32), np.zeros(leaf.shape, np.uint8)
+    x = np.array([[0.0, 1.0, 0.0], [0.0, 0.0, 1.0]], np.float32)
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    out = ctx.alloc(3 * 3 * 4)
+    ctx.call("mbk_treeshap", P(feature), P(threshold), P(flags), P(leaf), P(cover), None, 2, nodes,
+             0.25, 255, ctx.upload(x), 3, 2, out)
+    got = ctx.download(out, (3, 3), np.float32)
+    if nodes < 3:
+        want = [[0, 0, 0.25 + 1 + 16]] * 3
+    else:                                              # the second tree's children: no leaves
+        want = [[0, 2 - 3.5, 0.25 + 3.5 + 48], [0, 2 - 3.5, 0.25 + 3.5 + 48],
+                [0, 4 - 3.5, 0.25 + 3.5 + 48]]
+    assert np.allclose(got, want, rtol=1e-6, atol=1e-6)
+
+
 def test_treeshap_nan_thresholds(ctx):
     # nothing is at or below a NaN threshold, whichever way missing values go, and
     # an infinite one is a value like others
