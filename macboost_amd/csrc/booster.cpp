@@ -413,7 +413,7 @@ void Booster::contrib_class(const float *x, int64_t rows, int64_t cols, int k, f
     Device &d = device();
     DevBuf<float> xd((size_t)rows * (size_t)cols), od((size_t)rows * (size_t)width);
     upload(xd.ptr, x, xd.bytes(), d.stream);
-    // a call orders its plan's columns for its own rows, on the one stream anyway
+    // one call at a time, on the one stream anyway: the first makes the plan
     std::lock_guard<std::mutex> lock(made_mu);
     if (shap_plans.empty()) shap_plans.resize((size_t)K);
     ShapScratch scratch;

@@ -240,8 +240,7 @@ struct ShapPlan {
     bool made = false;
     std::vector<ShapSetPlan> sets;
     size_t num_sets = 0;
-    double evals = 0;          // path evaluations of the tables
-    double paths = 0;
+    int64_t paths = 0;
     bool fits = true;          // every group within SHAP_MAX_BITS
     std::vector<uint8_t> height;
 };

@@ -15,10 +15,17 @@ namespace {
 constexpr size_t SET_DOUBLES = (size_t)1 << 25;
 // Bytes of a slab's outcomes and of its runs.
 constexpr size_t SLAB_BYTES = (size_t)128 << 20;
-// Rows up to which the path kernel's time hardly depends on them (100 trees of
-// depth 6: 0.85 ms for 1 to 1,024 rows, against 0.48-0.60 ms with tables; 10
-// trees of depth 12: 9.4 against 2.2 ms).
-constexpr int64_t PATH_LATENCY_ROWS = 1024;
+// Workgroups that share the batches of a row block.  A share's end cuts a feature's
+// sum, so their number goes by the plan alone: a row's result does not depend on the
+// other rows of its call.  Each costs a store of its rows' sums, fewer leave the
+// chip idle for few rows.  100 trees of depth 6, 1k and 200k rows: 0.31 and 1.30 ms
+// with 32 shares, 0.28 and 1.24 with 64, 0.27 and 1.25 with 128 (0.26 and 1.32 when
+// each call took what filled the chip).  50 trees of depth 9, 20k rows: 4.21 ms with
+// 64, 3.83 with 128, 3.70 with 256, 3.74 with 512 (3.81); many batches a share repay
+// the stores there.
+int plan_shares(int32_t batches) {
+    return std::max(1, std::min(std::clamp(batches / 16, 128, 256), batches));
+}
 
 // One tree's groups, appended to a set.
 class TreeGroups {
@@ -133,9 +140,7 @@ private:
         sp_.set.max_bits = std::max(sp_.set.max_bits, G.bits);
         sp_.set.max_slots = std::max(sp_.set.max_slots, anc_ + extra);
         doubles_ += (size_t)nf << G.bits;
-        const double leaves = (double)__builtin_popcount(G.leaves);
-        plan_.evals += leaves * (double)(1u << G.bits);
-        plan_.paths += leaves;
+        plan_.paths += __builtin_popcount(G.leaves);
     }
 
     static constexpr int SHAP_FEATURES = 16;
@@ -151,9 +156,9 @@ private:
     int depth_ = 0, anc_ = 0;
 };
 
-// The set's columns in feature order, cut into LDS batches, and the runs of
-// `shares` workgroups per row block.
-void order_columns(ShapSetPlan &sp, int32_t cols, int shares) {
+// The set's columns in feature order, cut into LDS batches, and the runs of the
+// workgroups that share them.
+void order_columns(ShapSetPlan &sp, int32_t cols) {
     constexpr uint32_t BATCH = 4096;                   // doubles (SHAP_LDS_DOUBLES)
     const size_t n = sp.col_feature.size();
     std::vector<uint32_t> &at = sp.at, &order = sp.order;
@@ -186,7 +191,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols, int shares) {
     sp.set.table_len = off;
     sp.set.num_groups = (int32_t)sp.groups.size();
     sp.set.num_batches = (int32_t)sp.batches.size();
-    sp.set.shares = std::max(1, std::min(shares, sp.set.num_batches));
+    sp.set.shares = plan_shares(sp.set.num_batches);
     // a run ends with its feature or with its workgroup's share of the batches
     sp.run_first.assign((size_t)cols + 1, 0u);
     uint32_t run = 0;
@@ -210,7 +215,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols, int shares) {
 void make_plan(ShapPlan &plan, const std::vector<TreeView> &trees, size_t first, size_t step,
                int nodes_per_tree, int32_t cols) {
     plan.num_sets = 0;
-    plan.evals = plan.paths = 0;
+    plan.paths = 0;
     plan.fits = true;
     size_t doubles = SET_DOUBLES;
     for (size_t t = first; t < trees.size() && plan.fits; t += step) {
@@ -224,6 +229,8 @@ void make_plan(ShapPlan &plan, const std::vector<TreeView> &trees, size_t first,
         doubles += tg.add();
         if (doubles > 4 * SET_DOUBLES) plan.fits = false;   // one tree's tables pass 1 GB
     }
+    if (plan.fits)
+        for (size_t k = 0; k < plan.num_sets; ++k) order_columns(plan.sets[k], cols);
     plan.made = true;
 }
 
@@ -275,10 +282,13 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
               int nodes_per_tree, const ShapCall &c, ShapPlan &plan, ShapScratch &sc) {
     if (!plan.made) make_plan(plan, trees, first, step, nodes_per_tree, c.cols);
     if (plan.fits && plan.paths == 0) return false;
-    // The tables cost `evals` path evaluations whatever the number of rows; the
-    // path kernel costs rows * paths, and for few rows the latency of its
-    // chain of passes, which the tables' launch fills the chip for.
-    if (!plan.fits || plan.evals > plan.paths * (double)std::max<int64_t>(c.rows, PATH_LATENCY_ROWS)) {
+    // A row's last bits depend on the kernels, so the rows of the call do not enter the
+    // choice: tables wherever they fit.  They would lose to a path per lane at few
+    // rows and many outcomes, and do not: trees of depth 11 with another feature on
+    // every level (2^12 outcomes a group, the most that fit), 1 to 2,048 rows, 1.0 ms
+    // a call either way for one tree, 7.7 ms against 6.7 to 9.2 for 10, 40 against 57
+    // for 50.
+    if (!plan.fits) {
         run_paths(s, trees, first, step, nodes_per_tree, c, sc);
         MB_HIP(hipStreamSynchronize(s));               // the arrays leave with this call
         return true;
@@ -290,21 +300,18 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
     for (size_t k = 0; k < plan.num_sets; ++k) {
         const ShapSetPlan &sp = plan.sets[k];
         row_bytes = std::max({row_bytes, sp.groups.size() * (sp.set.max_bits > 8 ? 2 : 1),
-                              (std::min<size_t>((size_t)c.cols, sp.col_feature.size()) + 16) * 8});
+                              (size_t)sp.set.num_runs * 8});
     }
     const int64_t blocks = std::min<int64_t>(
         blocks_all, std::max<int64_t>(1, (int64_t)(SLAB_BYTES / row_bytes / BLOCK)));
     const int64_t slab = blocks * BLOCK;
-    // about four workgroups per CU
-    const int shares = (int)std::max<int64_t>(1, (1024 + blocks - 1) / blocks);
     std::vector<char> &blob = sc.blob;
     blob.clear();
     struct Offsets { size_t tests, groups, vals, col_off, items, batches, run_first; };
     std::vector<Offsets> offs;
     size_t table = 2, pattern_bytes = 16, runs = 1;
     for (size_t k = 0; k < plan.num_sets; ++k) {
-        ShapSetPlan &sp = plan.sets[k];
-        order_columns(sp, c.cols, shares);
+        const ShapSetPlan &sp = plan.sets[k];
         offs.push_back({append(blob, sp.tests), append(blob, sp.groups), append(blob, sp.vals),
                         append(blob, sp.col_off), append(blob, sp.items),
                         append(blob, sp.batches), append(blob, sp.run_first)});

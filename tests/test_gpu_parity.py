@@ -1477,6 +1477,43 @@ def test_treeshap_tables_edges(rows, cols, trees, depth):
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("trees,depth", [(40, 6), (6, 9), (1, 11)])
+def test_contributions_do_not_depend_on_the_batch(ctx, trees, depth):
+    # a row's sums are added in one order whatever other rows are in the call: every
+    # tree is there a second time with its leaves negated, so that nothing but the
+    # roundings of that order is left.  Depth 11, every level another feature: the
+    # largest tables against the rows of a call.
+    rng = np.random.default_rng(depth)
+    cols, inner = 12, 2 ** depth - 1
+    shape = (trees, 2 * inner + 1)
+    feature = np.full(shape, -1, np.int32)
+    feature[:, :inner] = (np.floor(np.log2(np.arange(inner) + 1)).astype(np.int32)
+                          + np.arange(trees)[:, None]) % cols
+    threshold = rng.random(shape, dtype=np.float32)
+    cover = np.zeros(shape, np.float32)
+    cover[:, inner:] = rng.integers(1, 50, (trees, inner + 1))
+    for n in range(inner - 1, -1, -1):
+        cover[:, n] = cover[:, 2 * n + 1] + cover[:, 2 * n + 2]
+    leaf = rng.standard_normal(shape).astype(np.float32)
+    twice = lambda a: np.ascontiguousarray(np.concatenate([a, a]))
+    feature, threshold, cover = twice(feature), twice(threshold), twice(cover)
+    leaf = np.concatenate([leaf, -leaf])
+    flags = np.zeros(feature.shape, np.uint8)
+    x = rng.random((cols, 20000), dtype=np.float32)
+    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+
+    def contrib(rows):
+        out = ctx.alloc(rows * (cols + 1) * 4)
+        ctx.call("mbk_treeshap", P(feature), P(threshold), P(flags), P(leaf), P(cover), None,
+                 *feature.shape, 0.5, 255, ctx.upload(x[:, :rows]), rows, cols, out)
+        return ctx.download(out, (rows, cols + 1), np.float32)
+
+    want = contrib(x.shape[1])
+    assert np.abs(want[:, :cols]).max() < 1e-9 and np.count_nonzero(want[:, :cols])
+    for rows in (1, 70, 2049, 5000):
+        assert np.array_equal(contrib(rows), want[:rows])
+
+
 @pytest.mark.parametrize("nodes", [1, 2, 3, 4])
 def test_treeshap_smallest_heaps(ctx, nodes):
     # a split without both its children in the heap is no split
