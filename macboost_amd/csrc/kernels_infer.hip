@@ -1019,14 +1019,15 @@ __global__ __launch_bounds__(SHAP_THREADS) void k_shap_sum(const ShapItem *__res
 }
 
 // Adds up each feature's runs (and, with several table sets, the sums of the
-// earlier ones: total, [cols][rows] f64), 64 rows x 64 features per workgroup
+// earlier ones: total, [cols][total_rows] f64), 64 rows x 64 features per workgroup
 // through an LDS transpose; the last set writes f32 rows and the bias.
 __global__ __launch_bounds__(256) void k_shap_finish(const double *__restrict__ runs,
                                                      size_t run_pitch,
                                                      const uint32_t *__restrict__ run_first,
                                                      int64_t row0, int64_t rows, int32_t cols,
-                                                     double *__restrict__ total, int first,
-                                                     int last, float bias,
+                                                     double *__restrict__ total,
+                                                     int64_t total_row0, int64_t total_rows,
+                                                     int first, int last, float bias,
                                                      float *__restrict__ out) {
     __shared__ float tile[64][65];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1036,11 +1037,12 @@ __global__ __launch_bounds__(256) void k_shap_finish(const double *__restrict__ 
     const int64_t row = r0 + lane;
     for (int f = wave; f < nf; f += 4) {
         double v = 0.0;
-        if (!first && row < rows) v = total[(size_t)(f0 + f) * (size_t)rows + (size_t)row];
+        double *sum = total + (size_t)(f0 + f) * (size_t)total_rows + (size_t)(row - total_row0);
+        if (!first && row < rows) v = *sum;
         for (uint32_t k = run_first[f0 + f]; k < run_first[f0 + f + 1]; ++k)
             v += runs[(size_t)k * run_pitch + (size_t)(row - row0)];
         if (!last) {
-            if (row < rows) total[(size_t)(f0 + f) * (size_t)rows + (size_t)row] = v;
+            if (row < rows) *sum = v;
         } else {
             tile[lane][f] = (float)v;
         }
@@ -1092,7 +1094,7 @@ static hipError_t shap_slab(hipStream_t s, const ShapSet &set, const ShapSetDev 
     const int64_t live = std::min<int64_t>(w.slab_rows, w.rows - w.row0);
     hipLaunchKernelGGL(k_shap_finish, dim3((unsigned)((live + 63) / 64), (unsigned)((w.cols + 63) / 64)),
                        dim3(256), 0, s, w.runs, (size_t)w.slab_rows, d.run_first, w.row0, w.rows,
-                       w.cols, w.total, w.first, w.last, w.bias, w.out);
+                       w.cols, w.total, w.total_row0, w.total_rows, w.first, w.last, w.bias, w.out);
     return hipGetLastError();
 }
 

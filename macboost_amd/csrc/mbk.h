@@ -830,8 +830,8 @@ struct ShapSetDev {
     const uint32_t *run_first;       // [cols + 1]
 };
 // Rows [row0, row0 + slab_rows) of x (slab_rows a multiple of SHAP_BLOCK_ROWS; rows past
-// the end are not written).  total: [cols][rows] f64, needed when there are
-// several sets; first / last: of the sets.
+// the end are not written).  total: [cols][total_rows] f64 of the rows from
+// total_row0 on, needed when there are several sets; first / last: of the sets.
 struct ShapSlab {
     const float *x;
     int64_t rows, row0, slab_rows;
@@ -841,6 +841,7 @@ struct ShapSlab {
     void *patterns;                  // num_groups * slab_rows bytes, 2 per row past 8 bits
     double *runs;                    // num_runs * slab_rows
     double *total;
+    int64_t total_row0, total_rows;
     int first, last;
     float bias;
     float *out;

@@ -10,11 +10,17 @@ namespace mb {
 
 namespace {
 
-// Doubles of one set's tables: trees are split into sets so that a set's
-// columns stay in the 256 MB last-level cache and scratch stays bounded.
+// Doubles of a set's tables before its last tree: trees are split into sets so
+// that a set's columns stay in the 256 MB last-level cache and scratch stays bounded
+// (the last tree adds 1,024 groups of 12 columns of 2^12 doubles at most: with it
+// below 0.7 GB).
 constexpr size_t SET_DOUBLES = (size_t)1 << 25;
 // Bytes of a slab's outcomes and of its runs.
 constexpr size_t SLAB_BYTES = (size_t)128 << 20;
+// Bytes of the sums that several sets share: more rows go in passes, each making
+// the sets' tables again (a pass is 671k rows
+// of 100 columns).
+constexpr size_t SUM_BYTES = (size_t)512 << 20;
 // Workgroups that share the batches of a row block.  A share's end cuts a feature's
 // sum, so their number goes by the plan alone: a row's result does not depend on the
 // other rows of its call.  Each costs a store of its rows' sums, fewer leave the
@@ -227,7 +233,6 @@ void make_plan(ShapPlan &plan, const std::vector<TreeView> &trees, size_t first,
         }
         TreeGroups tg(plan, plan.sets[plan.num_sets - 1], trees[t], t, nodes_per_tree, cols);
         doubles += tg.add();
-        if (doubles > 4 * SET_DOUBLES) plan.fits = false;   // one tree's tables pass 1 GB
     }
     if (plan.fits)
         for (size_t k = 0; k < plan.num_sets; ++k) order_columns(plan.sets[k], cols);
@@ -302,8 +307,11 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
         row_bytes = std::max({row_bytes, sp.groups.size() * (sp.set.max_bits > 8 ? 2 : 1),
                               (size_t)sp.set.num_runs * 8});
     }
-    const int64_t blocks = std::min<int64_t>(
-        blocks_all, std::max<int64_t>(1, (int64_t)(SLAB_BYTES / row_bytes / BLOCK)));
+    const bool several = plan.num_sets > 1;
+    const int64_t sum_rows = (int64_t)(SUM_BYTES / 8 / (size_t)c.cols);
+    int64_t blocks = (int64_t)(SLAB_BYTES / row_bytes / BLOCK);
+    if (several) blocks = std::min(blocks, sum_rows / BLOCK);
+    blocks = std::min(blocks_all, std::max<int64_t>(1, blocks));
     const int64_t slab = blocks * BLOCK;
     std::vector<char> &blob = sc.blob;
     blob.clear();
@@ -320,42 +328,51 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
                                                     (sp.set.max_bits > 8 ? 2 : 1));
         runs = std::max(runs, (size_t)sp.set.num_runs * (size_t)slab);
     }
-    const bool several = plan.num_sets > 1;
     char *d = reserve(sc.arrays, blob.size());
     reserve(sc.table, table);
     reserve(sc.patterns, pattern_bytes);
     reserve(sc.runs, runs);
-    if (several) reserve(sc.sums, (size_t)c.rows * (size_t)c.cols);
+    // rows of a pass over the sets, whole slabs
+    int64_t pass = c.rows;
+    if (several) {
+        pass = std::min(c.rows, std::max(slab, sum_rows / slab * slab));
+        reserve(sc.sums, (size_t)pass * (size_t)c.cols);
+    }
     MB_HIP(hipMemcpyAsync(d, blob.data(), blob.size(), hipMemcpyHostToDevice, s));
-    for (size_t k = 0; k < plan.num_sets; ++k) {
-        const ShapSetPlan &sp = plan.sets[k];
-        const Offsets &o = offs[k];
-        const mbk::ShapSetDev dev{reinterpret_cast<mbk::ShapTest *>(d + o.tests),
-                                  reinterpret_cast<mbk::ShapGroup *>(d + o.groups),
-                                  reinterpret_cast<double *>(d + o.vals),
-                                  reinterpret_cast<uint32_t *>(d + o.col_off),
-                                  reinterpret_cast<mbk::ShapItem *>(d + o.items),
-                                  reinterpret_cast<mbk::ShapBatch *>(d + o.batches),
-                                  reinterpret_cast<uint32_t *>(d + o.run_first)};
-        MB_HIP(mbk::launch_shap_tables(s, sp.set, dev, sc.table.ptr));
-        for (int64_t r0 = 0; r0 < c.rows; r0 += slab) {
-            mbk::ShapSlab w{};
-            w.x = c.x;
-            w.rows = c.rows;
-            w.row0 = r0;
-            w.slab_rows = std::min(slab, (c.rows - r0 + BLOCK - 1) / BLOCK * BLOCK);
-            w.cols = c.cols;
-            w.data_bins = c.data_bins;
-            w.masks = c.masks;
-            w.table = sc.table.ptr;
-            w.patterns = sc.patterns.ptr;
-            w.runs = sc.runs.ptr;
-            w.total = several ? sc.sums.ptr : nullptr;
-            w.first = k == 0;
-            w.last = k + 1 == plan.num_sets;
-            w.bias = c.bias;
-            w.out = c.out;
-            MB_HIP(mbk::launch_shap_slab(s, sp.set, dev, w));
+    for (int64_t p0 = 0; p0 < c.rows; p0 += pass) {
+        const int64_t p1 = std::min(c.rows, p0 + pass);
+        for (size_t k = 0; k < plan.num_sets; ++k) {
+            const ShapSetPlan &sp = plan.sets[k];
+            const Offsets &o = offs[k];
+            const mbk::ShapSetDev dev{reinterpret_cast<mbk::ShapTest *>(d + o.tests),
+                                      reinterpret_cast<mbk::ShapGroup *>(d + o.groups),
+                                      reinterpret_cast<double *>(d + o.vals),
+                                      reinterpret_cast<uint32_t *>(d + o.col_off),
+                                      reinterpret_cast<mbk::ShapItem *>(d + o.items),
+                                      reinterpret_cast<mbk::ShapBatch *>(d + o.batches),
+                                      reinterpret_cast<uint32_t *>(d + o.run_first)};
+            MB_HIP(mbk::launch_shap_tables(s, sp.set, dev, sc.table.ptr));
+            for (int64_t r0 = p0; r0 < p1; r0 += slab) {
+                mbk::ShapSlab w{};
+                w.x = c.x;
+                w.rows = c.rows;
+                w.row0 = r0;
+                w.slab_rows = std::min(slab, (p1 - r0 + BLOCK - 1) / BLOCK * BLOCK);
+                w.cols = c.cols;
+                w.data_bins = c.data_bins;
+                w.masks = c.masks;
+                w.table = sc.table.ptr;
+                w.patterns = sc.patterns.ptr;
+                w.runs = sc.runs.ptr;
+                w.total = several ? sc.sums.ptr : nullptr;
+                w.total_row0 = p0;
+                w.total_rows = pass;
+                w.first = k == 0;
+                w.last = k + 1 == plan.num_sets;
+                w.bias = c.bias;
+                w.out = c.out;
+                MB_HIP(mbk::launch_shap_slab(s, sp.set, dev, w));
+            }
         }
     }
     MB_HIP(hipStreamSynchronize(s));                   // the arrays leave with this call

@@ -1463,7 +1463,7 @@ def test_model_masks_end_at_last_categorical_node(tmp_path):
     (1, 8, 40, 6),            # one row: every share of the columns its own workgroup
     (2049, 9, 5, 1),          # one-split groups, a row past a row block
     (2047, 70, 30, 9),        # outcomes of more than 8 bits, features past one finish tile
-    (2000, 8, 60, 9),         # several table sets
+    (2000, 8, 60, 9),         # more than one share of the columns per feature
     (70, 4100, 3, 12),        # wide and too deep for tables: the lane-per-row kernel
 ])
 def test_treeshap_tables_edges(rows, cols, trees, depth):
@@ -1477,41 +1477,81 @@ def test_treeshap_tables_edges(rows, cols, trees, depth):
     assert np.allclose(c, want, rtol=1e-5, atol=1e-6)
 
 
-@pytest.mark.parametrize("trees,depth", [(40, 6), (6, 9), (1, 11)])
+def level_forest(rng, trees, depth, cols):
+    # complete trees, every level another feature (the next tree's one further on):
+    # the most outcomes a group of paths can have
+    inner = 2 ** depth - 1
+    f = O.Forest.empty(trees, 2 * inner + 1)
+    f.feature[:] = -1
+    f.feature[:, :inner] = (np.floor(np.log2(np.arange(inner) + 1)).astype(np.int32)
+                            + np.arange(trees)[:, None]) % cols
+    f.threshold[:] = rng.random(f.threshold.shape)
+    f.leaf[:] = rng.standard_normal(f.leaf.shape)
+    f.cover[:, inner:] = rng.integers(1, 50, (trees, inner + 1))
+    for n in range(inner - 1, -1, -1):
+        f.cover[:, n] = f.cover[:, 2 * n + 1] + f.cover[:, 2 * n + 2]
+    return f
+
+
+def seam_contributions(ctx, f, base, num_bins, x, taken=None):
+    # taken: appends the device memory that the call left allocated
+    cols, rows = x.shape
+    P = lambda a: np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)
+    xd, out = ctx.upload(x), ctx.alloc(rows * (cols + 1) * 4)
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        left, total = ctypes.c_size_t(), ctypes.c_size_t()
+        ctx.sync()
+        assert hip.hipMemGetInfo(ctypes.byref(left), ctypes.byref(total)) == 0
+        return left.value
+
+    before = free()
+    ctx.call("mbk_treeshap", P(f.feature), P(f.threshold), P(f.flags), P(f.leaf), P(f.cover), None,
+             *f.feature.shape, base, num_bins - 1, xd, rows, cols, out)
+    if taken is not None:
+        taken.append(before - free())
+    return ctx.download(out, (rows, cols + 1), np.float32)
+
+
+@pytest.mark.parametrize("trees,depth", [(40, 6), (6, 9), (8, 10), (1, 11)])
 def test_contributions_do_not_depend_on_the_batch(ctx, trees, depth):
     # a row's sums are added in one order whatever other rows are in the call: every
     # tree is there a second time with its leaves negated, so that nothing but the
-    # roundings of that order is left.  Depth 11, every level another feature: the
-    # largest tables against the rows of a call.
+    # roundings of that order is left.  One table set and (depth 10) several; depth
+    # 11: the largest tables against the rows of a call.
     rng = np.random.default_rng(depth)
-    cols, inner = 12, 2 ** depth - 1
-    shape = (trees, 2 * inner + 1)
-    feature = np.full(shape, -1, np.int32)
-    feature[:, :inner] = (np.floor(np.log2(np.arange(inner) + 1)).astype(np.int32)
-                          + np.arange(trees)[:, None]) % cols
-    threshold = rng.random(shape, dtype=np.float32)
-    cover = np.zeros(shape, np.float32)
-    cover[:, inner:] = rng.integers(1, 50, (trees, inner + 1))
-    for n in range(inner - 1, -1, -1):
-        cover[:, n] = cover[:, 2 * n + 1] + cover[:, 2 * n + 2]
-    leaf = rng.standard_normal(shape).astype(np.float32)
-    twice = lambda a: np.ascontiguousarray(np.concatenate([a, a]))
-    feature, threshold, cover = twice(feature), twice(threshold), twice(cover)
-    leaf = np.concatenate([leaf, -leaf])
-    flags = np.zeros(feature.shape, np.uint8)
-    x = rng.random((cols, 20000), dtype=np.float32)
-    P = lambda a: a.ctypes.data_as(ctypes.c_void_p)
-
-    def contrib(rows):
-        out = ctx.alloc(rows * (cols + 1) * 4)
-        ctx.call("mbk_treeshap", P(feature), P(threshold), P(flags), P(leaf), P(cover), None,
-                 *feature.shape, 0.5, 255, ctx.upload(x[:, :rows]), rows, cols, out)
-        return ctx.download(out, (rows, cols + 1), np.float32)
-
-    want = contrib(x.shape[1])
-    assert np.abs(want[:, :cols]).max() < 1e-9 and np.count_nonzero(want[:, :cols])
+    f = level_forest(rng, trees, depth, 12)
+    for name in ("feature", "threshold", "flags", "leaf", "cover"):
+        a = getattr(f, name)
+        setattr(f, name, np.concatenate([a, -a if name == "leaf" else a]))
+    x = rng.random((12, 20000), dtype=np.float32)
+    want = seam_contributions(ctx, f, 0.5, 256, x)
+    assert np.abs(want[:, :12]).max() < 1e-9 and np.count_nonzero(want[:, :12])
     for rows in (1, 70, 2049, 5000):
-        assert np.array_equal(contrib(rows), want[:rows])
+        xs = np.ascontiguousarray(x[:, :rows])
+        assert np.array_equal(seam_contributions(ctx, f, 0.5, 256, xs), want[:rows])
+
+
+def test_treeshap_several_table_sets():
+    # forests of several table sets (15 trees of 5.2M doubles, 2^25 a set): the sums
+    # they share hold a pass of rows, not all of them, and wide rows in several passes
+    # get the values of rows without the columns that no tree uses
+    rng = np.random.default_rng(5)
+    f = level_forest(rng, 15, 10, 11)
+    rows, cols = 40000, 6000
+    wide = np.zeros((cols, rows), np.float32)
+    wide[:11] = rng.random((11, rows))
+    ctx, taken = mb.Context(0), []
+    got = seam_contributions(ctx, f, 0.5, 256, wide, taken)
+    assert taken[0] < 1.2e9                            # rows x cols doubles are 1.9 GB
+    x = np.ascontiguousarray(wide[:11])
+    narrow = seam_contributions(ctx, f, 0.5, 256, x)
+    assert np.array_equal(got[:, :11], narrow[:, :11])
+    assert not got[:, 11:-1].any() and np.array_equal(got[:, -1], narrow[:, -1])
+    some = np.ascontiguousarray(x[:, ::400])
+    assert np.allclose(narrow[::400], O.treeshap(f, 0.5, 256, some), rtol=1e-5, atol=1e-6)
+    ctx.close()
 
 
 @pytest.mark.parametrize("nodes", [1, 2, 3, 4])
