@@ -802,7 +802,7 @@ struct ShapGroup {
 };
 // Items in feature order: one column of one group.  offset_run: the column's
 // first double within its batch | (run + 1) << 12 when its feature's sums go to
-// that run after this item (0: they continue).
+// that run after this item (0: they continue); fewer than 2^20 runs.
 struct ShapItem {
     uint32_t group, offset_run;
 };

@@ -18,8 +18,7 @@ constexpr size_t SET_DOUBLES = (size_t)1 << 25;
 // Bytes of a slab's outcomes and of its runs.
 constexpr size_t SLAB_BYTES = (size_t)128 << 20;
 // Bytes of the sums that several sets share: more rows go in passes, each making
-// the sets' tables again (a pass is 671k rows
-// of 100 columns).
+// the sets' tables again (a pass is 671k rows of 100 columns).
 constexpr size_t SUM_BYTES = (size_t)512 << 20;
 // Workgroups that share the batches of a row block.  A share's end cuts a feature's
 // sum, so their number goes by the plan alone: a row's result does not depend on the
@@ -234,8 +233,10 @@ void make_plan(ShapPlan &plan, const std::vector<TreeView> &trees, size_t first,
         TreeGroups tg(plan, plan.sets[plan.num_sets - 1], trees[t], t, nodes_per_tree, cols);
         doubles += tg.add();
     }
-    if (plan.fits)
-        for (size_t k = 0; k < plan.num_sets; ++k) order_columns(plan.sets[k], cols);
+    for (size_t k = 0; k < plan.num_sets && plan.fits; ++k) {
+        order_columns(plan.sets[k], cols);
+        plan.fits = plan.sets[k].set.num_runs < 1 << 20;   // an item's bits for its run
+    }
     plan.made = true;
 }
 

@@ -1554,6 +1554,22 @@ def test_treeshap_several_table_sets():
     ctx.close()
 
 
+def test_treeshap_more_features_than_runs(ctx):
+    # 2^20 + 3 stumps, each on a feature of its own: more sums per row than an item of the
+    # tables can name
+    n = 2 ** 20 + 3
+    f = O.Forest.empty(n, 3, with_cats=False)
+    f.feature[:, 0] = np.arange(n)
+    f.threshold[:, 0] = 0.5
+    f.leaf[:, 1:] = np.arange(2 * n).reshape(n, 2) % 1021
+    f.cover[:] = [4, 1, 3]
+    x = np.random.default_rng(2).random((n, 2), dtype=np.float32)
+    got = seam_contributions(ctx, f, 0.0, 256, x)
+    mean = 0.25 * f.leaf[:, 1] + 0.75 * f.leaf[:, 2]
+    want = np.where(x <= 0.5, f.leaf[:, 1:2], f.leaf[:, 2:]) - mean[:, None]
+    assert np.allclose(got[:, :-1], want.T, rtol=1e-5, atol=1e-6)
+
+
 @pytest.mark.parametrize("nodes", [1, 2, 3, 4])
 def test_treeshap_smallest_heaps(ctx, nodes):
     # a split without both its children in the heap is no split
