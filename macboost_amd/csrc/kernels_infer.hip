@@ -935,7 +935,7 @@ __global__ __launch_bounds__(SHAP_THREADS) void k_shap_patterns(
             for (int j = 0; j < 4; ++j) {
                 const uint32_t flags = T[j].flags, bit = 1u << (flags >> 16);
                 const bool when_left = (flags & 0x100u) != 0;
-                if (flags & (FLAG_CATEGORICAL | SHAP_GENERAL)) {
+                if (flags & FLAG_CATEGORICAL) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const bool left = raw_goes_left(

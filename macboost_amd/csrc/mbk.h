@@ -779,10 +779,8 @@ constexpr int SHAP_BLOCK_ROWS = 2048; // rows of a workgroup: a column's LDS loa
 constexpr int SHAP_MAX_BITS = 12;     // a column of 2^12 doubles is one LDS batch
 
 // One split whose outcome enters a group's bit (flags >> 16): the bit stays set
-// while the row goes left (0x100 in flags) or right (not); low flags as a split's.
-// SHAP_GENERAL: a NaN threshold, whose missing values going left are no single
-// compare.
-constexpr uint32_t SHAP_GENERAL = 0x200;
+// while the row goes left (0x100 in flags) or right (not); low flags as a split's (a
+// NaN threshold only where missing values go right).
 struct ShapTest {
     int32_t feature;
     float threshold;

@@ -61,10 +61,29 @@ private:
     mbk::ShapTest test(int n, bool left, int bit) const {
         if (tr_.feature[n] >= cols_) invalid("a tree splits on a feature past the data's columns");
         return {tr_.feature[n], tr_.threshold[n],
-                (uint32_t)tr_.flags[n] | (left ? 0x100u : 0u) |
-                    (std::isnan(tr_.threshold[n]) ? mbk::SHAP_GENERAL : 0u) |
-                    ((uint32_t)bit << 16),
+                (uint32_t)tr_.flags[n] | (left ? 0x100u : 0u) | ((uint32_t)bit << 16),
                 (int32_t)(node0_ + n)};
+    }
+
+    // Appends a group's test.  Where missing values go left at a NaN threshold they are
+    // all that does, which is no single compare with it: a row goes right there if it
+    // is at or below +inf, left if it is not above -inf and not -inf.  (As a case of its
+    // own in the kernel: outcomes of 20k rows x 50 trees of depth 8 394 -> 435 us.)
+    void push(mbk::ShapTest t) {
+        const uint32_t side = mbk::FLAG_DEFAULT_LEFT | 0x100u;
+        if (!std::isnan(t.threshold) || (t.flags & mbk::FLAG_CATEGORICAL) ||
+            !(t.flags & mbk::FLAG_DEFAULT_LEFT)) {
+            sp_.tests.push_back(t);
+        } else if (t.flags & 0x100u) {
+            t.threshold = -INFINITY;
+            sp_.tests.push_back(t);                    // NaN or -inf
+            t.flags &= ~side;
+            sp_.tests.push_back(t);                    // not -inf
+        } else {
+            t.threshold = INFINITY;
+            t.flags ^= side;
+            sp_.tests.push_back(t);                    // not NaN
+        }
     }
 
     // Repeated features of the ancestors share one bit, whose unfollowed share
@@ -97,7 +116,7 @@ private:
         G.col_start = (int32_t)sp_.col_feature.size();
         G.anc = anc_;
         G.bits = anc_;
-        sp_.tests.insert(sp_.tests.end(), path_, path_ + depth_);
+        for (int k = 0; k < depth_; ++k) push(path_[k]);
         sp_.vals.insert(sp_.vals.end(), anc_zero_, anc_zero_ + anc_);
         sp_.col_feature.insert(sp_.col_feature.end(), anc_feature_, anc_feature_ + anc_);
         int feature[SHAP_FEATURES];
@@ -106,7 +125,7 @@ private:
         const int at[3] = {g, 2 * g + 1, 2 * g + 2};
         for (int k = 0; k < 3; ++k) {
             if ((k > 0 && !split(g)) || !split(at[k])) continue;
-            sp_.tests.push_back(test(at[k], true, G.bits));
+            push(test(at[k], true, G.bits));
             const int32_t f = tr_.feature[at[k]];
             int c = 0;
             while (c < nf && feature[c] != f) ++c;
