@@ -23,13 +23,13 @@ constexpr size_t SUM_BYTES = (size_t)512 << 20;
 // Workgroups that share the batches of a row block.  A share's end cuts a feature's
 // sum, so their number goes by the plan alone: a row's result does not depend on the
 // other rows of its call.  Each costs a store of its rows' sums, fewer leave the
-// chip idle for few rows.  100 trees of depth 6, 1k and 200k rows: 0.31 and 1.30 ms
-// with 32 shares, 0.28 and 1.24 with 64, 0.27 and 1.25 with 128 (0.26 and 1.32 when
-// each call took what filled the chip).  50 trees of depth 9, 20k rows: 4.21 ms with
-// 64, 3.83 with 128, 3.70 with 256, 3.74 with 512 (3.81); many batches a share repay
-// the stores there.
+// chip idle for few rows.  100 trees of depth 6, 1k, 20k and 200k rows of 100 columns:
+// 0.31, 0.37 and 1.30 ms with 32 shares, 0.28, 0.34 and 1.24 with 64, 0.28, 0.33 and
+// 1.26 with 96, 0.28, 0.35 and 1.29 with 128 (0.26, 0.33 and 1.33 when each call took
+// what filled the chip).  50 trees of depth 9, 20k rows: 4.21 ms with 64, 3.83 with
+// 128, 3.70 with 256, 3.74 with 512 (3.81); many batches a share repay the stores.
 int plan_shares(int32_t batches) {
-    return std::max(1, std::min(std::clamp(batches / 16, 128, 256), batches));
+    return std::max(1, std::min(std::clamp(batches / 16, 96, 256), batches));
 }
 
 // One tree's groups, appended to a set.
