@@ -662,8 +662,10 @@ struct PredNode {
 constexpr int PRED_SLOTS = 384;       // features in LDS, at most (96 KB of 64 rows)
 constexpr int PRED_MAP = 4096;        // features the slot map covers
 constexpr size_t PRED_INFO_WORDS = 1 + PRED_SLOTS + PRED_MAP;
+// mark: PRED_MARK_WORDS zero words, which the launch leaves zero again.
+constexpr size_t PRED_MARK_WORDS = PRED_MAP / 32 + 2;
 hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
-                              uint32_t *info, PredNode *packed);
+                              uint32_t *mark, uint32_t *info, PredNode *packed);
 // info and packed as launch_forest_pack made them; either may be NULL.  The rows'
 // features go through LDS when the forest uses at most max_slots.
 hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x,

@@ -66,7 +66,7 @@ struct Scratch {
     DevBuf<uint32_t> shap_mask;
     std::mutex shap_mu;              // a call holds them until its work is done
     // mbk_predict_forest, allocated with the context (its calls allocate nothing)
-    DevBuf<uint32_t> forest_features;
+    DevBuf<uint32_t> forest_features, forest_mark;
     DevBuf<mbk::PredNode> nodes;
     std::mutex nodes_mu;             // listing, packing and walk queued together
 };
@@ -223,9 +223,12 @@ int mbk_context_create(int32_t device, mbk_context **out, char **err) {
     return guarded(err, [&]() -> int {
         auto c = std::make_unique<mbk_context>();
         c->dev = std::make_unique<mb::Device>(device);
-        c->scratch.forest_features.pooled = c->scratch.nodes.pooled = true;
-        c->scratch.forest_features.alloc(mbk::PRED_INFO_WORDS);
-        c->scratch.nodes.alloc((size_t)1 << 18);
+        Scratch &sc = c->scratch;
+        sc.forest_features.pooled = sc.forest_mark.pooled = sc.nodes.pooled = true;
+        sc.forest_features.alloc(mbk::PRED_INFO_WORDS);
+        sc.forest_mark.alloc(mbk::PRED_MARK_WORDS);
+        sc.nodes.alloc((size_t)1 << 18);
+        MB_HIP(hipMemsetAsync(sc.forest_mark.ptr, 0, sc.forest_mark.bytes(), c->dev->stream));
         *out = c.release();
         return 0;
     }, -1);
@@ -531,8 +534,8 @@ int mbk_predict_forest(mbk_context *ctx, const int32_t *feature, const float *th
         const bool prepared = rows >= 4096;
         const bool pack = prepared && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
         if (prepared)
-            MB_HIP(mbk::launch_forest_pack(s, f, PREDICT_SLOTS, sc.forest_features.ptr,
-                                           pack ? sc.nodes.ptr : nullptr));
+            MB_HIP(mbk::launch_forest_pack(s, f, PREDICT_SLOTS, sc.forest_mark.ptr,
+                                           sc.forest_features.ptr, pack ? sc.nodes.ptr : nullptr));
         MB_HIP(mbk::launch_predict_forest(s, f, x, rows, data_bins, base_score, out,
                                           prepared ? sc.forest_features.ptr : nullptr,
                                           pack ? sc.nodes.ptr : nullptr, PREDICT_SLOTS));

@@ -1407,14 +1407,16 @@ def test_predict_forest_edges(cols, trees, depth, leaves):
         assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
 
 
-@pytest.mark.parametrize("rows", [100, 4096, 5001])
-def test_predict_forest_slots_under_leaves(rows):
-    # no walk reaches a heap slot under a leaf, so it may name any feature:
-    # below and above the rows from which the used features are listed
+@pytest.mark.parametrize("rows,copies", [(100, 1), (4096, 1), (5001, 1), (17000, 26)])
+def test_predict_forest_slots_under_leaves(rows, copies):
+    # no walk reaches a heap slot under a leaf, so it may name any feature: also where
+    # the used features are listed, by one and by several workgroups
     x, y = O.friedman(6000, 6, 23)
     h, obj = gpu_fit(x, y, {"num_trees": 20, "max_depth": 5, "min_child_weight": 300.0})
     f = model_io.forest_from_json(obj)
-    xs = np.ascontiguousarray(x[:, :rows])
+    f = O.Forest(*(None if a is None else np.concatenate([a] * copies)
+                   for a in dataclasses.astuple(f)))
+    xs = np.ascontiguousarray(np.tile(x, (1, 3))[:, :rows])
     want = O.predict(f, obj["baseScore"], obj["numBins"], xs)
     feature = f.feature.copy()
     nodes, under = feature.shape[1], 0
@@ -1430,11 +1432,12 @@ def test_predict_forest_slots_under_leaves(rows):
     assert under > 50
     ctx = mb.Context(0)
     dev = [ctx.upload(a) for a in (feature, f.threshold, f.flags, f.leaf)]
-    out = ctx.alloc(rows * 4)
-    ctx.call("mbk_predict_forest", *dev, None, *feature.shape, ctx.upload(xs), rows,
-             obj["numBins"] - 1, obj["baseScore"], out)
-    ctx.sync()
-    assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
+    xd, out = ctx.upload(xs), ctx.alloc(rows * 4)
+    for _ in range(2):                                 # the marks are clear again
+        ctx.call("mbk_predict_forest", *dev, None, *feature.shape, xd, rows, obj["numBins"] - 1,
+                 obj["baseScore"], out)
+        ctx.sync()
+        assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
 
 
 def test_model_masks_end_at_last_categorical_node(tmp_path):
