@@ -218,8 +218,10 @@ void Booster::build_forest() {                    // forestBuffers, Booster.swif
         if (in && used < (uint32_t)mbk::PRED_SLOTS) info[1 + used] = f;
         used += in;
     }
-    const bool slots = !past && used <= (uint32_t)mbk::PRED_SLOTS;
-    info[0] = slots ? used : 0xFFFFFFFFu;
+    const int32_t per_class = (int32_t)nt / std::max(1, trained_num_classes);
+    const bool slots = !past && used <= (uint32_t)std::min(mbk::PRED_SLOTS,
+                                                           mbk::predict_slots(per_class));
+    info[0] = used;
     for (size_t t = 0; t < nt; ++t) {
         const Tree &tr = trees[t];
         const size_t size = tr.feature.size();
@@ -246,7 +248,8 @@ void Booster::build_forest() {                    // forestBuffers, Booster.swif
     MB_HIP(hipStreamSynchronize(d.stream));
     forest.packed = reinterpret_cast<mbk::PredNode *>(forest.memory.ptr);
     forest.mask = has_cats ? reinterpret_cast<uint32_t *>(forest.memory.ptr + mask_at) : nullptr;
-    forest.features = reinterpret_cast<uint32_t *>(forest.memory.ptr + info_at);
+    forest.features = slots ? reinterpret_cast<uint32_t *>(forest.memory.ptr + info_at) : nullptr;
+    forest.num_features = slots ? (int32_t)used : 0;
     forest.nodes_per_tree = nodes;
     forest.num_trees = (int)nt;
     forest.valid = true;
@@ -278,7 +281,7 @@ std::vector<float> Booster::predict_raw(const float *x, int64_t rows, int64_t co
             MB_HIP(mbk::launch_predict_forest(d.stream, f, xd.ptr, rows, trained_num_bins - 1,
                                               K > 1 ? base_scores[(size_t)k] : base_score,
                                               od.ptr + k, forest.features, forest.packed,
-                                              num_features));
+                                              forest.num_features));
         }
         MB_HIP(hipMemcpyAsync(out.data(), od.ptr, od.bytes(), hipMemcpyDeviceToHost, d.stream));
         MB_HIP(hipStreamSynchronize(d.stream));

@@ -203,7 +203,8 @@ struct ForestCache {
     int num_trees = 0;
     DevBuf<char> memory;
     const mbk::PredNode *packed = nullptr;
-    const uint32_t *features = nullptr;
+    const uint32_t *features = nullptr;  // listed, num_features of them, or NULL
+    int32_t num_features = 0;
     const uint32_t *mask = nullptr;      // NULL without categorical splits
 };
 

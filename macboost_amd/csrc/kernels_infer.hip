@@ -52,11 +52,11 @@ static int device_cus() {
 // (f32, as one thread walking them in turn would: bit for bit).  The first `stage`
 // heap slots of a chunk's trees are staged in LDS as one 8-byte word each
 // (threshold or leaf value; feature and flags, negative at a leaf), and so are the
-// rows' values of the features the forest uses ([slot][64]: lanes reading different
+// rows' values of the features a listed forest uses ([slot][64]: lanes reading different
 // features of their own rows hit different banks), so a step of the walk is two LDS
 // reads.  One thread per row took a chain of three dependent global loads per step,
-// each lane's on a line of its own: 100 trees of depth 6 over 100 features took 208
-// us for 1 to 20k rows (15 and 39 us now) and 603 us for 500k (480 us).  Bound by the
+// each lane's on a line of its own: 100 trees of depth 6 over 100 features took 230 us
+// for 1 to 20k rows (20 and 28 us now) and 795 us for 500k (309 us).  Bound by the
 // instructions and LDS latency of a step.  A forest whose nodes fit next to a tile's
 // features (160 KB) is staged once per workgroup; else LDS is held to 80 KB where the
 // features allow it, for two workgroups (32 wavefronts) per CU.
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void k_forest_pack(ForestDev f, int64_t nodes,
                                                      int32_t max_slots,
                                                      PredNode *__restrict__ packed) {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (g < nodes) packed[g] = pred_node(f, g, info[0] <= (uint32_t)max_slots, info);
+    if (g < nodes) packed[g] = pred_node(f, g, info && info[0] <= (uint32_t)max_slots, info);
 }
 
 hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
@@ -181,8 +181,9 @@ hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slo
     const int64_t nodes = (int64_t)f.num_trees * f.nodes_per_tree;
     const int64_t blocks = nodes <= FOREST_ALONE ? 1
                            : std::min<int64_t>((nodes + FOREST_NODES - 1) / FOREST_NODES, device_cus());
-    hipLaunchKernelGGL(k_forest_features, dim3((unsigned)blocks), dim3(1024), 0, s, f.feature,
-                       nodes, (uint32_t)f.nodes_per_tree, mark, info);
+    if (info)
+        hipLaunchKernelGGL(k_forest_features, dim3((unsigned)blocks), dim3(1024), 0, s, f.feature,
+                           nodes, (uint32_t)f.nodes_per_tree, mark, info);
     if (packed && nodes > 0)
         hipLaunchKernelGGL(k_forest_pack, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, s, f,
                            nodes, info, std::min(max_slots, PRED_SLOTS), packed);
@@ -290,17 +291,100 @@ __global__ __launch_bounds__(PRED_THREADS) void k_predict_forest(
                                        chunk, stage, steps);
 }
 
+// The same walk by a thread per row, for few trees and many rows: no tile to stage and
+// no barrier, a chain of dependent loads per tree that other rows' wavefronts hide.
+template <bool PACKED>
+__global__ __launch_bounds__(256) void k_predict_few(ForestDev f, const float *__restrict__ x,
+                                                     int64_t rows, int32_t data_bins, float base,
+                                                     float *__restrict__ out,
+                                                     const uint32_t *__restrict__ info,
+                                                     const PredNode *__restrict__ packed,
+                                                     int32_t max_slots, int32_t steps) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= rows) return;
+    const bool by_slot = PACKED && info && info[0] <= (uint32_t)max_slots;
+    float acc = base;                                  // seeded with the base, trees in order
+    for (int32_t t = f.tree_first; t < f.num_trees; t += f.tree_step) {
+        const int64_t h = (int64_t)t * f.nodes_per_tree;
+        int64_t g = h;
+        PredNode nd{};
+        auto load = [&] {
+            if (PACKED) nd = packed[g];
+            else nd.meta = f.feature[g];
+        };
+        load();
+        for (int32_t d = 0; d < steps && nd.meta >= 0; ++d) {
+            int64_t feat = PACKED ? nd.meta >> 2 : nd.meta;
+            if (by_slot) feat = info[1 + feat];
+            const uint32_t flags = PACKED ? (uint32_t)nd.meta & 3u : f.flags[g];
+            const float thr = PACKED ? nd.value : f.threshold[g];
+            const bool left = raw_goes_left(x[feat * rows + i], flags, thr,
+                                            f.mask ? f.mask + g * 8 : nullptr, data_bins);
+            g += g - h + (left ? 1 : 2);
+            load();
+        }
+        acc += PACKED ? nd.value : nd.meta < 0 ? f.leaf[g] : f.threshold[g];
+    }
+    out[i * f.out_stride] = acc;
+}
+
+// Trees the walk takes, splits on the longest path of the heap, and heap slots of a
+// tree that a tile stages: whole trees up to depth 7, the first seven levels of deeper
+// ones (a chunk has to hold a tree for every wavefront).
+static int32_t walked_trees(const ForestDev &f) {
+    return std::max(1, (f.num_trees - f.tree_first + f.tree_step - 1) / f.tree_step);
+}
+static int32_t heap_steps(int32_t npt) {
+    int32_t steps = 0;
+    while (steps < 30 && (2 << steps) <= npt) ++steps;
+    return steps;
+}
+static int32_t staged_slots(int32_t npt) { return npt <= 255 ? npt : 127; }
+static int64_t staged_bytes(int32_t npt) {             // and a tree's values of a tile
+    return staged_slots(npt) * (int64_t)sizeof(PredNode) + 64 * 4;
+}
+
+PredictRoute predict_route(const ForestDev &f, int64_t rows) {
+    const int32_t npt = std::max(1, f.nodes_per_tree), trees = walked_trees(f);
+    PredictRoute r{};
+    // With fewer trees than a tile has wavefronts its time no longer falls with them (2M
+    // rows of 100 columns, 1 / 10 / 15 / 20 trees of depth 6: 468 / 579 / 604 / 582 us), a
+    // thread per row's does: 36 / 421 / 574 / 761.  But a row's trees x splits are one
+    // chain of loads, which only many rows hide: 100k rows 8 / 51 us for 1 / 10 trees, in
+    // tiles 20 / 33; 500k rows 13 / 94 and 96 / 122.  Even near 80 (trees x splits)^2
+    // rows: 5 trees 50k, 8 200k, 12 400k.  Past depth 6 a tile reads the deepest nodes from
+    // memory too: 6 trees of depth 9 even near 80k, 10 400k, 3 of depth 12 20k.
+    const int64_t steps = (int64_t)trees * std::min(6, heap_steps(npt));
+    r.few = trees < PRED_WAVES && rows >= 80 * steps * steps;
+    // Packed nodes are one load each.  They pay for their launch (3 us) where every tile
+    // of rows reads them again: trees deeper than a tile stages, or more of them than it
+    // stages at once.  100 trees of depth 9, 20k / 500k rows: 62 / 796 us, packed 56 /
+    // 647; 300 of depth 6 79 / 1,216, packed 75 / 1,034; 100 of depth 6, staged once, 29 /
+    // 313, packed 32 / 308.  Below 16k rows nothing gains.
+    const bool once = npt == staged_slots(npt) && trees * staged_bytes(npt) <= 160 << 10;
+    r.pack = !r.few && !once && rows >= 16384;
+    // Features in LDS cost their columns' loads and save a load a step, which many trees
+    // repay, and rows enough the listing: 100 columns, 100 / 300 / 1,000 trees of depth 6,
+    // 500k rows 308 / 1,034 / 3,346 us without, 482 / 990 / 2,890 with them, 50k rows 53 /
+    // 144 / 465 and 82 / 151 / 419.
+    r.list = !r.few && trees >= 256 && rows * trees >= (int64_t)1 << 24;
+    return r;
+}
+
 hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x, int64_t rows,
                                  int32_t data_bins, float base, float *out, const uint32_t *info,
                                  const PredNode *packed, int32_t max_slots) {
     if (rows <= 0) return hipSuccess;
     const int32_t slots = info ? std::max(0, std::min(max_slots, PRED_SLOTS)) : 0;
-    const int32_t mine =
-        std::max(1, (f.num_trees - f.tree_first + f.tree_step - 1) / f.tree_step);
-    // whole trees up to depth 7, the first seven levels of deeper ones: a chunk
-    // has to hold a tree for every wavefront
-    const int32_t npt = std::max(1, f.nodes_per_tree), stage = npt <= 255 ? npt : 127;
-    const int32_t x_bytes = slots * 64 * 4, tree_bytes = stage * (int32_t)sizeof(PredNode) + 64 * 4;
+    const int32_t mine = walked_trees(f), npt = std::max(1, f.nodes_per_tree);
+    const int32_t stage = staged_slots(npt), steps = heap_steps(npt);
+    if (predict_route(f, rows).few) {
+        auto *few = packed ? &k_predict_few<true> : &k_predict_few<false>;
+        hipLaunchKernelGGL(few, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, f, x, rows,
+                           data_bins, base, out, info, packed, slots, steps);
+        return hipGetLastError();
+    }
+    const int32_t x_bytes = slots * 64 * 4, tree_bytes = (int32_t)staged_bytes(npt);
     const bool whole = x_bytes + (int64_t)mine * tree_bytes <= 160 << 10;
     const int32_t budget = (x_bytes <= (40 << 10) ? 80 : 160) << 10;
     int32_t chunk = (budget - x_bytes) / tree_bytes;
@@ -309,8 +393,6 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
     const size_t lds = (size_t)chunk * tree_bytes + (size_t)x_bytes;
     const int64_t tiles = (rows + 63) / 64, resident = lds <= (80 << 10) ? 2 : 1;
     const int64_t grid = whole ? std::min(tiles, resident * device_cus()) : tiles;
-    int32_t steps = 0;                                 // splits on the longest path of the heap
-    while (steps < 30 && (2 << steps) <= npt) ++steps;
     const bool deep = npt > stage;
     auto *kern = f.mask ? (deep ? &k_predict_forest<true, true> : &k_predict_forest<true, false>)
                         : (deep ? &k_predict_forest<false, true> : &k_predict_forest<false, false>);

@@ -652,8 +652,19 @@ struct PredNode {
     float value;          // threshold, or the leaf's value
     int32_t meta;         // feature (or its slot) << 2 | flags, or -1
 };
+// How launch_predict_forest walks f's trees for that many rows: by a thread per row
+// (few), else by tiles of rows, for which it pays to pack the nodes first, and to
+// list the features the trees split on for the tiles to hold them in LDS.
+struct PredictRoute {
+    bool few, pack, list;
+};
+PredictRoute predict_route(const ForestDev &f, int64_t rows);
+// The features that a tile may hold for that many trees: staging them costs their
+// columns' loads, and saves a load a step (100k rows x 100 trees of depth 6, columns used
+// of as many: 50 of 100 71 us staged, 75 not; 300 of 2,000 204 and 106).
+inline int32_t predict_slots(int32_t trees) { return trees / 2; }
 // A forest prepared for batch walks: the features it splits on in info, and in
-// packed its num_trees * nodes_per_tree heap slots, for walks with the same
+// packed its num_trees * nodes_per_tree heap slots, for walks with the same info and
 // max_slots.  info[0]: the number of features (0xFFFFFFFF: more than PRED_SLOTS, or
 // one past PRED_MAP), info[1 ..]: those features ascending, info[1 + PRED_SLOTS ..]:
 // the slot of every feature below PRED_MAP.  packed names features by slot when
@@ -664,10 +675,11 @@ constexpr int PRED_MAP = 4096;        // features the slot map covers
 constexpr size_t PRED_INFO_WORDS = 1 + PRED_SLOTS + PRED_MAP;
 // mark: PRED_MARK_WORDS zero words, which the launch leaves zero again.
 constexpr size_t PRED_MARK_WORDS = PRED_MAP / 32 + 2;
+// (Either of info and packed may be NULL: not made.)
 hipError_t launch_forest_pack(hipStream_t s, const ForestDev &f, int32_t max_slots,
                               uint32_t *mark, uint32_t *info, PredNode *packed);
-// info and packed as launch_forest_pack made them; either may be NULL.  The rows'
-// features go through LDS when the forest uses at most max_slots.
+// info and packed as launch_forest_pack made them (or NULL).  The rows' features go
+// through LDS when the forest uses at most max_slots.
 hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float *x,
                                  int64_t rows, int32_t data_bins, float base, float *out,
                                  const uint32_t *info, const PredNode *packed,

@@ -87,6 +87,7 @@ struct mbk_context {
 
 namespace {
 
+// Features in LDS for mbk_predict_forest: room for two workgroups per CU.
 constexpr int32_t PREDICT_SLOTS = 160;
 
 void need(bool ok, const char *what) {
@@ -525,20 +526,17 @@ int mbk_predict_forest(mbk_context *ctx, const int32_t *feature, const float *th
     return guarded(err, [&]() -> int {
         mbk::ForestDev f{feature, threshold, flags, leaf, mask, num_trees, nodes_per_tree, 0, 1, 1};
         need(ctx != nullptr, "null kernel-seam context");
-        // listing the features and packing the nodes pay for their launches
-        // from some thousand rows on; 160 features in LDS leave room for two
-        // workgroups per CU
         hipStream_t s = ctx->dev->stream;
         Scratch &sc = ctx->scratch;
         std::lock_guard<std::mutex> lock(sc.nodes_mu);
-        const bool prepared = rows >= 4096;
-        const bool pack = prepared && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
-        if (prepared)
-            MB_HIP(mbk::launch_forest_pack(s, f, PREDICT_SLOTS, sc.forest_mark.ptr,
-                                           sc.forest_features.ptr, pack ? sc.nodes.ptr : nullptr));
-        MB_HIP(mbk::launch_predict_forest(s, f, x, rows, data_bins, base_score, out,
-                                          prepared ? sc.forest_features.ptr : nullptr,
-                                          pack ? sc.nodes.ptr : nullptr, PREDICT_SLOTS));
+        const mbk::PredictRoute r = mbk::predict_route(f, rows);
+        const bool pack = r.pack && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
+        uint32_t *info = r.list ? sc.forest_features.ptr : nullptr;
+        mbk::PredNode *nodes = pack ? sc.nodes.ptr : nullptr;
+        const int32_t slots = std::min(PREDICT_SLOTS, mbk::predict_slots(num_trees));
+        MB_HIP(mbk::launch_forest_pack(s, f, slots, sc.forest_mark.ptr, info, nodes));
+        MB_HIP(mbk::launch_predict_forest(s, f, x, rows, data_bins, base_score, out, info, nodes,
+                                          slots));
         return 0;
     }, -1);
 }

@@ -6,8 +6,10 @@ of the oracle's double-precision recursive TreeSHAP.
 """
 import ctypes
 import json
+import tempfile
 import threading
 from concurrent.futures import ThreadPoolExecutor
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -1407,7 +1409,43 @@ def test_predict_forest_edges(cols, trees, depth, leaves):
         assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
 
 
-@pytest.mark.parametrize("rows,copies", [(100, 1), (4096, 1), (5001, 1), (17000, 26)])
+@pytest.mark.parametrize("trees,depth,cols,rows", [
+    (1, 1, 3, 79), (1, 1, 3, 80), (2, 3, 5, 2879), (2, 3, 5, 2880), (3, 4, 300, 11521),
+    (1, 12, 30, 2880), (15, 1, 4, 18000), (16, 1, 4, 20480),   # a thread per row, and not
+    (20, 8, 40, 16383), (20, 8, 40, 16384), (160, 6, 30, 16385),   # packed
+    (256, 2, 90, 65536), (255, 2, 90, 65800), (256, 2, 90, 65535),   # listed
+    (1100, 1, 400, 16000)])                            # listed, past its slots
+def test_predict_forest_routes(ctx, trees, depth, cols, rows):
+    # the walks that the size of the forest and the rows choose, at the lines between
+    # them, with categorical splits, NaN, infinities and unseen categories; host rows too
+    rng = np.random.default_rng(rows + trees)
+    f = level_forest(rng, trees, depth, cols)
+    inner = 2 ** depth - 1
+    f.feature[:, :inner] = rng.integers(0, cols, (trees, inner))
+    f.feature[0, 0] = 0                                # categorical, others numeric
+    f.flags[:, :inner] = np.where(f.feature[:, :inner] == 0, 2, rng.integers(0, 2, (trees, inner)))
+    f.cat_mask[:] = rng.integers(0, 2 ** 32, f.cat_mask.shape, dtype=np.uint32)
+    if depth > 2:                                      # a leaf above the last level
+        f.feature[:, 2] = -1
+    x = rng.random((cols, rows), dtype=np.float32)
+    x[0] = rng.integers(-2, 300, rows)
+    for v in (np.nan, np.inf, -np.inf):
+        x[rng.integers(0, cols, rows), np.arange(rows)] = np.where(
+            rng.random(rows) < 0.1, np.float32(v), x[0])
+    want = O.predict(f, 0.25, 256, x)
+    dev = [ctx.upload(a) for a in (f.feature, f.threshold, f.flags, f.leaf, f.cat_mask)]
+    out = ctx.alloc(rows * 4)
+    ctx.call("mbk_predict_forest", *dev, *f.feature.shape, ctx.upload(x), rows, 255, 0.25, out)
+    ctx.sync()
+    assert np.array_equal(ctx.download(out, (rows,), np.float32), want)
+    obj = model_io.forest_to_json(f, base=0.25, num_bins=256, num_features=cols, categorical=[0])
+    with tempfile.TemporaryDirectory() as d:
+        (Path(d) / "m.json").write_text(json.dumps(obj))
+        h = mb.load(Path(d) / "m.json")
+    assert np.array_equal(mb.predict(h, x, feature_major=True), want)
+
+
+@pytest.mark.parametrize("rows,copies", [(100, 1), (4096, 1), (5001, 1), (33000, 26)])
 def test_predict_forest_slots_under_leaves(rows, copies):
     # no walk reaches a heap slot under a leaf, so it may name any feature: also where
     # the used features are listed, by one and by several workgroups
@@ -1416,7 +1454,7 @@ def test_predict_forest_slots_under_leaves(rows, copies):
     f = model_io.forest_from_json(obj)
     f = O.Forest(*(None if a is None else np.concatenate([a] * copies)
                    for a in dataclasses.astuple(f)))
-    xs = np.ascontiguousarray(np.tile(x, (1, 3))[:, :rows])
+    xs = np.ascontiguousarray(np.tile(x, (1, 6))[:, :rows])
     want = O.predict(f, obj["baseScore"], obj["numBins"], xs)
     feature = f.feature.copy()
     nodes, under = feature.shape[1], 0
