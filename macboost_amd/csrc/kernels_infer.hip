@@ -361,7 +361,7 @@ PredictRoute predict_route(const ForestDev &f, int64_t rows) {
     // stages at once.  100 trees of depth 9, 20k / 500k rows: 62 / 796 us, packed 56 /
     // 647; 300 of depth 6 79 / 1,216, packed 75 / 1,034; 100 of depth 6, staged once, 29 /
     // 313, packed 32 / 308.  Below 16k rows nothing gains.
-    const bool once = npt == staged_slots(npt) && trees * staged_bytes(npt) <= 160 << 10;
+    const bool once = npt == staged_slots(npt) && trees * staged_bytes(npt) <= LDS_BYTES;
     r.pack = !r.few && !once && rows >= 16384;
     // Features in LDS cost their columns' loads and save a load a step, which many trees
     // repay, and rows enough the listing: 100 columns, 100 / 300 / 1,000 trees of depth 6,
@@ -385,7 +385,7 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
         return hipGetLastError();
     }
     const int32_t x_bytes = slots * 64 * 4, tree_bytes = (int32_t)staged_bytes(npt);
-    const bool whole = x_bytes + (int64_t)mine * tree_bytes <= 160 << 10;
+    const bool whole = x_bytes + (int64_t)mine * tree_bytes <= LDS_BYTES;
     const int32_t budget = (x_bytes <= (40 << 10) ? 80 : 160) << 10;
     int32_t chunk = (budget - x_bytes) / tree_bytes;
     if (chunk > PRED_WAVES) chunk -= chunk % PRED_WAVES;   // whole rounds of the wavefronts
@@ -396,8 +396,7 @@ hipError_t launch_predict_forest(hipStream_t s, const ForestDev &f, const float 
     const bool deep = npt > stage;
     auto *kern = f.mask ? (deep ? &k_predict_forest<true, true> : &k_predict_forest<true, false>)
                         : (deep ? &k_predict_forest<false, true> : &k_predict_forest<false, false>);
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e = allow_all_lds(reinterpret_cast<const void *>(kern));
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(PRED_THREADS), lds, s, f, x,
                        rows, data_bins, base, out, info, packed, slots, chunk, stage, steps);

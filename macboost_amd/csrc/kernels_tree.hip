@@ -5112,9 +5112,8 @@ hipError_t launch_small_level(hipStream_t s, const SmallArgs &a, const SplitPara
     int32_t copies = 4;
     while (copies > 2 && cells * (size_t)copies * 8 > (size_t)65536) copies /= 2;
     const size_t lds = cells * (size_t)copies * 8 + (has_cats ? SMALL_WAVES * sizeof(CatScratch) : 0);
-    if (lds > (size_t)160 << 10) return hipErrorInvalidValue;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_level),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (lds > (size_t)LDS_BYTES) return hipErrorInvalidValue;
+    const hipError_t e = allow_all_lds(reinterpret_cast<const void *>(&k_small_level));
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_small_level, dim3((unsigned)a.cols), dim3(SMALL_THREADS), lds, s, a, sp,
                        level, copies);

@@ -10,6 +10,14 @@ namespace mbk {
 constexpr uint32_t FLAG_DEFAULT_LEFT = 1u;
 constexpr uint32_t FLAG_CATEGORICAL = 2u;
 
+// Lets a kernel without static LDS be launched with any dynamic size.  The limit is
+// the process's: a call that set its own size could lower it between another thread's
+// setting and launch.
+constexpr int LDS_BYTES = 160 << 10;  // per workgroup
+inline hipError_t allow_all_lds(const void *kernel) {
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+}
+
 constexpr int PART_ENTRIES = 8192;    // entries per partition block
 constexpr int CURSOR_STRIDE = 16;     // u64 words per node cursor (one 128-B line each)
 constexpr int SPLIT_KEY_STRIDE = 16;  // u64 words per node split key (one 128-B line each)

@@ -1296,6 +1296,22 @@ def test_validation_metric_keeps_nan():
     assert np.isnan(mb.eval_history(h)[-1])
 
 
+def test_fits_and_predictions_from_several_threads():
+    # separate models at once, each kernel's LDS of another size in every thread (small
+    # fits by depth, predictions by trees)
+    x, y = O.friedman(5000, 9, 76)
+
+    def work(depth):
+        h = mb.train({"num_trees": 12 * depth, "max_depth": depth}, x, y, feature_major=True)
+        return mb.predict(h, x, feature_major=True)
+
+    depths = [7, 1, 6, 2, 5, 3]
+    want = [work(d) for d in depths]
+    with ThreadPoolExecutor(6) as pool:
+        for g, w in zip(pool.map(work, depths * 5), want * 5):
+            assert np.array_equal(g, w)
+
+
 def test_contributions_from_several_threads():
     # calls on one model, each with its own number of rows
     x, y = O.friedman(20000, 10, 77)
