@@ -1242,9 +1242,9 @@ def test_leaf_renewal_sizes(rows, depth, objective):
     ("regression", 1), ("mae", 255), ("quantile", 257), ("binary", 70001), ("poisson", 5000),
     ("tweedie", 66000), ("huber", 300), ("multiclass", 4099)])
 def test_validation_metric_on_device(objective, vrows):
-    # the device's block sums against a float64 restatement of the last round's
-    # metric (one f32 rounding apart at most), over several grow calls and more
-    # rounds than one readback holds
+    # the device's block sums against a float64 restatement of every round's metric from
+    # the trees' own values (one f32 rounding apart at most), over several grow calls and
+    # more rounds than one readback holds; the same values when every round is read back
     rng = np.random.default_rng(vrows)
     x, y = O.friedman(2000 + vrows, 7, 5)
     if objective == "binary":
@@ -1258,32 +1258,59 @@ def test_validation_metric_on_device(objective, vrows):
     params = {"num_trees": 1, "max_depth": 2, "objective": objective, "alpha": 0.7}
     if objective == "huber":
         params["alpha"] = 1.0
+    if objective == "tweedie":
+        params["tweedie_variance_power"] = 1.3
     K = 3 if objective == "multiclass" else 1
     if K > 1:
         params["num_class"] = K
-    t = mb.Trainer(params, xt, yt, eval_set=(xv.T, yv), feature_major=True)
-    for n in (3, 260, 1):
-        t.grow(n * K)
-    h = t.booster()
+
+    def history(extra):
+        t = mb.Trainer({**params, **extra}, xt, yt, eval_set=(xv.T, yv), feature_major=True)
+        for n in (3, 260, 1):
+            t.grow(n * K)
+        return t.booster()
+
+    h = history({})
     hist = mb.eval_history(h)
     assert hist.shape == (264,)
-    p, v = mb.predict(h, xv, feature_major=True).astype(np.float64), yv.astype(np.float64)
+    obj = model_io.saved_model(h)
+    f = model_io.forest_from_json(obj)
+    p = np.empty((vrows, K), np.float32)
+    p[:] = obj["baseScores"] if K > 1 else obj["baseScore"]
+    v, want = yv.astype(np.float64), []
+    for r in range(264):
+        for k in range(K):
+            one = O.Forest(*(None if a is None else a[r * K + k:r * K + k + 1].copy()
+                             for a in dataclasses.astuple(f)))
+            p[:, k] += O.predict(one, 0.0, obj["numBins"], xv)
+        want.append(validation_metric(objective, p.astype(np.float64), v))
+    assert np.allclose(hist, want, rtol=3e-7, atol=0)
+    assert mb.best_iteration(h) == np.argmin(hist) + 1
+    each = history({"early_stopping_rounds": 1000})
+    assert np.array_equal(mb.eval_history(each), hist)
+    assert mb.best_iteration(each) == mb.best_iteration(h)
+
+
+def validation_metric(objective, p, v):
+    q = p[:, 0]
     if objective in ("regression", "huber"):
-        want = np.sqrt(np.mean((p - v) ** 2))
-    elif objective == "mae":
-        want = np.mean(np.abs(p - v))
-    elif objective == "quantile":
-        want = np.mean(np.where(v >= p, 0.7 * (v - p), -0.3 * (v - p)))
-    elif objective == "binary":
-        q = 1 / (1 + np.exp(-p))
-        want = -np.mean(v * np.log(q) + (1 - v) * np.log(1 - q))
-    elif objective == "multiclass":
+        return np.sqrt(np.mean((q - v) ** 2))
+    if objective == "mae":
+        return np.mean(np.abs(q - v))
+    if objective == "quantile":
+        return np.mean(np.where(v >= q, 0.7 * (v - q), -0.3 * (v - q)))
+    if objective == "binary":
+        q = 1 / (1 + np.exp(-q))
+        return -np.mean(v * np.log(q) + (1 - v) * np.log(1 - q))
+    if objective == "multiclass":
         m = p.max(axis=1, keepdims=True)
         logp = p - m - np.log(np.exp(p - m).sum(axis=1, keepdims=True))
-        want = -np.mean(logp[np.arange(vrows), yv.astype(int)])
-    else:
-        return                      # predictions are on the exp scale, rounded to f32
-    assert np.isclose(hist[-1], want, rtol=3e-7, atol=0)
+        return -np.mean(logp[np.arange(len(v)), v.astype(int)])
+    mu = np.exp(q)
+    if objective == "poisson":
+        return np.mean(2 * (np.where(v > 0, v * np.log(np.maximum(v, 1) / mu), 0) - (v - mu)))
+    a = np.where(v > 0, v ** 0.7, 0) / (-0.3 * 0.7)
+    return np.mean(2 * (a - v * mu ** -0.3 / -0.3 + mu ** 0.7 / 0.7))
 
 
 def test_validation_metric_keeps_nan():
