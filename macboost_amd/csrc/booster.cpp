@@ -319,8 +319,6 @@ double Booster::shap_bias(int k) const {
     return bias;
 }
 
-// Root-to-leaf path decomposition (extractShapPaths, SHAP.swift:79-114), with
-// each path's repeated features merged into unique slots.
 // Contributions [rows][K][cols + 1]: class k from its own trees and bias.
 void Booster::predict_contrib(const float *x, int64_t rows, int64_t cols, float *out) {
     const int K = std::max(1, trained_num_classes);
@@ -338,14 +336,6 @@ void Booster::predict_contrib(const float *x, int64_t rows, int64_t cols, float 
     }
 }
 
-// TreeSHAP path tables (extractShapPaths, SHAP.swift:79-114) of trees
-// first, first + step, ...: one path per reachable leaf, taken leaf by leaf in
-// heap order.  A leaf's splits are found by climbing parent links
-// ((n - 1) / 2) to the root and stored root first; each element carries the
-// cover fraction of the child the path takes (0x100 in its flags when that
-// child is the left one), and repeated features on a path share one unique
-// slot whose zero fraction is the product of theirs.  A tree whose root is a
-// leaf contributes only to the bias.
 std::vector<TreeView> tree_views(const std::vector<Tree> &trees) {
     std::vector<TreeView> v;
     v.reserve(trees.size());
@@ -356,6 +346,14 @@ std::vector<TreeView> tree_views(const std::vector<Tree> &trees) {
     return v;
 }
 
+// TreeSHAP path tables (extractShapPaths, SHAP.swift:79-114) of trees
+// first, first + step, ...: one path per reachable leaf, taken leaf by leaf in
+// heap order.  A leaf's splits are found by climbing parent links
+// ((n - 1) / 2) to the root and stored root first; each element carries the
+// cover fraction of the child the path takes (0x100 in its flags when that
+// child is the left one), and repeated features on a path share one unique
+// slot whose zero fraction is the product of theirs.  A tree whose root is a
+// leaf contributes only to the bias.
 ShapTables shap_tables(const std::vector<TreeView> &trees, size_t first, size_t step,
                        int nodes_per_tree) {
     ShapTables st;

@@ -1102,7 +1102,6 @@ static void setup_shape(Trainer &t, int64_t rows, int64_t cols) {
     }
 }
 
-// Bins a raw feature-major validation set with the training edges (device).
 // The categorical id rule on raw features in device memory (as
 // validate_categoricals on the host, which then words the error): first[j] is the
 // first offending row of the j-th categorical column, all ones if none.  Queued on
@@ -1133,8 +1132,9 @@ struct CategoricalCheck {
     }
 };
 
-// Validation features to the device and into bins; check, when given, also
-// checks their categorical ids.  Waits for the stream.
+// Raw feature-major validation features to the device and into bins, by the training
+// edges there; check, when given, also checks their categorical ids.  Waits for the
+// stream.
 static void bin_valid(Trainer &t, const float *xv, int64_t vrows, const float *edges_dev,
                       CategoricalCheck *check = nullptr) {
     hipStream_t s = t.dev->stream;
