@@ -1218,11 +1218,21 @@ static bool small_trees(const Trainer &t) {
     const Params &p = t.p;
     if (t.leafwise || p.goss || p.subsample < 1.0f || !(p.min_child_hess > 0.0f)) return false;
     if (t.D > mbk::SMALL_MAX_DEPTH || (t.D == mbk::SMALL_MAX_DEPTH && t.has_cats)) return false;
-    // Measured crossings with the partitioning path (40 trees of depth 6): 135k rows
-    // at 10 columns, 210k at 37, 240k at 100, 290k at 200, 120k at 300, where a
-    // second round of workgroups starts.
+    // Measured crossings with the partitioning path, rows times rounds of workgroups, in
+    // thousands (trees of depth 6; depth 2 to 7 within a tenth):
+    //   bins \ columns    6   20  100  200  256  257  512  600 2000
+    //   16              117  150  181  187  179  173  154  129  <80
+    //   32              121  152  188  197  188  183  163  140   96
+    //   64              121  156  197  210  200  193  183  164  140
+    //   128             122 >156  214  234  221  220  221  212  313
+    //   256             125 >156  251  292  289  275  312  320 >325
+    // Few bins make the other path's items cheap, above all in wide data.  (At 1,000 to
+    // 16,000 rows of 3,000 / 5,000 / 10,000 columns and 32 bins: 0.98 to 1.04 / 1.09 to 1.17
+    // / 1.18 of that path's time, at 256 bins 0.5 to 0.6.)
     const int64_t rounds = (t.cols + t.dev->num_cus - 1) / t.dev->num_cus;
-    return t.rows <= (100000 + 1000 * (int64_t)std::min(t.cols, 150)) / rounds;
+    const int64_t line = 100000 + 1000 * (int64_t)std::min(t.cols, 70 + 5 * t.nb / 16) -
+                         (rounds - 1) * 125 * std::max(0, 128 - t.nb);
+    return t.rows * rounds <= line;
 }
 
 static void setup_buffers(Trainer &t, const float *y, const float *w, const float *yv,
