@@ -667,10 +667,6 @@ struct PredictRoute {
     bool few, pack, list;
 };
 PredictRoute predict_route(const ForestDev &f, int64_t rows);
-// The features that a tile may hold for that many trees: staging them costs their
-// columns' loads, and saves a load a step (100k rows x 100 trees of depth 6, columns used
-// of as many: 50 of 100 71 us staged, 75 not; 300 of 2,000 204 and 106).
-inline int32_t predict_slots(int32_t trees) { return trees / 2; }
 // A forest prepared for batch walks: the features it splits on in info, and in
 // packed its num_trees * nodes_per_tree heap slots, for walks with the same info and
 // max_slots.  info[0]: the number of features (0xFFFFFFFF: more than PRED_SLOTS, or

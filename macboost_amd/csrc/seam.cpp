@@ -533,10 +533,9 @@ int mbk_predict_forest(mbk_context *ctx, const int32_t *feature, const float *th
         const bool pack = r.pack && (int64_t)num_trees * nodes_per_tree <= (int64_t)sc.nodes.n;
         uint32_t *info = r.list ? sc.forest_features.ptr : nullptr;
         mbk::PredNode *nodes = pack ? sc.nodes.ptr : nullptr;
-        const int32_t slots = std::min(PREDICT_SLOTS, mbk::predict_slots(num_trees));
-        MB_HIP(mbk::launch_forest_pack(s, f, slots, sc.forest_mark.ptr, info, nodes));
+        MB_HIP(mbk::launch_forest_pack(s, f, PREDICT_SLOTS, sc.forest_mark.ptr, info, nodes));
         MB_HIP(mbk::launch_predict_forest(s, f, x, rows, data_bins, base_score, out, info, nodes,
-                                          slots));
+                                          PREDICT_SLOTS));
         return 0;
     }, -1);
 }
