@@ -3123,7 +3123,7 @@ __device__ void plan_level(const Shape &sh, const LevelArgs &la, uint32_t target
     const bool mine = p < num_prev;
     bool split = false;
     uint32_t cl = 0, cr = 0, seg = 0;
-    if (mine) {
+    auto route_counts = [&](uint32_t p) {            // parent p's children
         const uint32_t n = ls_prev + p;
         const uint32_t cnt = count[n];
         const uint32_t left = (uint32_t)__hip_atomic_load(&cursors[(size_t)p * CURSOR_STRIDE],
@@ -3140,9 +3140,18 @@ __device__ void plan_level(const Shape &sh, const LevelArgs &la, uint32_t target
         out.cover[la.level_start + 2 * p + 1] = (float)cr;
         seg_start_next[2 * p] = seg;
         seg_start_next[2 * p + 1] = seg + cl;
+    };
+    uint32_t beyond = 0;
+    if (la.terminal)                                 // no pairs are planned: any level fits
+        for (uint32_t q = p + PLAN_MAX_PAIRS; q < num_prev; q += PLAN_MAX_PAIRS) {
+            route_counts(q);
+            beyond += cl + cr;
+        }
+    if (mine) {
+        route_counts(p);
         s_idx[p] = split ? 1u : 0u;
     }
-    const uint32_t act = wave_sum(cl + cr);
+    const uint32_t act = wave_sum(cl + cr + beyond);
     __syncthreads();
     if (lane_id() == 0) atomicAdd(&s_active, act);
     __syncthreads();
@@ -3187,7 +3196,7 @@ hipError_t launch_plan_level(hipStream_t s, const Shape &sh, const LevelArgs &la
                              const uint32_t *seg_start_prev, uint32_t *seg_start_next,
                              uint32_t *count, const uint64_t *cursors, const TreeOut out,
                              Pair *pairs, HistItem *items) {
-    if ((la.num_level >> 1) > PLAN_MAX_PAIRS) return hipErrorInvalidValue;
+    if ((la.num_level >> 1) > PLAN_MAX_PAIRS && !la.terminal) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_plan_level, dim3(1), dim3(1024), 0, s, sh, la, target_items, min_chunk,
                        ctl, seg_start_prev, seg_start_next, count, cursors, out, pairs, items);
     return hipGetLastError();
@@ -3550,7 +3559,8 @@ hipError_t launch_route(hipStream_t s, const Shape &sh, const LevelArgs &la,
     if (built_only && (!decide || !write_entries)) return hipErrorInvalidValue;
     RoutePlan rp{};
     if (plan) {
-        if ((plan->next.num_level >> 1) > PLAN_MAX_PAIRS || !plan->done) return hipErrorInvalidValue;
+        if (((plan->next.num_level >> 1) > PLAN_MAX_PAIRS && !plan->next.terminal) || !plan->done)
+            return hipErrorInvalidValue;
         rp = *plan;
     }
     const size_t lds = (size_t)la.num_level * sizeof(uint32_t);

@@ -1226,6 +1226,15 @@ def test_deep_levels_reduce_in_search(cols, depth, tile, params, monkeypatch):
     check_identical(x, y.astype(np.float32), {"num_trees": 3, "max_depth": depth, **params})
 
 
+@pytest.mark.parametrize("objective", ["regression", "mae"])
+def test_deepest_sampled_trees_count_by_partition(objective):
+    # depth 12, sampled, children of any hessian: the deepest nodes' rows come from a last
+    # partition, of 2,048 parents
+    x, y = O.friedman(30011, 6, 37)
+    check_identical(x, y, {"num_trees": 3, "max_depth": 12, "subsample": 0.7,
+                           "min_child_weight": 0.0, "objective": objective})
+
+
 @pytest.mark.parametrize("rows,depth,objective", [
     (3, 2, "mae"), (8191, 1, "mae"), (8193, 1, "quantile"), (40000, 1, "mae"),
     (300001, 2, "quantile")])
