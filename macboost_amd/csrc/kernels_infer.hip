@@ -6,7 +6,7 @@
 // TreeSHAP here computes path contributions once per split outcome into tables
 // and looks every row's up, all in double precision with a fixed summation order
 // and a single rounding to f32 at the end.  Trees too deep for tables (more
-// outcomes than rows) give each row a wavefront and each root-to-leaf path a
+// than 12 outcome bits) give each row a wavefront and each root-to-leaf path a
 // lane, with the row's phi in LDS.
 #include <algorithm>
 
@@ -918,7 +918,7 @@ __global__ __launch_bounds__(64) void k_treeshap_rows(const float *__restrict__ 
 // Two levels per group: one level (leaf pairs) needs 192 lookups per row and
 // depth-6 tree, two 112, three 80 out of tables 6 times the size that no longer
 // stream through LDS.  200k rows x 100 trees of depth 6: 36.4 ms with a path
-// evaluation per row, now 1.2 ms (outcomes 0.62, sums 0.46, tables 0.03).
+// evaluation per row, now 1.1 ms (outcomes 0.62, sums 0.35, finish 0.11, tables 0.03).
 
 constexpr int SHAP_LDS_DOUBLES = 4096;                 // one batch of columns
 constexpr int SHAP_THREADS = SHAP_BLOCK_ROWS / 4;      // four rows per thread
@@ -1086,9 +1086,9 @@ __global__ __launch_bounds__(SHAP_THREADS) void k_shap_patterns(
 // through LDS, where 64 lanes look up their outcomes.  A lane's four rows sum in
 // registers until the feature ends or the share does (a run), then the run's
 // sums are stored: no atomics, so the order is fixed.  Bound by the random
-// 8-byte LDS reads (depth 6: 2.2G of them for 200k rows x 100 trees in 459 us)
-// and, for long columns, by their loads: 20k rows x 50 trees of depth 8 took 405
-// us with 1,024 rows per workgroup and 249 us with 2,048.
+// 8-byte LDS reads (depth 6: 2.2G of them for 200k rows x 100 trees in 349 us; 459 with
+// fewer shares) and, for long columns, by their loads: 20k rows x 50 trees of depth 8
+// took 405 us with 1,024 rows per workgroup and 231 to 249 us with 2,048.
 template <typename PT>
 __global__ __launch_bounds__(SHAP_THREADS) void k_shap_sum(const ShapItem *__restrict__ items,
                                                   const ShapBatch *__restrict__ batches,

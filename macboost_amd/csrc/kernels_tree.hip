@@ -4740,7 +4740,7 @@ hipError_t launch_lwb_select(hipStream_t s, const Shape &sh, const SplitParams &
 // k_small_route 4.2, k_small_start 7.0, the last route 6.4: 11.3 ms; with the search in
 // 32 bits and covers by level 11.4, 4.0, 4.0 and 6.4 us: 9.9 ms); 1,000 x 10, 20 trees
 // of depth 4: 2.52 -> 1.32 ms.  A workgroup streams some 6.5 rows per ns, so the form
-// pays up to 100k to 250k rows (small_trees in trainer.cpp).
+// pays up to 100k to 250k rows (small_trees in trainer.cpp), less in wide data of few bins.
 // Histograms are packed words (HIST_QH_BITS: rows below 2^20), [feature][node][bin],
 // which one workgroup writes and reads again at the next level.
 // ---------------------------------------------------------------------------
