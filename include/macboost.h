@@ -267,7 +267,7 @@ int mbk_grow_tree(mbk_context *ctx, const mbk_tree_shape *shape, const mbk_split
  * categorical splits); out (device) receives [rows][cols + 1] f32, the bias
  * base_score + the trees' cover-weighted leaf means in the last column.  The
  * contribution tables (up to 0.7 GB, usually under 256 MB), split outcomes and fp64
- * sums (128 MB each; forests of several tables 512 MB of sums more) are context
+ * sums or, for few rows, contributions (128 MB each; forests of several tables 512 MB of sums more) are context
  * scratch: more rows go in passes.  Trees too deep for tables on more than 4,096
  * columns take rows x cols doubles. */
 int mbk_treeshap(mbk_context *ctx, const int32_t *feature, const float *threshold,

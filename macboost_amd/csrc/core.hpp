@@ -226,7 +226,7 @@ struct ShapSetPlan {
     std::vector<mbk::ShapGroup> groups;
     std::vector<double> vals;
     std::vector<int32_t> col_feature;        // per column: its feature
-    std::vector<uint32_t> col_off, run_first, at, order;
+    std::vector<uint32_t> col_off, run_first, col_at, run_item, at, order;
     std::vector<mbk::ShapItem> items;
     std::vector<mbk::ShapBatch> batches;
     void clear() {
@@ -242,6 +242,7 @@ struct ShapPlan {
     std::vector<ShapSetPlan> sets;
     size_t num_sets = 0;
     int64_t paths = 0;
+    int64_t evals = 0;         // path evaluations of the tables
     bool fits = true;          // every group within SHAP_MAX_BITS
     std::vector<uint8_t> height;
 };

@@ -4,8 +4,9 @@
 // exact TreeSHAP (gpu_treeshap, :1656-1734).
 //
 // TreeSHAP here computes path contributions once per split outcome into tables
-// and looks every row's up, all in double precision with a fixed summation order
-// and a single rounding to f32 at the end.  Trees too deep for tables (more
+// and looks every row's up (few rows: by the row's own outcomes, no tables), all in
+// double precision with a fixed summation order and a single rounding to f32 at the
+// end.  Trees too deep for tables (more
 // than 12 outcome bits) give each row a wavefront and each root-to-leaf path a
 // lane, with the row's phi in LDS.
 #include <algorithm>
@@ -923,6 +924,56 @@ __global__ __launch_bounds__(64) void k_treeshap_rows(const float *__restrict__ 
 constexpr int SHAP_LDS_DOUBLES = 4096;                 // one batch of columns
 constexpr int SHAP_THREADS = SHAP_BLOCK_ROWS / 4;      // four rows per thread
 
+// The contributions of a group's leaf position q to the group's columns, for an
+// outcome: emit(column, contribution), each column at most once.
+template <int MAXU, typename Emit>
+__device__ __forceinline__ void leaf_contributions(const ShapGroup &g,
+                                                   const double *__restrict__ vals, int q,
+                                                   uint32_t pattern, Emit emit) {
+    const double *anc = vals + g.val_start, *share = anc + g.anc;
+    double zero[MAXU];
+    int col[MAXU];
+    uint32_t ones = pattern & ((1u << g.anc) - 1u);
+#pragma unroll
+    for (int u = 0; u < MAXU; ++u) {
+        zero[u] = u < g.anc ? anc[u] : 1.0;
+        col[u] = u;
+    }
+    int slots = g.anc;
+    // the splits inside on this leaf's path: the root, then a child
+    const double *sh = share;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t in = g.inside[k];
+        if (in == 0) continue;
+        const double left = sh[0], right = sh[1];
+        sh += 2;
+        if (k > 0 && (q >> 1) != k - 1) continue;
+        const bool go_left = k == 0 ? q < 2 : (q & 1) == 0;
+        const bool follows = (((pattern >> ((in >> 8) & 0xFFu)) & 1u) != 0) == go_left;
+        const int c = (int)(in & 0xFFu);
+        int at = slots;
+#pragma unroll
+        for (int u = 0; u < MAXU; ++u)
+            if (u < slots && col[u] == c) at = u;
+#pragma unroll
+        for (int u = 0; u < MAXU; ++u) {
+            if (u == at) {
+                zero[u] *= go_left ? left : right;
+                col[u] = c;
+            }
+        }
+        if (at == slots) {
+            ones |= 1u << at;
+            ++slots;
+        }
+        if (!follows) ones &= ~(1u << at);
+    }
+    path_contributions<MAXU>(slots, zero, ones, vals[g.leaf_start + q], [&](int u, double v) {
+        emit(col[u], v);
+    });
+}
+
 // One workgroup of one wavefront per (group, 64 outcomes): a lane per outcome
 // walks the group's leaves; sums per column in LDS (a lane's own slots), then
 // stored coalesced.  Bound by fp64 arithmetic, but 128 outcomes per group
@@ -940,51 +991,9 @@ __global__ __launch_bounds__(64) void k_shap_tables(const ShapGroup *__restrict_
     const int lane = threadIdx.x;
     const uint32_t pattern = first + (uint32_t)lane;
     for (int c = 0; c < g.num_cols; ++c) acc[c][lane] = 0.0;
-    const double *anc = vals + g.val_start, *share = anc + g.anc;
-    for (int q = 0; q < 4; ++q) {
-        if (!((g.leaves >> q) & 1u)) continue;
-        double zero[MAXU];
-        int col[MAXU];
-        uint32_t ones = pattern & ((1u << g.anc) - 1u);
-#pragma unroll
-        for (int u = 0; u < MAXU; ++u) {
-            zero[u] = u < g.anc ? anc[u] : 1.0;
-            col[u] = u;
-        }
-        int slots = g.anc;
-        // the splits inside on this leaf's path: the root, then a child
-        const double *sh = share;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const uint32_t in = g.inside[k];
-            if (in == 0) continue;
-            const double left = sh[0], right = sh[1];
-            sh += 2;
-            if (k > 0 && (q >> 1) != k - 1) continue;
-            const bool go_left = k == 0 ? q < 2 : (q & 1) == 0;
-            const bool follows = (((pattern >> ((in >> 8) & 0xFFu)) & 1u) != 0) == go_left;
-            const int c = (int)(in & 0xFFu);
-            int at = slots;
-#pragma unroll
-            for (int u = 0; u < MAXU; ++u)
-                if (u < slots && col[u] == c) at = u;
-#pragma unroll
-            for (int u = 0; u < MAXU; ++u) {
-                if (u == at) {
-                    zero[u] *= go_left ? left : right;
-                    col[u] = c;
-                }
-            }
-            if (at == slots) {
-                ones |= 1u << at;
-                ++slots;
-            }
-            if (!follows) ones &= ~(1u << at);
-        }
-        path_contributions<MAXU>(slots, zero, ones, vals[g.leaf_start + q], [&](int u, double v) {
-            acc[col[u]][lane] += v;
-        });
-    }
+    for (int q = 0; q < 4; ++q)
+        if ((g.leaves >> q) & 1u)
+            leaf_contributions<MAXU>(g, vals, q, pattern, [&](int c, double v) { acc[c][lane] += v; });
     if (pattern < (1u << g.bits))
         for (int c = 0; c < g.num_cols; ++c)
             table[(size_t)col_off[g.col_start + c] + pattern] = acc[c][lane];
@@ -1173,6 +1182,134 @@ __global__ __launch_bounds__(256) void k_shap_finish(const double *__restrict__ 
         if (lane < nf) o[f0 + lane] = tile[q][lane];
         if (lane == 0 && f0 + 64 >= cols) o[cols] = bias;
     }
+}
+
+// Few rows: the same sums, to the last bit, without tables.  100 trees of depth 6, one row
+// 210 us a call with tables, 126 so.  Two launches:
+//   k_shap_entries    every row's entries of the columns, by its own outcome per group
+//   k_shap_entry_sums per row the runs of k_shap_sum, then their sums as k_shap_finish's
+// A row costs a path evaluation per leaf where the tables cost 2^bits of them for all
+// rows, so it takes over while rows are fewer than a share of that (few_rows in shap.cpp).
+
+// One workgroup per (group, 64 rows), a row per lane: wavefront w checks every fourth
+// quad of the group's tests, then takes leaf position w; the leaves' contributions
+// to a column are added in their order (a leaf without the column adds 0, which
+// changes no sum).  Bound by the latency of one fp64 path evaluation.
+template <int MAXU>
+__global__ __launch_bounds__(256) void k_shap_entries(ShapRows a, ShapSetDev d, int32_t max_cols) {
+    extern __shared__ double s_part[];                 // [4][max_cols][64]
+    __shared__ uint32_t s_fail[4][64];
+    const ShapGroup g = d.groups[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double *part = s_part + lane;
+    auto slot = [&](int leaf, int c) { return (leaf * max_cols + c) * 64; };
+    const int64_t local = (int64_t)blockIdx.y * 64 + lane;
+    const int64_t r = a.row0 + (local < a.num_rows ? local : a.num_rows - 1);
+    uint32_t fail = 0;
+    for (int t = wave * 4; t < g.num_tests; t += 16) {  // padded to whole quads
+        ShapTest T[4];
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) T[j] = d.tests[g.test_start + t + j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = a.x[(int64_t)T[j].feature * a.rows + r];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t flags = T[j].flags;
+            const bool left = raw_goes_left(v[j], flags & 0xFFu, T[j].threshold,
+                                            a.masks ? a.masks + (int64_t)T[j].node * 8 : nullptr,
+                                            a.data_bins);
+            if (left != ((flags & 0x100u) != 0)) fail |= 1u << (flags >> 16);
+        }
+    }
+    s_fail[wave][lane] = fail;
+    for (int c = 0; c < g.num_cols; ++c) part[slot(wave, c)] = 0.0;
+    __syncthreads();
+    const uint32_t pattern = ~(s_fail[0][lane] | s_fail[1][lane] | s_fail[2][lane] | s_fail[3][lane]) &
+                             ((1u << g.bits) - 1u);
+    const int q = __builtin_amdgcn_readfirstlane(wave);
+    if ((g.leaves >> q) & 1u)
+        leaf_contributions<MAXU>(g, d.vals, q, pattern,
+                                 [&](int c, double v) { part[slot(q, c)] = v; });
+    __syncthreads();
+    if (local >= a.num_rows) return;
+    for (int c = wave; c < g.num_cols; c += 4) {
+        double sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += part[slot(k, c)];
+        a.entries[(size_t)d.col_at[g.col_start + c] * (size_t)a.num_rows + (size_t)local] = sum;
+    }
+}
+
+// One workgroup per a.tile rows (a power of two): a thread per run and row, then per
+// feature and row.  Bound by the longest run's chain of adds.
+constexpr int SHAP_SUM_THREADS = 256;
+__global__ __launch_bounds__(SHAP_SUM_THREADS) void k_shap_entry_sums(ShapRows a, ShapSetDev d,
+                                                                      int32_t num_runs) {
+    extern __shared__ double s_run[];                  // [num_runs][tile]
+    const int64_t first = (int64_t)blockIdx.x * a.tile;
+    const uint32_t n = (uint32_t)num_runs * (uint32_t)a.tile;
+    for (uint32_t k = threadIdx.x; k < n; k += SHAP_SUM_THREADS) {
+        const uint32_t run = k / (uint32_t)a.tile;
+        const int64_t local = first + (k & (uint32_t)(a.tile - 1));
+        const double *src = a.entries + (size_t)(local < a.num_rows ? local : a.num_rows - 1);
+        const uint32_t i1 = d.run_item[run + 1];
+        uint32_t i = d.run_item[run];
+        double sum = 0.0;
+        for (; i + 8 <= i1; i += 8) {
+            double v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = src[(size_t)(i + j) * (size_t)a.num_rows];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sum += v[j];
+        }
+        for (; i < i1; ++i) sum += src[(size_t)i * (size_t)a.num_rows];
+        s_run[k] = sum;
+    }
+    __syncthreads();
+    const int32_t live = (int32_t)(a.num_rows - first < a.tile ? a.num_rows - first : a.tile);
+    for (int32_t k = threadIdx.x; k < live * a.cols; k += SHAP_SUM_THREADS) {
+        const int32_t t = k / a.cols, f = k - t * a.cols;
+        double *total = a.total + (size_t)f * (size_t)a.num_rows + (size_t)(first + t);
+        double v = 0.0;
+        if (!a.first) v = *total;
+        for (uint32_t run = d.run_first[f]; run < d.run_first[f + 1]; ++run)
+            v += s_run[run * (uint32_t)a.tile + (uint32_t)t];
+        if (!a.last) {
+            *total = v;
+            continue;
+        }
+        float *o = a.out + (a.row0 + first + t) * (int64_t)(a.cols + 1);
+        o[f] = (float)v;
+        if (f == 0) o[a.cols] = a.bias;
+    }
+}
+
+hipError_t launch_shap_rows(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                            const ShapRows &w) {
+    if (w.num_rows <= 0 || w.num_rows > (int64_t)65535 * 64 || set.num_runs > SHAP_FEW_RUNS ||
+        set.max_bits > SHAP_MAX_BITS || (!(w.first && w.last) && !w.total))
+        return hipErrorInvalidValue;
+    ShapRows a = w;
+    a.tile = 1;
+    while (a.tile < 8 && a.tile < w.num_rows && 2 * a.tile * set.num_runs <= SHAP_FEW_RUNS) a.tile *= 2;
+    const dim3 grid((unsigned)set.num_groups, (unsigned)((w.num_rows + 63) / 64));
+    // a group's features: its longest path's and one more split inside
+    const int32_t max_cols = std::min(set.max_slots + 1, SHAP_MAX_COLS);
+#define MBK_SHAP_ENTRIES(U)                                                                    \
+    hipLaunchKernelGGL(k_shap_entries<U>, grid, dim3(256),                                     \
+                       (size_t)max_cols * 4 * 64 * sizeof(double), s, a, d, max_cols)
+    if (set.num_groups > 0) {
+        if (set.max_slots <= 4) MBK_SHAP_ENTRIES(4);
+        else if (set.max_slots <= 6) MBK_SHAP_ENTRIES(6);
+        else if (set.max_slots <= 8) MBK_SHAP_ENTRIES(8);
+        else MBK_SHAP_ENTRIES(SHAP_MAX_U);
+    }
+#undef MBK_SHAP_ENTRIES
+    hipLaunchKernelGGL(k_shap_entry_sums, dim3((unsigned)((w.num_rows + a.tile - 1) / a.tile)),
+                       dim3(SHAP_SUM_THREADS), (size_t)set.num_runs * (size_t)a.tile * sizeof(double),
+                       s, a, d, set.num_runs);
+    return hipGetLastError();
 }
 
 hipError_t launch_shap_tables(hipStream_t s, const ShapSet &set, const ShapSetDev &d,

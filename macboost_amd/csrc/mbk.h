@@ -844,6 +844,9 @@ struct ShapSetDev {
     const ShapItem *items;
     const ShapBatch *batches;
     const uint32_t *run_first;       // [cols + 1]
+    // for launch_shap_rows instead of col_off, items and batches:
+    const uint32_t *col_at;          // per column its place among the items
+    const uint32_t *run_item;        // [num_runs + 1] the first item of a run
 };
 // Rows [row0, row0 + slab_rows) of x (slab_rows a multiple of SHAP_BLOCK_ROWS; rows past
 // the end are not written).  total: [cols][total_rows] f64 of the rows from
@@ -866,5 +869,22 @@ hipError_t launch_shap_tables(hipStream_t s, const ShapSet &set, const ShapSetDe
                               double *table);
 hipError_t launch_shap_slab(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
                             const ShapSlab &w);
+// Few rows, [row0, row0 + num_rows) of x, without tables: what launch_shap_slab writes, bit
+// for bit.  Sets of at most SHAP_FEW_RUNS runs.
+constexpr int32_t SHAP_FEW_RUNS = 6144;   // 48 KB of LDS
+struct ShapRows {
+    const float *x;
+    int64_t rows, row0, num_rows;
+    int32_t cols, data_bins;
+    const uint32_t *masks;
+    double *entries;                 // the set's columns * num_rows
+    double *total;                   // [cols][num_rows], needed when there are several sets
+    int first, last;
+    float bias;
+    float *out;
+    int32_t tile;                    // rows of a workgroup's sums (set by the launch)
+};
+hipError_t launch_shap_rows(hipStream_t s, const ShapSet &set, const ShapSetDev &d,
+                            const ShapRows &w);
 
 }  // namespace mbk

@@ -164,7 +164,9 @@ private:
         sp_.set.max_bits = std::max(sp_.set.max_bits, G.bits);
         sp_.set.max_slots = std::max(sp_.set.max_slots, anc_ + extra);
         doubles_ += (size_t)nf << G.bits;
-        plan_.paths += __builtin_popcount(G.leaves);
+        const int64_t leaves = __builtin_popcount(G.leaves);
+        plan_.paths += leaves;
+        plan_.evals += leaves << G.bits;
     }
 
     static constexpr int SHAP_FEATURES = 16;
@@ -189,6 +191,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
     at.assign((size_t)cols + 1, 0u);
     order.resize(2 * n);
     sp.col_off.resize(n);
+    sp.col_at.resize(n);
     sp.items.resize(n);
     sp.batches.clear();
     for (int32_t f : sp.col_feature) at[(size_t)f + 1]++;
@@ -208,6 +211,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
         mbk::ShapBatch &b = sp.batches.back();
         sp.items[k] = {g, b.table_len};
         sp.col_off[order[2 * k]] = off;
+        sp.col_at[order[2 * k]] = (uint32_t)k;
         b.num_items += 1;
         b.table_len += len;
         off += len;
@@ -218,6 +222,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
     sp.set.shares = plan_shares(sp.set.num_batches);
     // a run ends with its feature or with its workgroup's share of the batches
     sp.run_first.assign((size_t)cols + 1, 0u);
+    sp.run_item.assign(1, 0u);
     uint32_t run = 0;
     size_t k = 0;
     for (int64_t q = 0; q < sp.set.shares; ++q) {
@@ -229,6 +234,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
             if (k + 1 < end && sp.col_feature[order[2 * k + 2]] == f) continue;
             sp.items[k].offset_run |= ++run << 12;
             sp.run_first[(size_t)f + 1] = run;
+            sp.run_item.push_back((uint32_t)k + 1);
         }
     }
     for (int32_t f = 0; f < cols; ++f)
@@ -239,7 +245,7 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
 void make_plan(ShapPlan &plan, const std::vector<TreeView> &trees, size_t first, size_t step,
                int nodes_per_tree, int32_t cols) {
     plan.num_sets = 0;
-    plan.paths = 0;
+    plan.paths = plan.evals = 0;
     plan.fits = true;
     size_t doubles = SET_DOUBLES;
     for (size_t t = first; t < trees.size() && plan.fits; t += step) {
@@ -282,6 +288,78 @@ T *reserve(DevBuf<T> &b, size_t n) {
     return b.ptr;
 }
 
+// Whether the call's rows are few enough for launch_shap_rows, which costs a path
+// evaluation per path and row where tables cost `evals` of them and two launches more.
+// Host rows of 20 columns, tables / few rows, us a call:
+//   1 tree of depth 6     1 row 80 / 54, 4,000 100 / 78, 16,000 192 / 198
+//   20 of depth 6         1 row 113 / 76, 500 101 / 94, 1,000 104 / 119
+//   100 of depth 9        1 row 1,967 / 636, 500 1,961 / 2,029
+//   10 of depth 11        1 row 2,666 / 372, 1,000 2,660 / 1,800, 2,000 2,679 / 3,102
+//   100 stumps            1 row 93 / 64, 5,000 118 / 97, 8,000 131 / 124
+//   100 of depth 3        1 row 140 / 74, 4,000 151 / 143, 8,000 174 / 220
+//   1,000 of depth 4      64 rows 338 / 311, 500 331 / 426
+// (short paths are the cheaper ones).  With tables for any rows, calls of few rows and few
+// trees took up to 1.7 times as long as by path.
+bool few_rows(const ShapPlan &plan, int64_t rows) {
+    int32_t slots = 0;                                 // features of the longest path
+    for (size_t k = 0; k < plan.num_sets; ++k) {
+        if (plan.sets[k].set.num_runs > mbk::SHAP_FEW_RUNS) return false;
+        slots = std::max(slots, plan.sets[k].set.max_slots);
+    }
+    const int64_t launches = slots <= 4 ? 1600000 : 700000;   // in path evaluations
+    return rows <= 8192 && rows * plan.paths <= launches + plan.evals * 2 / 5;
+}
+
+// TreeSHAP of few rows, in slabs of rows whose entries and sums stay bounded.
+void run_rows(hipStream_t s, const ShapCall &c, const ShapPlan &plan, ShapScratch &sc) {
+    std::vector<char> &blob = sc.blob;
+    blob.clear();
+    struct Offsets { size_t tests, groups, vals, run_first, col_at, run_item; };
+    std::vector<Offsets> offs;
+    size_t columns = 1;
+    for (size_t k = 0; k < plan.num_sets; ++k) {
+        const ShapSetPlan &sp = plan.sets[k];
+        offs.push_back({append(blob, sp.tests), append(blob, sp.groups), append(blob, sp.vals),
+                        append(blob, sp.run_first), append(blob, sp.col_at),
+                        append(blob, sp.run_item)});
+        columns = std::max(columns, sp.col_at.size());
+    }
+    const bool several = plan.num_sets > 1;
+    int64_t slab = (int64_t)(SLAB_BYTES / 8 / columns);
+    if (several) slab = std::min(slab, (int64_t)(SUM_BYTES / 8 / (size_t)c.cols));
+    slab = std::min(c.rows, std::max<int64_t>(1, slab));
+    char *d = reserve(sc.arrays, blob.size());
+    reserve(sc.runs, columns * (size_t)slab);
+    if (several) reserve(sc.sums, (size_t)slab * (size_t)c.cols);
+    MB_HIP(hipMemcpyAsync(d, blob.data(), blob.size(), hipMemcpyHostToDevice, s));
+    for (int64_t r0 = 0; r0 < c.rows; r0 += slab)
+        for (size_t k = 0; k < plan.num_sets; ++k) {
+            const Offsets &o = offs[k];
+            mbk::ShapSetDev dev{};
+            dev.tests = reinterpret_cast<mbk::ShapTest *>(d + o.tests);
+            dev.groups = reinterpret_cast<mbk::ShapGroup *>(d + o.groups);
+            dev.vals = reinterpret_cast<double *>(d + o.vals);
+            dev.run_first = reinterpret_cast<uint32_t *>(d + o.run_first);
+            dev.col_at = reinterpret_cast<uint32_t *>(d + o.col_at);
+            dev.run_item = reinterpret_cast<uint32_t *>(d + o.run_item);
+            mbk::ShapRows w{};
+            w.x = c.x;
+            w.rows = c.rows;
+            w.row0 = r0;
+            w.num_rows = std::min(slab, c.rows - r0);
+            w.cols = c.cols;
+            w.data_bins = c.data_bins;
+            w.masks = c.masks;
+            w.entries = sc.runs.ptr;
+            w.total = several ? sc.sums.ptr : nullptr;
+            w.first = k == 0;
+            w.last = k + 1 == plan.num_sets;
+            w.bias = c.bias;
+            w.out = c.out;
+            MB_HIP(mbk::launch_shap_rows(s, plan.sets[k].set, dev, w));
+        }
+}
+
 // TreeSHAP by path per lane (k_treeshap_rows / k_treeshap).
 void run_paths(hipStream_t s, const std::vector<TreeView> &trees, size_t first, size_t step,
                int nodes_per_tree, const ShapCall &c, ShapScratch &sc) {
@@ -318,15 +396,17 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
               int nodes_per_tree, const ShapCall &c, ShapPlan &plan, ShapScratch &sc) {
     if (!plan.made) make_plan(plan, trees, first, step, nodes_per_tree, c.cols);
     if (plan.fits && plan.paths == 0) return false;
-    // A row's last bits depend on the kernels, so the rows of the call do not enter the
-    // choice: tables wherever they fit.  They would lose to a path per lane at few
-    // rows and many outcomes, and do not: trees of depth 11 with another feature on
-    // every level (2^12 outcomes a group, the most that fit), 1 to 2,048 rows, 1.0 ms
-    // a call either way for one tree, 7.7 ms against 6.7 to 9.2 for 10, 40 against 57
-    // for 50.
+    // A row's last bits depend on the order of its sums, which the path kernels do not
+    // share: the rows of the call do not enter that choice (they do between tables and
+    // few rows, whose sums are the same).
     if (!plan.fits) {
         run_paths(s, trees, first, step, nodes_per_tree, c, sc);
         MB_HIP(hipStreamSynchronize(s));
+        return true;
+    }
+    if (few_rows(plan, c.rows)) {
+        run_rows(s, c, plan, sc);
+        MB_HIP(hipStreamSynchronize(s));               // the arrays leave with this call
         return true;
     }
     // Slab: rows whose outcomes (and runs) take SLAB_BYTES at most.
@@ -381,7 +461,8 @@ bool treeshap(hipStream_t s, const std::vector<TreeView> &trees, size_t first, s
                                       reinterpret_cast<uint32_t *>(d + o.col_off),
                                       reinterpret_cast<mbk::ShapItem *>(d + o.items),
                                       reinterpret_cast<mbk::ShapBatch *>(d + o.batches),
-                                      reinterpret_cast<uint32_t *>(d + o.run_first)};
+                                      reinterpret_cast<uint32_t *>(d + o.run_first),
+                                      nullptr, nullptr};
             MB_HIP(mbk::launch_shap_tables(s, sp.set, dev, sc.table.ptr));
             for (int64_t r0 = p0; r0 < p1; r0 += slab) {
                 mbk::ShapSlab w{};

@@ -1553,7 +1553,7 @@ def test_model_masks_end_at_last_categorical_node(tmp_path):
 
 
 @pytest.mark.parametrize("rows,cols,trees,depth", [
-    (1, 8, 40, 6),            # one row: every share of the columns its own workgroup
+    (1, 8, 40, 6),            # one row
     (2049, 9, 5, 1),          # one-split groups, a row past a row block
     (2047, 70, 30, 9),        # outcomes of more than 8 bits, features past one finish tile
     (2000, 8, 60, 9),         # more than one share of the columns per feature
@@ -1622,6 +1622,32 @@ def test_contributions_do_not_depend_on_the_batch(ctx, trees, depth):
     want = seam_contributions(ctx, f, 0.5, 256, x)
     assert np.abs(want[:, :12]).max() < 1e-9 and np.count_nonzero(want[:, :12])
     for rows in (1, 70, 2049, 5000):
+        xs = np.ascontiguousarray(x[:, :rows])
+        assert np.array_equal(seam_contributions(ctx, f, 0.5, 256, xs), want[:rows])
+
+
+@pytest.mark.parametrize("trees,depth", [(1, 1), (3, 4), (30, 6), (4, 12)])
+def test_contributions_of_few_rows(ctx, trees, depth):
+    # calls of few rows make no tables and get the same bits: categories, missing values,
+    # repeated features, leaves at any depth; then thresholds that are no numbers, and
+    # flags at random.  Rows around 64 and the last and first of the two kinds of call.
+    x, y = _mixed(9000)
+    x[1, ::9] = np.nan
+    h, obj = gpu_fit(x, y, {"num_trees": trees, "max_depth": depth, "categorical_features": [6]})
+    f = model_io.forest_from_json(obj)
+    few = max(n for n in range(1, 8193) if n * (f.feature >= 0).sum() < 500000)
+    sizes = [1, 63, 64, 65, min(few, 1500), 8192, 8193]
+    want = mb.predict_contrib(h, x, feature_major=True)
+    for rows in sizes:
+        xs = np.ascontiguousarray(x[:, :rows])
+        assert np.array_equal(mb.predict_contrib(h, xs, feature_major=True), want[:rows])
+    x[3, 5::17] = -np.inf
+    for k, (t, n) in enumerate(np.argwhere(f.feature >= 0)):
+        f.flags[t, n] = k % 2
+        if k % 3 == 0:
+            f.threshold[t, n] = (np.nan, np.inf, -np.inf)[k // 3 % 3]
+    want = seam_contributions(ctx, f, 0.5, 256, x)
+    for rows in sizes:
         xs = np.ascontiguousarray(x[:, :rows])
         assert np.array_equal(seam_contributions(ctx, f, 0.5, 256, xs), want[:rows])
 
