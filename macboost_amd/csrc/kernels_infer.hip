@@ -292,8 +292,8 @@ __global__ __launch_bounds__(PRED_THREADS) void k_predict_forest(
                                        chunk, stage, steps);
 }
 
-// The same walk by a thread per row, for few trees and many rows: no tile to stage and
-// no barrier, a chain of dependent loads per tree that other rows' wavefronts hide.
+// The same walk by a thread per row, for few trees: no tile to stage and no barrier, a
+// chain of dependent loads per tree that other rows' wavefronts hide.
 template <bool PACKED>
 __global__ __launch_bounds__(256) void k_predict_few(ForestDev f, const float *__restrict__ x,
                                                      int64_t rows, int32_t data_bins, float base,
@@ -350,13 +350,17 @@ PredictRoute predict_route(const ForestDev &f, int64_t rows) {
     PredictRoute r{};
     // With fewer trees than a tile has wavefronts its time no longer falls with them (2M
     // rows of 100 columns, 1 / 10 / 15 / 20 trees of depth 6: 468 / 579 / 604 / 582 us), a
-    // thread per row's does: 36 / 421 / 574 / 761.  But a row's trees x splits are one
-    // chain of loads, which only many rows hide: 100k rows 8 / 51 us for 1 / 10 trees, in
-    // tiles 20 / 33; 500k rows 13 / 94 and 96 / 122.  Even near 80 (trees x splits)^2
-    // rows: 5 trees 50k, 8 200k, 12 400k.  Past depth 6 a tile reads the deepest nodes from
-    // memory too: 6 trees of depth 9 even near 80k, 10 400k, 3 of depth 12 20k.
-    const int64_t steps = (int64_t)trees * std::min(6, heap_steps(npt));
-    r.few = trees < PRED_WAVES && rows >= 80 * steps * steps;
+    // thread per row's does: 36 / 421 / 574 / 761.  But a row's trees x (splits + leaf) are
+    // one chain of loads, which only many rows hide: 100k rows 8 / 51 us for 1 / 10 trees, in
+    // tiles 20 / 33; 500k rows 13 / 94 and 96 / 122.  Even near 60 chain^2 rows: 5 trees
+    // 50k, 8 200k, 12 400k, 12 stumps 50k, 36 stumps 250k (36 x 4 never).  Past depth 6 a
+    // tile reads the deepest nodes from memory too: 6 trees of depth 9 even near 80k, 10
+    // 400k, 3 of depth 12 20k.  One tree, or chains of 12, take no longer than a tile's
+    // barriers at any rows: 1 row, 1 tree of depth 6 / 9 / 11 4.6 / 4.7 / 5.1 us, in tiles
+    // 5.5 / 6.5 / 7.8; 3 of depth 3 4.6 and 5.2, of depth 4 5.3 and 5.3.
+    const int64_t chain = (int64_t)trees * (1 + std::min(6, heap_steps(npt)));
+    r.few = trees == 1 || chain <= 12 ||
+            ((trees < PRED_WAVES || chain <= 80) && rows >= 60 * chain * chain);
     // Packed nodes are one load each.  They pay for their launch (3 us) where every tile
     // of rows reads them again: trees deeper than a tile stages, or more of them than it
     // stages at once.  100 trees of depth 9, 20k / 500k rows: 62 / 796 us, packed 56 /
