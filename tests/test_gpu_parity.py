@@ -1466,7 +1466,7 @@ def test_predict_forest_edges(cols, trees, depth, leaves):
     (1, 12, 30, 2880), (15, 1, 4, 18000), (16, 1, 4, 20480),   # a thread per row, and not
     (1, 11, 9, 1), (4, 2, 5, 1), (13, 1, 5, 300), (2, 6, 9, 11759), (2, 6, 9, 11760),
     (15, 1, 4, 54000), (16, 4, 6, 383999), (16, 4, 6, 384000), (17, 4, 6, 440000),
-    (20, 8, 40, 16383), (20, 8, 40, 16384), (160, 6, 30, 16385),   # packed
+    (20, 8, 40, 16383), (20, 8, 40, 16384), (160, 6, 30, 16385), (70, 11, 9, 16400),   # packed
     (256, 2, 90, 65536), (255, 2, 90, 65800), (256, 2, 90, 65535),   # listed
     (1100, 1, 400, 16000)])                            # listed, past its slots
 def test_predict_forest_routes(ctx, trees, depth, cols, rows):
