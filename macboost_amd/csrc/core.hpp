@@ -235,6 +235,7 @@ struct ShapSetPlan {
         groups.clear();
         vals.clear();
         col_feature.clear();
+        col_at.clear();
     }
 };
 struct ShapPlan {

@@ -191,7 +191,6 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
     at.assign((size_t)cols + 1, 0u);
     order.resize(2 * n);
     sp.col_off.resize(n);
-    sp.col_at.resize(n);
     sp.items.resize(n);
     sp.batches.clear();
     for (int32_t f : sp.col_feature) at[(size_t)f + 1]++;
@@ -211,7 +210,6 @@ void order_columns(ShapSetPlan &sp, int32_t cols) {
         mbk::ShapBatch &b = sp.batches.back();
         sp.items[k] = {g, b.table_len};
         sp.col_off[order[2 * k]] = off;
-        sp.col_at[order[2 * k]] = (uint32_t)k;
         b.num_items += 1;
         b.table_len += len;
         off += len;
@@ -310,17 +308,27 @@ bool few_rows(const ShapPlan &plan, int64_t rows) {
     return rows <= 8192 && rows * plan.paths <= launches + plan.evals * 2 / 5;
 }
 
+// Every column's place in the feature order, made by the plan's first call of few rows.
+const std::vector<uint32_t> &column_places(ShapSetPlan &sp) {
+    const size_t n = sp.col_feature.size();
+    if (sp.col_at.size() != n) {
+        sp.col_at.resize(n);
+        for (size_t k = 0; k < n; ++k) sp.col_at[sp.order[2 * k]] = (uint32_t)k;
+    }
+    return sp.col_at;
+}
+
 // TreeSHAP of few rows, in slabs of rows whose entries and sums stay bounded.
-void run_rows(hipStream_t s, const ShapCall &c, const ShapPlan &plan, ShapScratch &sc) {
+void run_rows(hipStream_t s, const ShapCall &c, ShapPlan &plan, ShapScratch &sc) {
     std::vector<char> &blob = sc.blob;
     blob.clear();
     struct Offsets { size_t tests, groups, vals, run_first, col_at, run_item; };
     std::vector<Offsets> offs;
     size_t columns = 1;
     for (size_t k = 0; k < plan.num_sets; ++k) {
-        const ShapSetPlan &sp = plan.sets[k];
+        ShapSetPlan &sp = plan.sets[k];
         offs.push_back({append(blob, sp.tests), append(blob, sp.groups), append(blob, sp.vals),
-                        append(blob, sp.run_first), append(blob, sp.col_at),
+                        append(blob, sp.run_first), append(blob, column_places(sp)),
                         append(blob, sp.run_item)});
         columns = std::max(columns, sp.col_at.size());
     }
