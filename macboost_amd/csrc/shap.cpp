@@ -305,7 +305,7 @@ bool few_rows(const ShapPlan &plan, int64_t rows) {
         slots = std::max(slots, plan.sets[k].set.max_slots);
     }
     const int64_t launches = slots <= 4 ? 1600000 : 700000;   // in path evaluations
-    return rows <= 8192 && rows * plan.paths <= launches + plan.evals * 2 / 5;
+    return rows <= 8192 && rows * plan.paths <= launches + plan.evals / 2;
 }
 
 // Every column's place in the feature order, made by the plan's first call of few rows.
