@@ -1654,6 +1654,16 @@ def test_contributions_of_few_rows(ctx, trees, depth):
         assert np.array_equal(seam_contributions(ctx, f, 0.5, 256, xs), want[:rows])
 
 
+def test_contributions_of_few_rows_in_slabs(ctx):
+    # 16,896 columns of a table set: 1,040 rows' entries take two slabs, in each of three sets
+    rng = np.random.default_rng(12)
+    f = level_forest(rng, 16, 10, 12)
+    x = rng.random((12, 6000), dtype=np.float32)
+    want = seam_contributions(ctx, f, 0.5, 256, x)
+    got = seam_contributions(ctx, f, 0.5, 256, np.ascontiguousarray(x[:, :1040]))
+    assert np.array_equal(got, want[:1040])
+
+
 def test_treeshap_several_table_sets():
     # forests of several table sets (15 trees of 5.2M doubles, 2^25 a set): the sums
     # they share hold a pass of rows, not all of them, and wide rows in several passes
